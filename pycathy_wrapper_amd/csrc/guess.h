@@ -15,9 +15,9 @@
 // Parameters (fp32, 40385): per layer W[k][ci][co] then b[co].
 //
 // Device layout: activations bf16 [column][Lp][channels], Lp = levels
-// rounded up to 16 (levels >= L hold zeros).  One wavefront computes one
-// 16-level block of one column with v_mfma_f32_16x16x16bf16_1k tiles; the
-// weights are pre-packed in the MFMA B-operand order.
+// rounded up to 16 (levels >= L hold zeros).  All products are
+// v_mfma_f32_16x16x16bf16_1k tiles on weights pre-packed in the MFMA B-operand
+// order; columns of up to 64 levels run the whole network in one launch.
 #pragma once
 
 #include <array>
@@ -66,7 +66,7 @@ struct GuessNet {
   DBuf<unsigned short> act[4], gb[2], ghead, xs, X;
   DBuf<float> y32, ts, T, part;
   DBuf<int> bidx;
-  int cap = 0, nsplit_cap = 0;
+  int cap = 0;
   int64_t nsamp = 0;
   long adam_t = 0;
   // serialises users of the work buffers (flows on several threads may
@@ -81,9 +81,13 @@ struct GuessNet {
   void ensure(int ncol);
   // device pointers; x: [ncol or idx-range][Lp][8] bf16, y: [ncol][Lp] fp32
   void forward(const unsigned short *x, const int *idx, int ncol, float *y);
-  // one gradient of the mean squared error over levels < L into grad
-  void gradient(const unsigned short *x, const int *idx, const float *t, int ncol, float *loss_slot);
-  void adam(float lr);
+  // one gradient of the mean squared error over levels < L into grad; with lr
+  // the Adam step on it too
+  void gradient(const unsigned short *x, const int *idx, const float *t, int ncol, float *loss_slot,
+                const float *lr);
+  int layered_gradient(const unsigned short *x, const int *idx, const float *t, int ncol, float inv);
+  bool fused() const;
+  int tiles(int ncol) const;
 };
 
 std::shared_ptr<GuessNet> guess_lookup(int64_t h);

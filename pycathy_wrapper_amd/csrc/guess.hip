@@ -179,18 +179,6 @@ __global__ __launch_bounds__(256) void k_gdw(int ncol, int Lp, int L, const int 
     part[((size_t)split * NCW * 16 + 16 * j + 4 * grp + t) * GS + co] = acc[t];
 }
 
-// Sums the split partials in split order into the gradient vector.
-__global__ void k_gdw_reduce(const float *__restrict__ part, int nsplit, int rows, int gs, int K, int cout,
-                             int off_w, int off_b, float *__restrict__ grad) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (K + 1) * cout) return;
-  const int kk = e / cout, c = e - kk * cout;
-  float s = 0.f;
-  for (int p = 0; p < nsplit; ++p) s += part[((size_t)p * rows + kk) * gs + c];
-  if (kk < K) grad[off_w + kk * cout + c] = s;
-  else grad[off_b + c] = s;
-}
-
 // ------------------------------------------------------- loss, Adam --
 // Mean squared error over live levels: gradient 2 d / (ncol L) into the
 // head's 16-channel gradient tensor (channel 0), per-block sums of d^2.
@@ -223,30 +211,359 @@ __global__ __launch_bounds__(256) void k_gloss(int ncol, int Lp, int L, const fl
   if (threadIdx.x == 0) lossp[blockIdx.x] = red[0];
 }
 
-__global__ __launch_bounds__(256) void k_gloss_sum(const float *__restrict__ lossp, int nb, float inv,
-                                                   float *__restrict__ slot) {
-  __shared__ float red[256];
-  float s = 0.f;
-  for (int i = threadIdx.x; i < nb; i += 256) s += lossp[i];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int k = 128; k > 0; k >>= 1) {
-    if ((int)threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
+// Where the partials of a gradient lie: entry (kk, co) of layer l of split p
+// at part[off[l] + p * stride[l] + kk * gs[l] + co] (row kk = K: the bias).
+struct GradParts {
+  const float *part;
+  size_t off[kGuessLayers], stride[kGuessLayers];
+  int gs[kGuessLayers], nsplit;
+};
+// The layers' parameter and pack layout (GuessLayer) for k_gstep.
+struct GradLayers {
+  int off_w[kGuessLayers], cin[kGuessLayers], cout[kGuessLayers], nb[kGuessLayers];
+  unsigned fpack[kGuessLayers], bpack[kGuessLayers];  // bf16x4 units
+};
+
+// Sums the split partials into the gradient vector (STEP: and takes the Adam
+// step and rewrites the parameter's entries of the MFMA packs, whose padding
+// entries stay zero); work-group 0 also sums the loss partials.  A
+// work-group owns kStepCols consecutive parameters: its 16 groups of 64 lanes
+// read every 16th split of the 64 parameters side by side, and their sums
+// meet in LDS in a fixed order.  One thread per parameter adding 256 splits
+// one after the other took 63 us a layer, and the packs nine launches of
+// 4.4 us; here all layers, Adam and the packs are one launch of 18 us at 256
+// splits (48 MB of partials, 2.7 TB/s).
+constexpr int kStepCols = 64, kStepRows = 16;
+template <bool STEP>
+__global__ __launch_bounds__(kStepCols *kStepRows) void k_gstep(GradParts gp, GradLayers ly, const float *__restrict__ lossp,
+                                                                 int nloss, float inv, float *__restrict__ slot,
+                                                                 float *__restrict__ grad, float *__restrict__ w,
+                                                                 float *__restrict__ m, float *__restrict__ v, float lr_t,
+                                                                 float b1, float b2, float eps, short *__restrict__ pack) {
+  __shared__ float sh[kStepRows][kStepCols];
+  const int c = threadIdx.x % kStepCols, q = threadIdx.x / kStepCols;
+  if (blockIdx.x == 0) {
+    float s = 0.f;
+    for (int i = threadIdx.x; i < nloss; i += kStepCols * kStepRows) s += lossp[i];
+    sh[q][c] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      float t = 0.f;
+      for (int i = 0; i < kStepRows; ++i) {
+        float u = 0.f;
+        for (int k = 0; k < kStepCols; ++k) u += sh[i][k];
+        t += u;
+      }
+      slot[0] = t * inv;
+    }
     __syncthreads();
   }
-  if (threadIdx.x == 0) slot[0] = red[0] * inv;
+  const int e = blockIdx.x * kStepCols + c;
+  int l = 0, kk = 0, co = 0;
+  float s = 0.f;
+  if (e < kGuessParams) {
+#pragma unroll
+    for (int i = 1; i < kGuessLayers; ++i)
+      if (e >= ly.off_w[i]) l = i;
+    kk = (e - ly.off_w[l]) / ly.cout[l];  // the bias follows the weights: row K
+    co = (e - ly.off_w[l]) - kk * ly.cout[l];
+    const float *p = gp.part + gp.off[l] + (size_t)kk * gp.gs[l] + co;
+    const size_t st = gp.stride[l];
+    float a[4] = {0.f, 0.f, 0.f, 0.f};  // four loads in flight
+    int i = q;
+    for (; i + 3 * kStepRows < gp.nsplit; i += 4 * kStepRows)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) a[u] += p[(size_t)(i + u * kStepRows) * st];
+    for (; i < gp.nsplit; i += kStepRows) a[0] += p[(size_t)i * st];
+    s = (a[0] + a[1]) + (a[2] + a[3]);
+  }
+  sh[q][c] = s;
+  __syncthreads();
+  if (q != 0 || e >= kGuessParams) return;
+  float gi = 0.f;
+#pragma unroll
+  for (int i = 0; i < kStepRows; i += 4)
+    gi += (sh[i][c] + sh[i + 1][c]) + (sh[i + 2][c] + sh[i + 3][c]);
+  grad[e] = gi;
+  if (!STEP) return;
+  const float mi = b1 * m[e] + (1.f - b1) * gi;
+  const float vi = b2 * v[e] + (1.f - b2) * gi * gi;
+  const float wi = w[e] - lr_t * mi / (sqrtf(vi) + eps);
+  m[e] = mi;
+  v[e] = vi;
+  w[e] = wi;
+  if (kk >= 3 * ly.cin[l]) return;  // a bias: not packed
+  const short h = (short)f2bf(wi);
+  const int r = kk & 15;
+  pack[4 * ((size_t)ly.fpack[l] + ((kk >> 4) * ly.nb[l] + (co >> 4)) * 64 + (r >> 2) * 16 + (co & 15)) + (r & 3)] = h;
+  if (l > 0) {  // k_gpack_bwd: row kp * cin_b + co with kp = 2 - k, column ci
+    const int cin = ly.cin[l], k = kk / cin, ci = kk - k * cin;
+    const int kb = (2 - k) * 16 * ly.nb[l] + co, rb = kb & 15;
+    pack[4 * ((size_t)ly.bpack[l] + ((kb >> 4) * (cin >> 4) + (ci >> 4)) * 64 + (rb >> 2) * 16 + (ci & 15)) + (rb & 3)] = h;
+  }
 }
 
-__global__ void k_gadam(int np, float *__restrict__ w, float *__restrict__ m, float *__restrict__ v,
-                        const float *__restrict__ g, float lr_t, float b1, float b2, float eps) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= np) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.f - b1) * gi;
-  const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  w[i] -= lr_t * mi / (sqrtf(vi) + eps);
+// ------------------------------------------------ the network in one launch --
+// Columns of at most kTileRows levels (Lp <= 64): a work-group takes tiles of
+// whole columns (64 / Lp of them) through all layers in LDS, and in training
+// on through the loss and every layer's gradients, so activations and
+// gradients never reach HBM.  Wave w computes output channels 16w .. 16w+15
+// of every layer (waves w and w + 4 share them and take every other row block),
+// with the layer's B operand (the k_gpack_* packs, 24 VGPRs) loaded once per
+// tile; the weight gradients of the 16 output channels accumulate in MFMA
+// tiles (25 a wave, 100 VGPRs: w the input channels 0 .. 31 and the
+// biases, w + 4 the others and the head) over all tiles of the work-group and are
+// written once, as one split of the partials k_gstep sums.  Rounding points are those of the layer-by-layer
+// kernels (bf16 inputs, weights, activations, gradients; fp32 sums).
+// Bound by LDS latency and barriers (about 18 us per tile) and by writing the
+// partials (48 MB): a training step on 1024 columns of 31 levels took 550 us
+// in 31 launches, 65 us of them convolutions and 87 us weight gradients; it
+// takes 51 us here and 18 us in k_gstep.  With four waves instead of
+// eight (448 registers each) this kernel took 63 us.
+// A row of an LDS tile is padded to 136 bytes (40 for 16 channels) so that the
+// 16 rows of an operand read start in different banks; row kTileRows is zero and
+// stands for the levels outside a column.
+constexpr int kTileRows = 64, kTileBlocks = kTileRows / 16;
+constexpr int kTrainGroups = 256;  // one work-group per CU, one split of the partials each
+constexpr int kFwdGroups = 1024;   // four per CU
+constexpr int kWS = kGuessWidth + 4, kXS = kGuessIn + 4;  // row strides (shorts)
+constexpr int kPartSize = 4 * 16 * 64 + 3 * 13 * 16 * 64 + 13 * 16 * 16;  // floats of one split
+constexpr int kPartOff[kGuessLayers] = {0, 4096, 4096 + 13312, 4096 + 2 * 13312, 4096 + 3 * 13312};
+static_assert(kPartSize == 4096 + 3 * 13312 + 3328, "partial layout");
+
+struct FusedNet {
+  const bf16x4 *pack;
+  const float *w;
+  size_t fpack[kGuessLayers], bpack[kGuessLayers];
+  int off_b[kGuessLayers];
+};
+
+// LDS row of a level's neighbour: row `row` of the tile holds level `lv` of
+// its column (zero row outside [0, L)).
+__device__ __forceinline__ int tile_row(int row, int lv, int L) { return lv >= 0 && lv < L ? row : kTileRows; }
+
+// acc = conv of row block rb of the LDS tile `in` with the wave's B operand.
+template <int CIN, int SS>
+__device__ __forceinline__ f32x4 tile_conv(const short *in, const bf16x4 (&wr)[3 * CIN / 16], int rb, int lv0, int L,
+                                           int grp, int r16) {
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const short *src = in + tile_row(rb * 16 + r16 + k - 1, lv0 + r16 + k - 1, L) * SS + 4 * grp;
+#pragma unroll
+    for (int cb = 0; cb < CIN / 16; ++cb)
+      acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(*(const bf16x4 *)(src + 16 * cb), wr[k * (CIN / 16) + cb], acc, 0,
+                                                      0, 0);
+  }
+  return acc;
+}
+// the wave's B operand of a layer: chunk j of output block b
+template <int N>
+__device__ __forceinline__ void load_pack(bf16x4 (&wr)[N], const bf16x4 *p, int nb, int b, int lane) {
+#pragma unroll
+  for (int j = 0; j < N; ++j) wr[j] = p[(j * nb + b) * 64 + lane];
+}
+// Weight-gradient tiles of one row block: dw[3 cb-blocks k][c] += x_k^T g for the channel
+// blocks [C0, C0 + NC) of `in`, g = the block's gradient operand.
+template <int NC, int SS>
+__device__ __forceinline__ void tile_dw(f32x4 *dw, const short *in, int c0, bf16x4 g, int rb, int lv0, int L, int grp,
+                                        int r16) {
+#pragma unroll
+  for (int cb = 0; cb < NC; ++cb) {
+    short u[6];
+#pragma unroll
+    for (int q = 0; q < 6; ++q)
+      u[q] = in[tile_row(rb * 16 + 4 * grp + q - 1, lv0 + 4 * grp + q - 1, L) * SS + 16 * (c0 + cb) + r16];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const bf16x4 a = {u[k], u[k + 1], u[k + 2], u[k + 3]};
+      dw[k * NC + cb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, g, dw[k * NC + cb], 0, 0, 0);
+    }
+  }
+}
+
+template <bool TRAIN>
+__global__ __launch_bounds__(512, 2) void k_gfused(FusedNet net, int ncol, int Lp, int L, const int *__restrict__ idx,
+                                                   const unsigned short *__restrict__ x, const float *__restrict__ t,
+                                                   float inv, float *__restrict__ y, float *__restrict__ lossp,
+                                                   float *__restrict__ part) {
+  __shared__ __align__(16) short xs[(kTileRows + 1) * kXS];
+  __shared__ __align__(16) short act[TRAIN ? 4 : 2][(kTileRows + 1) * kWS];
+  __shared__ __align__(16) short gr[TRAIN ? 2 : 1][TRAIN ? (kTileRows + 1) * kWS : 4];
+  __shared__ __align__(16) short gh[TRAIN ? (kTileRows + 1) * kXS : 4];
+  __shared__ float red[4];
+  const int lane = threadIdx.x & 63, w = (threadIdx.x >> 6) & 3, h = threadIdx.x >> 8;
+  const int grp = lane >> 4, r16 = lane & 15;
+  const int rbs = Lp >> 4, cpt = kTileBlocks / rbs, nrb = cpt * rbs;  // columns and row blocks per tile
+  const int ntile = (ncol + cpt - 1) / cpt;
+  for (int i = threadIdx.x; i < (kTileRows + 1) * kXS; i += 512) {
+    xs[i] = 0;
+    if (TRAIN) gh[i] = 0;
+  }
+  for (int i = threadIdx.x; i < kWS; i += 512) {
+#pragma unroll
+    for (int a = 0; a < (TRAIN ? 4 : 2); ++a) act[a][kTileRows * kWS + i] = 0;
+    if (TRAIN) gr[0][kTileRows * kWS + i] = gr[1][kTileRows * kWS + i] = 0;
+  }
+  f32x4 dwe[4], dw[3][7];  // input layer (h = 0) or head (h = 1), hidden layers (last tile: the bias)
+  float d2 = 0.f;
+  if (TRAIN) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dwe[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int l = 0; l < 3; ++l)
+#pragma unroll
+      for (int i = 0; i < 7; ++i) dw[l][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  for (int tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
+    __syncthreads();  // the previous tile's readers (and the zero rows) are done
+    // an offset the compiler cannot see through: it would keep every layer's B
+    // operand (180 VGPRs) in registers across the tiles, and spill
+    int opaque = 0;
+    asm volatile("" : "+s"(opaque));
+    const bf16x4 *pack = net.pack + opaque;
+    if (threadIdx.x < 4 * kTileRows) {
+      const int row = threadIdx.x >> 2, c4 = 4 * (threadIdx.x & 3);
+      const int col = tile * cpt + row / Lp, lv = row % Lp;
+      bf16x4 v = {0, 0, 0, 0};
+      if (row < nrb * 16 && col < ncol)
+        v = *(const bf16x4 *)(x + ((size_t)(idx ? idx[col] : col) * Lp + lv) * kGuessIn + c4);
+      *(bf16x4 *)(xs + row * kXS + c4) = v;
+    }
+    // ---- forward: hidden layers
+    bf16x4 w3[3], w12[12];
+    load_pack(w3, pack + net.fpack[0], 4, w, lane);
+#pragma unroll
+    for (int l = 0; l < 4; ++l) {
+      const float bias = net.w[net.off_b[l] + 16 * w + r16];
+      if (l > 0) load_pack(w12, pack + net.fpack[l], 4, w, lane);
+      __syncthreads();
+      short *out = act[TRAIN ? l : l & 1];
+      const short *in = l == 0 ? xs : act[TRAIN ? l - 1 : (l - 1) & 1];
+#pragma unroll
+      for (int i = 0; i < kTileBlocks / 2; ++i) {
+        const int rb = 2 * i + h;
+        if (rb >= nrb) break;
+        const int lv0 = (rb % rbs) * 16;
+        const f32x4 acc = l == 0 ? tile_conv<kGuessIn, kXS>(in, w3, rb, lv0, L, grp, r16)
+                                 : tile_conv<kGuessWidth, kWS>(in, w12, rb, lv0, L, grp, r16);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          float v = fmaxf(acc[u] + bias, 0.f);
+          if (lv0 + 4 * grp + u >= L) v = 0.f;
+          out[(rb * 16 + 4 * grp + u) * kWS + 16 * w + r16] = (short)f2bf(v);
+        }
+      }
+    }
+    // ---- head: wave w takes row block w; channel 0 is the output
+    const short *last = act[TRAIN ? 3 : 1];
+    load_pack(w12, pack + net.fpack[4], 1, 0, lane);
+    __syncthreads();
+    if (h == 0 && w < nrb) {
+      const int lv0 = (w % rbs) * 16, col = tile * cpt + w / rbs;
+      const f32x4 acc = tile_conv<kGuessWidth, kWS>(last, w12, w, lv0, L, grp, r16);
+      if (r16 == 0) {
+        const float bias = net.w[net.off_b[4]];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int lv = lv0 + 4 * grp + u;
+          const float v = lv < L ? acc[u] + bias : 0.f;
+          if (TRAIN) {
+            float gv = 0.f;
+            if (lv < L && col < ncol) {
+              const float d = v - t[(size_t)(idx ? idx[col] : col) * Lp + lv];
+              d2 += d * d;
+              gv = 2.f * d * inv;
+            }
+            gh[(w * 16 + 4 * grp + u) * kXS] = (short)f2bf(gv);
+          } else if (col < ncol) {
+            y[(size_t)col * Lp + lv] = v;
+          }
+        }
+      }
+    }
+    if constexpr (TRAIN) {
+      // ---- backward: head, then hidden layers 3, 2, 1
+      load_pack(w3, pack + net.bpack[4], 4, w, lane);
+      __syncthreads();
+#pragma unroll
+      for (int l = 4; l >= 0; --l) {
+        // gradient at layer l's output: gh (head), else gr[l & 1]; its inputs
+        // are act[l - 1] (xs for layer 0); the next gradient goes to gr[(l - 1) & 1]
+        const short *g = l == 4 ? gh : gr[l & 1];
+        const int gs = l == 4 ? kXS : kWS, gc = l == 4 ? r16 : 16 * w + r16;
+#pragma unroll 1
+        for (int rb = 0; rb < nrb; ++rb) {
+          const int lv0 = (rb % rbs) * 16;
+          bf16x4 gv, one;
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            gv[u] = g[(rb * 16 + 4 * grp + u) * gs + gc];
+            one[u] = r16 == 0 && lv0 + 4 * grp + u < L ? (short)0x3F80 : (short)0;
+          }
+          if (l == 4) {  // input channels 16w .. 16w+15, w = 0 also the bias
+            if (h == 1) {
+              tile_dw<1, kWS>(dwe, act[3], w, gv, rb, lv0, L, grp, r16);
+              if (w == 0) dwe[3] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(one, gv, dwe[3], 0, 0, 0);
+            }
+          } else if (l == 0) {
+            if (h == 0) {
+              tile_dw<1, kXS>(dwe, xs, 0, gv, rb, lv0, L, grp, r16);
+              dwe[3] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(one, gv, dwe[3], 0, 0, 0);
+            }
+          } else {
+            tile_dw<2, kWS>(dw[l - 1], act[l - 1], 2 * h, gv, rb, lv0, L, grp, r16);
+            if (h == 0) dw[l - 1][6] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(one, gv, dw[l - 1][6], 0, 0, 0);
+          }
+        }
+        if (l > 0) {
+#pragma unroll
+          for (int i = 0; i < kTileBlocks / 2; ++i) {
+            const int rb = 2 * i + h;
+            if (rb >= nrb) break;
+            const int lv0 = (rb % rbs) * 16;
+            const f32x4 acc = l == 4 ? tile_conv<kGuessIn, kXS>(g, w3, rb, lv0, L, grp, r16)
+                                     : tile_conv<kGuessWidth, kWS>(g, w12, rb, lv0, L, grp, r16);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const int o = (rb * 16 + 4 * grp + u) * kWS + 16 * w + r16;
+              float v = acc[u];
+              if (lv0 + 4 * grp + u >= L) v = 0.f;
+              if (!(bf2f((unsigned short)act[l - 1][o]) > 0.f)) v = 0.f;
+              gr[(l - 1) & 1][o] = (short)f2bf(v);
+            }
+          }
+        }
+        if (l > 1) load_pack(w12, pack + net.bpack[l - 1], 4, w, lane);
+        if (l > 0) __syncthreads();
+      }
+    }
+  }
+  if constexpr (TRAIN) {
+    // hidden tile 2k + cb of wave half h is chunk 4k + 2h + cb, head tile k chunk
+    // 4k + w; the last tile is the bias chunk
+    float *P = part + (size_t)blockIdx.x * kPartSize;
+#pragma unroll
+    for (int l = 0; l < 3; ++l)
+#pragma unroll
+      for (int i = 0; i < 7; ++i) {
+        if (i == 6 && h == 1) break;
+        const int j = i == 6 ? 12 : 4 * (i >> 1) + 2 * h + (i & 1);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) P[kPartOff[l + 1] + (16 * j + 4 * grp + u) * 64 + 16 * w + r16] = dw[l][i][u];
+      }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (h == 0) P[kPartOff[0] + (16 * i + 4 * grp + u) * 64 + 16 * w + r16] = dwe[i][u];
+        else if (i < 3 || w == 0) P[kPartOff[4] + (16 * (i < 3 ? 4 * i + w : 12) + 4 * grp + u) * 16 + r16] = dwe[i][u];
+      }
+    for (int o = 32; o > 0; o >>= 1) d2 += __shfl_down(d2, o, 64);
+    if (lane == 0 && h == 0) red[w] = d2;
+    __syncthreads();
+    if (threadIdx.x == 0) lossp[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+  }
 }
 
 // ------------------------------------------------------ flow-side ops --
@@ -453,26 +770,54 @@ void GuessNet::ensure(int ncol) {
   CG_REQUIRE(ncol > 0, "guess net: no columns");
   if (ncol <= cap) return;
   const size_t pos = (size_t)ncol * Lp;
-  for (auto &a : act) a.alloc(pos * kGuessWidth);
-  for (auto &a : gb) a.alloc(pos * kGuessWidth);
-  ghead.alloc(pos * 16);
   xs.alloc(pos * kGuessIn);
   y32.alloc(pos);
   ts.alloc(pos);
-  lossp.alloc(grid_for(pos));
-  nsplit_cap = split_count(ncol, Lp);
-  size_t po = 0;
-  for (int l = 0; l < kGuessLayers; ++l) {
-    ly[l].part = po;
-    po += (size_t)nsplit_cap * ly[l].nchunk_w * 16 * ly[l].nb * 16;
-  }
-  part.alloc(po);
   if (!hist.p) hist.alloc(1);
+  if (!fused()) {
+    for (auto &a : act) a.alloc(pos * kGuessWidth);
+    for (auto &a : gb) a.alloc(pos * kGuessWidth);
+    ghead.alloc(pos * 16);
+    lossp.alloc(grid_for(pos));
+    const int nsplit = split_count(ncol, Lp);
+    size_t po = 0;
+    for (int l = 0; l < kGuessLayers; ++l) {
+      ly[l].part = po;
+      po += (size_t)nsplit * ly[l].nchunk_w * 16 * ly[l].nb * 16;
+    }
+    part.alloc(po);
+  }
   cap = ncol;
+}
+
+// Columns of at most kTileRows levels run through k_gfused (a tile of 64 rows
+// keeps the activations and gradients of a training pass in 58 KB of LDS);
+// deeper ones do not fit a tile and run layer by layer.
+bool GuessNet::fused() const { return Lp <= kTileRows; }
+int GuessNet::tiles(int ncol) const {
+  const int cpt = kTileBlocks / (Lp >> 4);
+  return (ncol + cpt - 1) / cpt;
+}
+
+static FusedNet fused_net(const GuessNet &g) {
+  FusedNet f{};
+  f.pack = g.pack.p;
+  f.w = g.w.p;
+  for (int l = 0; l < kGuessLayers; ++l) {
+    f.fpack[l] = g.ly[l].fpack;
+    f.bpack[l] = g.ly[l].bpack;
+    f.off_b[l] = g.ly[l].off_b;
+  }
+  return f;
 }
 
 void GuessNet::forward(const unsigned short *x, const int *idx, int ncol, float *y) {
   ensure(ncol);
+  if (fused()) {
+    hipLaunchKernelGGL(k_gfused<false>, dim3(std::min(tiles(ncol), kFwdGroups)), dim3(512), 0, st, fused_net(*this), ncol,
+                       Lp, L, idx, x, (const float *)nullptr, 0.f, y, (float *)nullptr, (float *)nullptr);
+    return;
+  }
   const int gw = waves_blocks((long)ncol * (Lp / 16));
   const float *W = w.p;
   hipLaunchKernelGGL((k_gconv<kGuessIn, 4>), dim3(gw), dim3(kBlock), 0, st, ncol, Lp, L, idx, x, pack.p + ly[0].fpack,
@@ -486,15 +831,65 @@ void GuessNet::forward(const unsigned short *x, const int *idx, int ncol, float 
                      (unsigned short *)nullptr, y);
 }
 
-void GuessNet::gradient(const unsigned short *x, const int *idx, const float *t, int ncol, float *loss_slot) {
-  forward(x, idx, ncol, y32.p);
-  const size_t pos = (size_t)ncol * Lp;
-  const int gl = grid_for(pos);
+// One gradient of the mean squared error into grad and its loss into
+// loss_slot; with lr the Adam step on it (the packs follow the weights).
+void GuessNet::gradient(const unsigned short *x, const int *idx, const float *t, int ncol, float *loss_slot,
+                        const float *lr) {
+  ensure(ncol);
   const float inv = 1.0f / ((float)ncol * (float)L);
+  GradParts gp{};
+  int nloss;
+  if (fused()) {
+    const int G = std::min(tiles(ncol), kTrainGroups);
+    if (part.n < (size_t)G * kPartSize) {
+      part.alloc((size_t)G * kPartSize);
+      lossp.alloc(G);
+    }
+    hipLaunchKernelGGL(k_gfused<true>, dim3(G), dim3(512), 0, st, fused_net(*this), ncol, Lp, L, idx, x, t, inv,
+                       (float *)nullptr, lossp.p, part.p);
+    nloss = gp.nsplit = G;
+    for (int l = 0; l < kGuessLayers; ++l) {
+      gp.off[l] = kPartOff[l];
+      gp.stride[l] = kPartSize;
+    }
+  } else {
+    nloss = layered_gradient(x, idx, t, ncol, inv);
+    gp.nsplit = split_count(ncol, Lp);
+    for (int l = 0; l < kGuessLayers; ++l) {
+      gp.off[l] = ly[l].part;
+      gp.stride[l] = (size_t)ly[l].nchunk_w * 16 * ly[l].nb * 16;
+    }
+  }
+  gp.part = part.p;
+  GradLayers gl{};
+  for (int l = 0; l < kGuessLayers; ++l) {
+    gp.gs[l] = ly[l].nb * 16;
+    gl.off_w[l] = ly[l].off_w;
+    gl.cin[l] = ly[l].cin;
+    gl.cout[l] = ly[l].cout;
+    gl.nb[l] = ly[l].nb;
+    gl.fpack[l] = (unsigned)ly[l].fpack;
+    gl.bpack[l] = (unsigned)ly[l].bpack;
+  }
+  const dim3 g(grid_for(kGuessParams, kStepCols)), b(kStepCols * kStepRows);
+  short *pk = reinterpret_cast<short *>(pack.p);
+  if (!lr) {
+    hipLaunchKernelGGL(k_gstep<false>, g, b, 0, st, gp, gl, lossp.p, nloss, inv, loss_slot, grad.p, w.p, m.p, v.p, 0.f,
+                       0.f, 0.f, 0.f, pk);
+    return;
+  }
+  ++adam_t;
+  const double b1 = 0.9, b2 = 0.999;
+  const double lr_t = *lr * std::sqrt(1.0 - std::pow(b2, (double)adam_t)) / (1.0 - std::pow(b1, (double)adam_t));
+  hipLaunchKernelGGL(k_gstep<true>, g, b, 0, st, gp, gl, lossp.p, nloss, inv, loss_slot, grad.p, w.p, m.p, v.p,
+                     (float)lr_t, (float)b1, (float)b2, 1e-8f, pk);
+}
+
+// The gradient's partials layer by layer; returns the count of loss partials.
+int GuessNet::layered_gradient(const unsigned short *x, const int *idx, const float *t, int ncol, float inv) {
+  forward(x, idx, ncol, y32.p);
+  const int gl = grid_for((size_t)ncol * Lp);
   hipLaunchKernelGGL(k_gloss, dim3(gl), dim3(kBlock), 0, st, ncol, Lp, L, y32.p, idx, t, inv, ghead.p, lossp.p);
-  hipLaunchKernelGGL(k_gloss_sum, dim3(1), dim3(kBlock), 0, st, lossp.p, gl, 1.0f / ((float)ncol * (float)L),
-                     loss_slot);
-  // the loss partials hold sums of d^2; k_gloss_sum scales by 1/(ncol L)
   const int ns = split_count(ncol, Lp);
   const int gw = waves_blocks((long)ncol * (Lp / 16));
   auto dw_blocks = [&](const GuessLayer &g) { return waves_blocks((long)g.nchunk_w * g.nb * ns); };
@@ -515,20 +910,7 @@ void GuessNet::gradient(const unsigned short *x, const int *idx, const float *t,
   }
   hipLaunchKernelGGL((k_gdw<kGuessIn, 64>), dim3(dw_blocks(ly[0])), dim3(kBlock), 0, st, ncol, Lp, L, idx, x, gb[cur].p,
                      ns, part.p + ly[0].part);
-  for (int l = 0; l < kGuessLayers; ++l) {
-    const GuessLayer &g = ly[l];
-    hipLaunchKernelGGL(k_gdw_reduce, dim3(grid_for((size_t)(g.K + 1) * g.cout)), dim3(kBlock), 0, st,
-                       part.p + g.part, ns, g.nchunk_w * 16, g.nb * 16, g.K, g.cout, g.off_w, g.off_b, grad.p);
-  }
-}
-
-void GuessNet::adam(float lr) {
-  ++adam_t;
-  const double b1 = 0.9, b2 = 0.999;
-  const double lr_t = lr * std::sqrt(1.0 - std::pow(b2, (double)adam_t)) / (1.0 - std::pow(b1, (double)adam_t));
-  hipLaunchKernelGGL(k_gadam, dim3(grid_for(kGuessParams)), dim3(kBlock), 0, st, kGuessParams, w.p, m.p, v.p,
-                     grad.p, (float)lr_t, (float)b1, (float)b2, 1e-8f);
-  repack();
+  return gl;
 }
 
 // ------------------------------------------------------------ handles --
@@ -642,7 +1024,7 @@ int cathy_gpu_guess_gradient(int64_t *net, const int *ncol, const uint16_t *x, c
     const size_t pos = (size_t)*ncol * g->Lp;
     g->xs.upload(x, pos * kGuessIn, g->st);
     g->ts.upload(t, pos, g->st);
-    g->gradient(g->xs.p, nullptr, g->ts.p, *ncol, g->hist.p);
+    g->gradient(g->xs.p, nullptr, g->ts.p, *ncol, g->hist.p, nullptr);
     if (loss) g->hist.download(loss, 1, g->st);
     if (grad) g->grad.download(grad, kGuessParams, g->st);
     CG_HIP(hipStreamSynchronize(g->st));
@@ -680,10 +1062,8 @@ int cathy_gpu_guess_train(int64_t *net, const int *nsteps, const int *batch, con
     g->bidx.alloc(nidx);
     g->bidx.upload(idx, nidx, g->st);
     DBuf<float> h(*nsteps);
-    for (int s = 0; s < *nsteps; ++s) {
-      g->gradient(g->X.p, g->bidx.p + (size_t)s * *batch, g->T.p, *batch, h.p + s);
-      g->adam(*lr);
-    }
+    for (int s = 0; s < *nsteps; ++s)
+      g->gradient(g->X.p, g->bidx.p + (size_t)s * *batch, g->T.p, *batch, h.p + s, lr);
     if (loss) h.download(loss, *nsteps, g->st);
     CG_HIP(hipStreamSynchronize(g->st));
     CG_HIP(hipGetLastError());

@@ -70,6 +70,67 @@ def test_gradient_matches_oracle(L):
             assert np.linalg.norm(a - b) <= 3e-2 * np.linalg.norm(b) + 1e-12, li
 
 
+def _rel_layers(p, x, t, L):
+    """Largest relative gradient error of a layer, and the loss's."""
+    net = GU.GuessNet(L, p)
+    try:
+        loss, g = net.gradient(x, t)
+    finally:
+        net.close()
+    lo, go = GO.backward(p, GO.from_bits(x), t, L)
+    worst = 0.0
+    for (ow, ob), co in zip(GO.offsets(), GO.COUT):
+        for a, b in ((g[ow:ob], go[ow:ob]), (g[ob:ob + co], go[ob:ob + co])):
+            worst = max(worst, float(np.linalg.norm(a - b) / (np.linalg.norm(b) + 1e-12)))
+    return worst, abs(loss - lo) / lo
+
+
+@pytest.mark.parametrize("L,ncol", [(2, 1), (16, 5), (17, 2), (33, 3), (48, 7), (64, 1), (64, 300), (11, 2053), (65, 3)])
+def test_columns_at_tile_edges_match_oracle(L, ncol):
+    """One to four columns a tile (Lp = 64, 48, 32, 16), a last tile that is
+    not full, more tiles than work-groups, and columns too deep for a tile (the
+    layer-by-layer kernels).  Bounds as above: the sums differ in order
+    only; relu and bf16 ties can flip single roundings."""
+    p = _params(11)
+    x = _inputs(12, ncol, L)
+    net = GU.GuessNet(L, p)
+    try:
+        y = net.forward(x)
+    finally:
+        net.close()
+    yo, _ = GO.forward(p, GO.from_bits(x), L)
+    top = np.max(np.abs(yo))
+    assert np.all(y[:, L:] == 0) and np.max(np.abs(y - yo)) <= 1e-2 * top
+    t = np.random.default_rng(13).standard_normal((ncol, GU.padded(L))).astype(np.float32)
+    grad, loss = _rel_layers(p, x, t, L)
+    assert grad <= 3e-2 and loss <= 1e-3, (grad, loss)
+
+
+@pytest.mark.parametrize("L", [31, 65])
+def test_training_step_is_adam_on_the_gradient(L):
+    """One training step from zero moments is Adam's on the gradient of the
+    batch, and the packs follow the weights: the next forward pass is that of a
+    network set to them.  Bound: the update is of the size of lr, formed in fp32
+    (a few ulp of the weights)."""
+    p, lr = _params(21), 1e-3
+    x, t = _inputs(22, 24, L), np.random.default_rng(23).standard_normal((24, GU.padded(L))).astype(np.float32)
+    net, ref = GU.GuessNet(L, p), GU.GuessNet(L, p)
+    try:
+        _, g = net.gradient(x, t)
+        net.load(x, t)
+        net.train(1, 24, lr, seed=1)       # the whole set in another order
+        w = net.get()[0]
+        y = net.forward(x)
+        ref.set(w)
+        assert np.array_equal(y, ref.forward(x))
+    finally:
+        net.close()
+        ref.close()
+    big = np.abs(g) > 1e-3 * np.max(np.abs(g))   # away from gradients that rounding can turn round
+    step = lr * g[big] / (np.abs(g[big]) + 1e-8 / np.sqrt(1e-3))
+    assert np.max(np.abs((p[big] - w[big]) - step)) <= 1e-2 * lr + 4e-7 * np.max(np.abs(p))
+
+
 def test_training_fits_a_column_operator():
     """Adam on a target the network can represent (a smooth nonlinear
     function of neighbouring levels): the loss falls tenfold, and the run is
