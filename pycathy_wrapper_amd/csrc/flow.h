@@ -29,34 +29,41 @@ namespace cg {
 // ------------------------------------------------------------- schedule --
 struct Schedule {
   std::vector<ColDesc> cols;     // column ordering: colour classes
-  std::vector<ListLevel> lv;     // natural ordering: DAG levels
-  DBuf<int> rows;                // row lists of the natural levels
+  std::vector<ListLevel> lv;     // natural ordering: DAG levels (rows in device numbering)
+  DBuf<int> lev;                 // their bounds: level l holds rows lev[l] .. lev[l+1]-1
+  int width = 0, reach = 0;      // longest level; farthest row a row couples to
+  DBuf<uint32_t> tab;            // level tables (level table words) where every row has at most kLevLow lower entries
+  bool tab_ok = false, run_ok = false;  // tables built; the one-work-group sweeps apply
+  int ring = 0, slots = 0;       // their LDS ring's rows; most entries on one side of the diagonal
+  DBuf<uint32_t> q0[2], idx[2];  // LevSweep forward, backward
 };
 
-// Level schedule of the natural elimination order on a full CSR (sorted
-// columns): level(r) = 1 + max level of its lower neighbours.
-inline void natural_levels(int n, const std::vector<int> &rowptr, const std::vector<int> &col,
-                           Schedule &sch, hipStream_t st) {
+// Device numbering of the natural elimination order: rows sorted by
+// level(r) = 1 + max level of its lower neighbours, CATHY ids ascending within
+// a level.  Coupled rows keep their order, so the factor is the natural order's
+// own; the rows a level gathers become neighbours in memory.  upper(r, f)
+// calls f(c) for every coupled c > r.
+template <typename U>
+inline void natural_levels(int n, U &&upper, std::vector<int> &perm, std::vector<int> &iperm, Schedule &sch) {
   std::vector<int> lev(n, 0);
   int nlev = 0;
   for (int r = 0; r < n; ++r) {
-    int l = 0;
-    for (int p = rowptr[r]; p < rowptr[r + 1]; ++p) {
-      int j = col[p];
-      if (j >= r) break;
-      l = std::max(l, lev[j] + 1);
-    }
-    lev[r] = l;
-    nlev = std::max(nlev, l + 1);
+    const int l = lev[r] + 1;
+    upper(r, [&](int c) { lev[c] = std::max(lev[c], l); });
+    nlev = std::max(nlev, l);
   }
-  std::vector<int> cnt(nlev + 1, 0), rows(n);
+  std::vector<int> cnt(nlev + 1, 0);
   for (int r = 0; r < n; ++r) cnt[lev[r] + 1]++;
   for (int l = 0; l < nlev; ++l) cnt[l + 1] += cnt[l];
+  perm.resize(n);
+  iperm.resize(n);
   std::vector<int> fill(cnt.begin(), cnt.end() - 1);
-  for (int r = 0; r < n; ++r) rows[fill[lev[r]]++] = r;
+  for (int r = 0; r < n; ++r) {
+    perm[r] = fill[lev[r]]++;
+    iperm[perm[r]] = r;
+  }
   sch.lv.clear();
   for (int l = 0; l < nlev; ++l) sch.lv.push_back(ListLevel{cnt[l], cnt[l + 1] - cnt[l]});
-  sch.rows.upload(rows, st);
 }
 
 // --------------------------------------------------------------- params --
@@ -477,9 +484,14 @@ struct Flow {
     CG_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
     CG_HIP(hipEventCreate(&ev0));
     CG_HIP(hipEventCreate(&ev1));
-    perm.resize(n);
-    iperm.resize(n);
-    for (int i = 0; i < n; ++i) perm[i] = iperm[i] = i;
+    natural_levels(
+        n,
+        [&](int r, auto &&f) {
+          for (int q = topol[r]; q < topol[r + 1] - 1; ++q) f(ja[q] - 1);
+        },
+        perm, iperm, sched);
+    d_perm.upload(perm, st);
+    d_iperm.upload(iperm, st);
     build_pattern(nullptr, topol, ja);
     std::vector<int> hmap(nnz_sell, -1);
     auto find = [&](int r, int c) {  // COEF1 index of (r, c), r <= c
@@ -489,17 +501,19 @@ struct Flow {
     };
     for (int r = 0; r < n; ++r)
       for (int k = h_rowptr[r]; k < h_rowptr[r + 1]; ++k) {
-        const int c = h_col[k];
-        const int q = c >= r ? find(r, c) : find(c, r);
+        const int nr = iperm[r], nc = iperm[h_col[k]];
+        const int q = nc >= nr ? find(nr, nc) : find(nc, nr);
         CG_REQUIRE(q >= 0, "pattern entry missing from the upper CSR");
         hmap[h_so[r >> 6] + 64 * (k - h_rowptr[r]) + (r & 63)] = q;
       }
     csr_map.upload(hmap, st);
     alloc_solver();
     coef.alloc(nterm);
+    nat.alloc(n);
     CG_HIP(hipStreamSynchronize(st));
   }
-  DBuf<double> coef;
+  DBuf<double> coef, nat;        // COEF1; TNOTI / PNEW in the caller's numbering
+  DBuf<int> d_perm, d_iperm;
   std::vector<uint8_t> h_isdir;
 
   // SYMSLV (solscal-extended.f:4669-4699): INCLDP + PRODDP + GRADDP +
@@ -512,11 +526,12 @@ struct Flow {
     h_isdir.assign(n, 0);
     for (int k = 0; k < numdir; ++k) {
       CG_REQUIRE(noddir[k] >= 1 && noddir[k] <= n, "NODDIR entry out of range");
-      h_isdir[noddir[k] - 1] = 1;
+      h_isdir[perm[noddir[k] - 1]] = 1;
     }
     isdir.upload(h_isdir.data(), n, st);
     coef.upload(coef1, nterm, st);
-    tnoti.upload(tnoti_h, n, st);
+    nat.upload(tnoti_h, n, st);
+    hipLaunchKernelGGL(k_gather, dim3(grid_for(n)), dim3(kBlock), 0, st, n, d_iperm.p, nat.p, tnoti.p);
     hipLaunchKernelGGL(k_gather_coef, dim3(grid_for(nnz_sell)), dim3(kBlock), 0, st, nnz_sell, csr_map.p, coef.p,
                        A.p);
     double err = 0.0;
@@ -531,7 +546,8 @@ struct Flow {
     hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(kBlock), 0, st, G, P(1), res.p + 1);
     double hr[2];
     res.download(hr, 2, st);
-    pdiff.download(pnew_h, n, st);
+    hipLaunchKernelGGL(k_gather, dim3(grid_for(n)), dim3(kBlock), 0, st, n, d_perm.p, pdiff.p, nat.p);
+    nat.download(pnew_h, n, st);
     CG_HIP(hipStreamSynchronize(st));
     *niter_out = niter;
     *err_out = err;
@@ -626,7 +642,23 @@ struct Flow {
     sched.lv.clear();
     sched.cols.clear();
     if (ordering == CATHY_GPU_ORDER_NATURAL) {
-      for (int i = 0; i < n; ++i) perm[i] = iperm[i] = i;
+      std::vector<int> ptr(n + 1, 0), inc((size_t)4 * nt);  // elements of each node
+      for (int e = 0; e < nt; ++e)
+        for (int k = 0; k < 4; ++k) ptr[tetra[5 * (size_t)e + k]]++;
+      for (int i = 0; i < n; ++i) ptr[i + 1] += ptr[i];
+      std::vector<int> fill(ptr.begin(), ptr.end() - 1);
+      for (int e = 0; e < nt; ++e)
+        for (int k = 0; k < 4; ++k) inc[fill[tetra[5 * (size_t)e + k] - 1]++] = e;
+      natural_levels(
+          n,
+          [&](int r, auto &&f) {
+            for (int i = ptr[r]; i < ptr[r + 1]; ++i)
+              for (int k = 0; k < 4; ++k) {
+                const int c = tetra[5 * (size_t)inc[i] + k] - 1;
+                if (c > r) f(c);
+              }
+          },
+          perm, iperm, sched);
       return;
     }
     int ncolr = 0;
@@ -728,6 +760,73 @@ struct Flow {
     ftab_ok = true;
   }
 
+  // Level tables of the natural order (see kLevWords) and whether its sweeps run in one
+  // work-group: every row a level gathers must still be in the LDS ring (reach +
+  // the longest level at most kRingRows rows) and a row's entries fit the
+  // kernels' window of kLevLow on either side of the diagonal.
+  void build_level_tables(const std::vector<int> &hrp, const std::vector<int> &hcol, const std::vector<int> &hsd,
+                          const std::vector<int> &htpos, const std::vector<int> &hso) {
+    sched.tab_ok = sched.run_ok = false;
+    sched.width = sched.reach = 0;
+    int low = 0, up = 0, prev = 0;
+    std::vector<int> bounds(1, 0);
+    for (const ListLevel &L : sched.lv) {
+      CG_REQUIRE(L.off == prev, "levels not contiguous");
+      prev = L.off + L.cnt;
+      bounds.push_back(prev);
+      sched.width = std::max(sched.width, L.cnt);
+      for (int r = L.off; r < prev; ++r)
+        for (int j = 0; j < hsd[r]; ++j) CG_REQUIRE(hcol[hrp[r] + j] < L.off, "coupling inside a level");
+    }
+    CG_REQUIRE(prev == n, "levels do not cover the rows");
+    for (int r = 0; r < n; ++r) {
+      low = std::max(low, hsd[r]);
+      up = std::max(up, hrp[r + 1] - hrp[r] - hsd[r] - 1);
+      sched.reach = std::max(sched.reach, std::max(r - hcol[hrp[r]], hcol[hrp[r + 1] - 1] - r));
+    }
+    sched.lev.upload(bounds, st);
+    if (low > kLevLow) return;
+    std::vector<uint32_t> tab((size_t)kLevWords * n);
+    constexpr int NP = kLevLow * (kLevLow - 1) / 2;
+    uint8_t b[4 * kLevWords];
+    for (int r = 0; r < n; ++r) {
+      std::fill(b, b + sizeof b, (uint8_t)0xFF);
+      for (int j = 0; j < hsd[r]; ++j) {
+        const int p = hrp[r] + j, c = hcol[p];
+        for (int a = 0; a < j; ++a) {
+          const int *e = &hcol[hrp[c + 1]], *f = std::lower_bound(&hcol[hrp[c]], e, hcol[hrp[r] + a]);
+          if (f != e && *f == hcol[hrp[r] + a]) b[j * (j - 1) / 2 + a] = (uint8_t)(f - &hcol[hrp[c]]);
+        }
+        b[NP + j] = (uint8_t)(htpos[p] - hrp[c]);
+      }
+      for (int w = 0; w < kLevWords; ++w)
+        tab[(size_t)w * n + r] = (uint32_t)b[4 * w] | ((uint32_t)b[4 * w + 1] << 8) | ((uint32_t)b[4 * w + 2] << 16) |
+                                 ((uint32_t)b[4 * w + 3] << 24);
+    }
+    sched.tab.upload(tab, st);
+    CG_HIP(hipStreamSynchronize(st));
+    sched.tab_ok = true;
+    if (up > kLevLow || sched.reach + sched.width > kRingRows || bounds.size() > 4096 || nnz_sell > (1 << 28)) return;
+    sched.ring = 64;
+    while (sched.ring < sched.reach + sched.width) sched.ring *= 2;
+    sched.slots = std::max(low, up);
+    std::vector<uint32_t> q0(n), idx((size_t)kRingWords * n);
+    for (int d = 0; d < 2; ++d) {
+      for (int r = 0; r < n; ++r) {
+        const int j0 = d ? hsd[r] + 1 : 0, nj = d ? hrp[r + 1] - hrp[r] - j0 : hsd[r];
+        q0[r] = (uint32_t)(hso[r >> 6] + 64 * j0 + (r & 63));
+        uint32_t pos[kLevLow] = {0};
+        for (int j = 0; j < nj; ++j) pos[j] = (uint32_t)(hcol[hrp[r] + j0 + j] & (sched.ring - 1));
+        for (int i = 0; i < kRingWords; ++i)
+          idx[(size_t)i * n + r] = pos[2 * i] | (pos[2 * i + 1] << 14) | (i == 0 ? (uint32_t)nj << 28 : 0u);
+      }
+      sched.q0[d].upload(q0, st);
+      sched.idx[d].upload(idx, st);
+      CG_HIP(hipStreamSynchronize(st));
+    }
+    sched.run_ok = true;
+  }
+
   // Full pattern in device numbering, from the tetrahedra (tetra != null)
   // or from a 1-based upper CSR (topol, ja) in natural order.
   void build_pattern(const int *tetra, const int *topol = nullptr, const int *ja = nullptr) {
@@ -751,10 +850,11 @@ struct Flow {
           for (int b = 0; b < 4; ++b) ins(v[a], v[b]);
       }
     } else {
-      for (int r = 0; r < n; ++r) {
+      for (int i = 0; i < n; ++i) {
+        const int r = perm[i];
         ins(r, r);
-        for (int q = topol[r] - 1; q < topol[r + 1] - 1; ++q) {
-          const int c = ja[q] - 1;
+        for (int q = topol[i] - 1; q < topol[i + 1] - 1; ++q) {
+          const int c = perm[ja[q] - 1];
           ins(r, c);
           ins(c, r);
         }
@@ -858,7 +958,7 @@ struct Flow {
     slen.upload(hlen, st);
     sdiag.upload(hsd, st);
     stpos.upload(hst, st);
-    if (ordering == CATHY_GPU_ORDER_NATURAL) natural_levels(n, hrp, hcol, sched, st);
+    if (ordering == CATHY_GPU_ORDER_NATURAL) build_level_tables(hrp, hcol, hsd, htpos, hso);
     // every level row must have its same-column neighbours where the column
     // kernels expect them: predecessor = last lower slot, successor = first
     // upper slot
@@ -1080,8 +1180,9 @@ struct Flow {
       F32.alloc(nnz_sell);
       CG_HIP(hipMemsetAsync(F32.p, 0, sizeof(float) * nnz_sell, st));
     } else {
-      F64.alloc(nnz_sell);
-      CG_HIP(hipMemsetAsync(F64.p, 0, sizeof(double) * nnz_sell, st));
+      // the level sweeps read windows of kLevLow slots from a row's first one
+      F64.alloc((size_t)nnz_sell + 64 * kLevLow);
+      CG_HIP(hipMemsetAsync(F64.p, 0, sizeof(double) * F64.n, st));
     }
     part.alloc((size_t)kSlots * kMaxRedBlocks);
     ipart.alloc(kMaxRedBlocks);
@@ -1164,14 +1265,32 @@ struct Flow {
       for (size_t c = fuse ? nc - 1 : nc; c-- > 0;)
         launch_bwd_col3<FT>(sched.cols[c], sl, F, dinv.p, out, out, done);
     } else {
-      for (const ListLevel &L : sched.lv)
-        hipLaunchKernelGGL(k_fwd_list<FT>, dim3(grid_for(L.cnt, 64)), dim3(64), 0, st, L, sched.rows.p, sl, F,
-                           dinv.p, tin, out, done);
-      for (size_t l = sched.lv.size(); l-- > 0;) {
-        const ListLevel &L = sched.lv[l];
-        hipLaunchKernelGGL(k_bwd_list<FT>, dim3(grid_for(L.cnt, 64)), dim3(64), 0, st, L, sched.rows.p, sl, F,
-                           dinv.p, out, out, done);
-      }
+      sweep_levels<false>(dinv.p, tin, out, done);
+      sweep_levels<true>(dinv.p, out, out, done);
+    }
+  }
+  // One sweep over the levels of the natural order (FP64 factor): in one
+  // work-group where its ring holds what a level gathers (meshes up to about
+  // 200,000 nodes; at 66,885 nodes and 173 levels of 387 rows 1.0 us a level
+  // against 5.5 us for a launch each), else a launch per level.
+  template <bool UP>
+  void sweep_levels(const double *di, const double *tin, double *out, const int *done) {
+    const Sell sl = sell();
+    if (sched.run_ok) {
+      const int d = UP ? 1 : 0, nlev = (int)sched.lv.size();
+      const LevSweep S{sched.q0[d].p, sched.idx[d].p};
+      const dim3 b(std::min(1024, (sched.width + 63) / 64 * 64));
+      const size_t sm = sizeof(double) * sched.ring + sizeof(int) * (nlev + 1);
+      auto k = sched.slots <= 7 ? k_sweep_levels<UP, 7> : k_sweep_levels<UP, 8>;
+      hipLaunchKernelGGL(k, dim3(1), b, sm, st, nlev, sched.lev.p, n, S, F64.p, di, tin, out, sched.ring - 1, done);
+      return;
+    }
+    const size_t nl = sched.lv.size();
+    for (size_t i = 0; i < nl; ++i) {
+      const ListLevel &L = sched.lv[UP ? nl - 1 - i : i];
+      const dim3 g(grid_for(L.cnt, 64)), b(64);
+      if (UP) hipLaunchKernelGGL(k_bwd_list, g, b, 0, st, L, sl, F64.p, di, tin, out, done);
+      else hipLaunchKernelGGL(k_fwd_list, g, b, 0, st, L, sl, F64.p, di, tin, out, done);
     }
   }
   void precond_apply(const double *tin, double *out, const int *done) {
@@ -1201,11 +1320,28 @@ struct Flow {
         }
       }
     } else {
-      for (const ListLevel &L : sched.lv)
-        hipLaunchKernelGGL(k_ic_factor_list<FT>, dim3(grid_for(L.cnt, 64)), dim3(64), 0, st, L, sched.rows.p,
-                           sl, pairs(), stpos.p, A.p, isdir.p, F, dinv.p, flags.p + 1);
+      factor_levels();
     }
   }
+  // IC(0) level by level (natural order, FP64).  One work-group for levels of at
+  // most kLevOneGroup rows (its threads), 2.5 us a level; wider ones would take
+  // several rounds of its loads, where a launch per level takes 4.1 us.
+  void factor_levels() {
+    const Sell sl = sell();
+    if (sched.tab_ok && sched.width <= kLevOneGroup) {
+      hipLaunchKernelGGL(k_ic_factor_levels, dim3(1), dim3(512), 0, st, (int)sched.lv.size(), sched.lev.p, n, sl,
+                         sched.tab.p, A.p, isdir.p, F64.p, dinv.p, flags.p + 1);
+      return;
+    }
+    for (const ListLevel &L : sched.lv) {
+      const dim3 g(grid_for(L.cnt, 64)), b(64);
+      if (sched.tab_ok) hipLaunchKernelGGL(k_ic_factor_level, g, b, 0, st, L, n, sl, sched.tab.p, A.p, isdir.p, F64.p,
+                                           dinv.p, flags.p + 1);
+      else hipLaunchKernelGGL(k_ic_factor_list, g, b, 0, st, L, sl, pairs(), stpos.p, A.p, isdir.p, F64.p, dinv.p,
+                              flags.p + 1);
+    }
+  }
+  static constexpr int kLevOneGroup = 512;
   void factor() {
     if (f32) factor_t<float>(F32.p);
     else factor_t<double>(F64.p);
@@ -1330,9 +1466,7 @@ struct Flow {
     if (column_order()) {
       for (const ColDesc &C : sched.cols) launch_fwd_col3<FT>(C, sl, F, dinv.p, tin, out, done);
     } else {
-      for (const ListLevel &L : sched.lv)
-        hipLaunchKernelGGL(k_fwd_list<FT>, dim3(grid_for(L.cnt, 64)), dim3(64), 0, st, L, sched.rows.p, sl, F,
-                           dinv.p, tin, out, done);
+      sweep_levels<false>(dinv.p, tin, out, done);
     }
   }
   template <typename FT>
@@ -1341,11 +1475,7 @@ struct Flow {
     if (column_order()) {
       for (size_t c = sched.cols.size(); c-- > 0;) launch_bwd_col3<FT>(sched.cols[c], sl, F, ones.p, xin, out, done);
     } else {
-      for (size_t l = sched.lv.size(); l-- > 0;) {
-        const ListLevel &L = sched.lv[l];
-        hipLaunchKernelGGL(k_bwd_list<FT>, dim3(grid_for(L.cnt, 64)), dim3(64), 0, st, L, sched.rows.p, sl, F,
-                           ones.p, xin, out, done);
-      }
+      sweep_levels<true>(ones.p, xin, out, done);
     }
   }
   void ilu_fwd(const double *tin, double *out, const int *done) {
@@ -1365,8 +1495,7 @@ struct Flow {
                            sl, pairs(), stpos.p, A.p, isdir.p, F, dinv.p, flags.p + 1);
     } else {
       for (const ListLevel &L : sched.lv)
-        hipLaunchKernelGGL(k_ilu_factor_list<FT>, dim3(grid_for(L.cnt, 64)), dim3(64), 0, st, L, sched.rows.p,
-                           sl, pairs(), stpos.p, A.p, isdir.p, F, dinv.p, flags.p + 1);
+        hipLaunchKernelGGL(k_ilu_factor_list<FT>, dim3(grid_for(L.cnt, 64)), dim3(64), 0, st, L, sl, pairs(), stpos.p, A.p, isdir.p, F, dinv.p, flags.p + 1);
     }
   }
   size_t ilu_smem(const ColDesc &C) const { return (sizeof(double) * 3 + sizeof(int) * 3) * (size_t)C.len * kChains; }

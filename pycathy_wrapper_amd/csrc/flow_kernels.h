@@ -192,7 +192,7 @@ __device__ __forceinline__ int chain_lds(const ColDesc &C, int tl, int k) {
 }
 __device__ __forceinline__ int chain_step(const ColDesc &C) { return C.tw == 1 ? 1 : kChains; }
 
-// One level of the natural-order schedule: rows lvl_rows[off .. off+cnt).
+// One level of the natural-order schedule: rows [off, off+cnt).
 struct ListLevel {
   int off, cnt;
 };
@@ -318,15 +318,36 @@ __global__ void k_bwd_col3(ColDesc C, Sell sl, const FT *F, const double *dinv, 
 // Gather window of the column sweeps: the smallest instantiated size that
 // covers n slots (larger rows take the kernels' loop).
 inline int sweep_window(int n) { return n <= 0 ? 0 : (n <= 4 ? 4 : (n <= 8 ? 8 : (n <= 12 ? 12 : 16))); }
-template <typename FT>
-__global__ void k_ic_factor_list(ListLevel L, const int *rows, Sell sl, PairList pl, const int *tpos,
-                                 const double *A, const uint8_t *isdir, FT *F, double *dinv, int *nfall);
-template <typename FT>
-__global__ void k_fwd_list(ListLevel L, const int *rows, Sell sl, const FT *F, const double *dinv,
-                           const double *tin, double *y, const int *done);
-template <typename FT>
-__global__ void k_bwd_list(ListLevel L, const int *rows, Sell sl, const FT *F, const double *dinv,
-                           const double *xin, double *x, const int *done);
+__global__ void k_ic_factor_list(ListLevel L, Sell sl, PairList pl, const int *tpos, const double *A,
+                                 const uint8_t *isdir, double *F, double *dinv, int *nfall);
+__global__ void k_fwd_list(ListLevel L, Sell sl, const double *F, const double *dinv, const double *tin, double *y,
+                           const int *done);
+__global__ void k_bwd_list(ListLevel L, Sell sl, const double *F, const double *dinv, const double *xin, double *x,
+                           const int *done);
+// Level tables of the natural order: kLevWords words per row, word w of row
+// r at w[w * n + r]: byte j(j-1)/2 + a (a < j < kLevLow) = slot b of row
+// c = col(r, j) with col(c, b) = col(r, a), or 0xFF; byte NP + j = the slot of
+// r in row col(r, j).
+constexpr int kLevLow = 8;    // most lower entries of a row
+constexpr int kLevWords = 9;  // 28 + 8 bytes
+__global__ void k_ic_factor_level(ListLevel L, int n, Sell sl, const uint32_t *tab, const double *A,
+                                  const uint8_t *isdir, double *F, double *dinv, int *nfall);
+__global__ void k_ic_factor_levels(int nlev, const int *lev, int n, Sell sl, const uint32_t *tab, const double *A,
+                                   const uint8_t *isdir, double *F, double *dinv, int *nfall);
+constexpr int kRingRows = 8192;   // most rows of the sweeps' LDS ring (64 KB)
+// One direction of the one-work-group sweeps, per row: the SELL position of its
+// first slot (lower entries forward, upper entries backward) and kRingWords
+// words, word i of row r at idx[i * n + r]: the ring positions (column mod ring
+// rows, 14 bits each) of entries 2i and 2i + 1, and in the top four bits of
+// word 0 their count.
+constexpr int kRingWords = kLevLow / 2;
+struct LevSweep {
+  const uint32_t *q0, *idx;
+};
+template <bool UP, int NW>
+__global__ void k_sweep_levels(int nlev, const int *lev, int n, LevSweep S, const double *F, const double *dinv,
+                               const double *tin, double *y, int mask, const int *done);
+__global__ void k_gather(int n, const int *idx, const double *src, double *dst);
 
 __global__ void k_residual0(int n, Sell sl, const double *A, const double *x, const double *b,
                             const uint8_t *isdir, double *r, double *part);
@@ -466,7 +487,7 @@ template <typename FT>
 __global__ void k_ilu_factor_col3(ColDesc C, Sell sl, PairList pl, const int *tpos, const double *A,
                                   const uint8_t *isdir, FT *F, double *dinv, int *nfall);
 template <typename FT>
-__global__ void k_ilu_factor_list(ListLevel L, const int *rows, Sell sl, PairList pl, const int *tpos,
+__global__ void k_ilu_factor_list(ListLevel L, Sell sl, PairList pl, const int *tpos,
                                   const double *A, const uint8_t *isdir, FT *F, double *dinv, int *nfall);
 template <typename FT>
 __global__ void k_mul_upper(int n, Sell sl, const FT *F, const double *x, double *y);

@@ -866,25 +866,24 @@ __global__ __launch_bounds__(256) void k_bwd_col3(ColDesc C, Sell sl, const FT *
   bwd_col3_body<FT, NW>(self_xcd_blk(), smem, C, sl, F, dinv, xin, x, done);
 }
 
-// Natural order: one row per thread, levels of the reference's
-// elimination DAG launched in sequence (exact INCLDP/PRODDP order).
-template <typename FT>
-__global__ void k_ic_factor_list(ListLevel L, const int *__restrict__ rows, Sell sl, PairList pl,
-                                 const int *__restrict__ tpos, const double *__restrict__ A,
-                                 const uint8_t *__restrict__ isdir, FT *__restrict__ F,
-                                 double *__restrict__ dinv, int *nfall) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= L.cnt) return;
-  const int r = rows[L.off + t];
+// ---- natural order: levels of the reference's elimination DAG.  The device
+// numbering sorts the rows by level, so a level is a run of rows, coupled rows
+// keep the reference's elimination order (exact INCLDP / PRODDP), and the
+// rows a level gathers lie in the few levels beside it.
+
+// IC(0) of one row, one level of the pair list at a time (any row length).
+__device__ __forceinline__ void ic_row_list(int r, const Sell &sl, const PairList &pl, const int *__restrict__ tpos,
+                                            const double *__restrict__ A, const uint8_t *__restrict__ isdir,
+                                            double *__restrict__ F, double *__restrict__ dinv, int *nfall) {
   const int jd = sl.diag[r];
   const int base = sl.so[r >> 6] + (r & 63);
   if (isdir[r]) {
     for (int j = 0; j < jd; ++j) {
       const int pj = base + 64 * j;
-      F[pj] = FT(0);
-      F[tpos[pj]] = FT(0);
+      F[pj] = 0.0;
+      F[tpos[pj]] = 0.0;
     }
-    F[base + 64 * jd] = FT(1);
+    F[base + 64 * jd] = 1.0;
     dinv[r] = 0.0;
     return;
   }
@@ -894,8 +893,8 @@ __global__ void k_ic_factor_list(ListLevel L, const int *__restrict__ rows, Sell
     const int c = sl.col[pj];
     double Lv = 0.0;
     if (!isdir[c]) Lv = (A[pj] - pair_dot(pl, F, pj)) * dinv[c];
-    F[pj] = FT(Lv);
-    F[tpos[pj]] = FT(Lv);
+    F[pj] = Lv;
+    F[tpos[pj]] = Lv;
     s -= Lv * Lv;
   }
   if (!(s > 0.0)) {
@@ -904,44 +903,252 @@ __global__ void k_ic_factor_list(ListLevel L, const int *__restrict__ rows, Sell
     atomicAdd(nfall, 1);
   }
   const double d = sqrt(s);
-  F[base + 64 * jd] = FT(d);
+  F[base + 64 * jd] = d;
   dinv[r] = 1.0 / d;
 }
+__global__ void k_ic_factor_list(ListLevel L, Sell sl, PairList pl, const int *__restrict__ tpos,
+                                 const double *__restrict__ A, const uint8_t *__restrict__ isdir,
+                                 double *__restrict__ F, double *__restrict__ dinv, int *nfall) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= L.cnt) return;
+  ic_row_list(L.off + t, sl, pl, tpos, A, isdir, F, dinv, nfall);
+}
 
-template <typename FT>
-__global__ void k_fwd_list(ListLevel L, const int *__restrict__ rows, Sell sl, const FT *__restrict__ F,
-                           const double *__restrict__ dinv, const double *__restrict__ tin,
-                           double *__restrict__ y, const int *__restrict__ done) {
+// The same for rows of at most kLevLow lower entries from the level tables
+// (see kLevWords): a row's loads go out as four batches (its layout; its entries and
+// table words; its neighbours' positions and inverse diagonals; their factor
+// entries) instead of a chain of three dependent loads per entry, and its own
+// entries stay in registers.  Sums in the pair lists' order.
+__device__ __forceinline__ void ic_row_tab(int r, int n, const Sell &sl, const uint32_t *__restrict__ tab,
+                                           const double *__restrict__ A, const uint8_t *__restrict__ isdir,
+                                           double *F, double *dinv, int *nfall) {
+  constexpr int NL = kLevLow, NP = NL * (NL - 1) / 2;
+  const int jd = sl.diag[r];
+  const int base = sl.so[r >> 6] + (r & 63);
+  uint32_t w[kLevWords];
+#pragma unroll
+  for (int i = 0; i < kLevWords; ++i) w[i] = tab[(size_t)i * n + r];
+  const bool rdir = isdir[r] != 0;
+  const double ad = A[base + 64 * jd];
+  int c[NL], sc[NL];
+  double av[NL], dc[NL], G[NP];
+  uint8_t ic[NL];
+#pragma unroll
+  for (int j = 0; j < NL; ++j) {  // entries past the diagonal read index 0 and are not used
+    const int q = j < jd ? base + 64 * j : 0;
+    c[j] = sl.col[q];
+    av[j] = A[q];
+  }
+#pragma unroll
+  for (int j = 0; j < NL; ++j) {
+    const int cj = j < jd ? c[j] : 0;
+    dc[j] = dinv[cj];
+    ic[j] = isdir[cj];
+    sc[j] = sl.so[cj >> 6] + (cj & 63);
+  }
+#pragma unroll
+  for (int j = 1; j < NL; ++j)
+#pragma unroll
+    for (int a = 0; a < j; ++a) {
+      const int q = j * (j - 1) / 2 + a, b = tab_byte(w, q);
+      G[q] = F[b == 0xFF ? 0 : sc[j] + 64 * b];
+    }
+  double s = ad, L[NL];
+#pragma unroll
+  for (int j = 0; j < NL; ++j) {
+    double v = 0.0;
+#pragma unroll
+    for (int a = 0; a < j; ++a) {
+      const int q = j * (j - 1) / 2 + a;
+      v = tab_byte(w, q) != 0xFF ? fma(L[a], G[q], v) : v;
+    }
+    L[j] = (!rdir && j < jd && !ic[j]) ? (av[j] - v) * dc[j] : 0.0;
+    if (j < jd) {
+      F[base + 64 * j] = L[j];
+      F[sc[j] + 64 * tab_byte(w, NP + j)] = L[j];
+    }
+    s -= L[j] * L[j];
+  }
+  if (rdir) {
+    F[base + 64 * jd] = 1.0;
+    dinv[r] = 0.0;
+    return;
+  }
+  if (!(s > 0.0)) {
+    const double a = fabs(ad);
+    s = a > 0.0 ? a : 1.0;
+    atomicAdd(nfall, 1);
+  }
+  const double d = sqrt(s);
+  F[base + 64 * jd] = d;
+  dinv[r] = 1.0 / d;
+}
+// One level over many work-groups (19 us in the pair-list form, 4.1 us here at 387
+// rows).
+__global__ __launch_bounds__(64) void k_ic_factor_level(ListLevel L, int n, Sell sl, const uint32_t *__restrict__ tab,
+                                                        const double *__restrict__ A,
+                                                        const uint8_t *__restrict__ isdir, double *__restrict__ F,
+                                                        double *__restrict__ dinv, int *nfall) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < L.cnt) ic_row_tab(L.off + t, n, sl, tab, A, isdir, F, dinv, nfall);
+}
+// All levels in one work-group, a barrier between levels (2.5 us each: the four
+// batches of loads, then the row's recurrence).  7,056 rows in 86 levels:
+// 1,079 us as a launch of the pair-list form per level, 216 us here.
+__global__ __launch_bounds__(512) void k_ic_factor_levels(int nlev, const int *__restrict__ lev, int n, Sell sl,
+                                                          const uint32_t *__restrict__ tab,
+                                                          const double *__restrict__ A,
+                                                          const uint8_t *__restrict__ isdir, double *F, double *dinv,
+                                                          int *nfall) {
+  for (int l = 0; l < nlev; ++l) {
+    const int r1 = lev[l + 1];
+    for (int r = lev[l] + threadIdx.x; r < r1; r += blockDim.x) ic_row_tab(r, n, sl, tab, A, isdir, F, dinv, nfall);
+    __syncthreads();
+  }
+}
+
+__global__ void k_fwd_list(ListLevel L, Sell sl, const double *__restrict__ F, const double *__restrict__ dinv,
+                           const double *__restrict__ tin, double *__restrict__ y, const int *__restrict__ done) {
   if (done && *done) return;
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= L.cnt) return;
-  const int r = rows[L.off + t];
+  const int r = L.off + t;
   const int jd = sl.diag[r];
   const int base = sl.so[r >> 6] + (r & 63);
   double s = tin[r];
   for (int j = 0; j < jd; ++j) {
     const int pj = base + 64 * j;
-    s -= (double)F[pj] * y[sl.col[pj]];
+    s -= F[pj] * y[sl.col[pj]];
   }
   y[r] = s * dinv[r];
 }
 
-template <typename FT>
-__global__ void k_bwd_list(ListLevel L, const int *__restrict__ rows, Sell sl, const FT *__restrict__ F,
-                           const double *__restrict__ dinv, const double *xin, double *x,
-                           const int *__restrict__ done) {
+__global__ void k_bwd_list(ListLevel L, Sell sl, const double *__restrict__ F, const double *__restrict__ dinv,
+                           const double *xin, double *x, const int *__restrict__ done) {
   if (done && *done) return;
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= L.cnt) return;
-  const int r = rows[L.off + t];
+  const int r = L.off + t;
   const int jd = sl.diag[r], len = sl.len[r];
   const int base = sl.so[r >> 6] + (r & 63);
   double s = xin[r];
   for (int j = jd + 1; j < len; ++j) {
     const int pj = base + 64 * j;
-    s -= (double)F[pj] * x[sl.col[pj]];
+    s -= F[pj] * x[sl.col[pj]];
   }
   x[r] = s * dinv[r];
+}
+
+// A row of a level sweep: factor entries, right-hand side, inverse diagonal and the
+// ring positions of its entries' columns.
+template <int NW>
+struct LevRow {
+  double f[NW], t, di;
+  uint32_t w[kRingWords];
+};
+template <int NW>
+__device__ __forceinline__ void lev_load(LevRow<NW> &R, uint32_t q, const LevSweep &S, int n,
+                                         const double *__restrict__ F, const double *__restrict__ dinv,
+                                         const double *tin, int r) {
+  const char *f = (const char *)F + (size_t)(q * 8u);  // one offset, 512 bytes between slots
+#pragma unroll
+  for (int j = 0; j < NW; ++j) R.f[j] = *(const double *)(f + 512 * j);  // past the row's slots: in bounds, masked
+#pragma unroll
+  for (int i = 0; i < kRingWords; ++i) R.w[i] = S.idx[(size_t)i * n + r];
+  R.t = tin[r];
+  R.di = dinv[r];
+}
+template <int NW>
+__device__ __forceinline__ void lev_solve(const LevRow<NW> &R, double *ring, int mask, double *y, int r) {
+  const int nj = (int)(R.w[0] >> 28);
+  double s = R.t, v[NW];
+#pragma unroll
+  for (int j = 0; j < NW; ++j) v[j] = ring[(R.w[j >> 1] >> (14 * (j & 1))) & 0x3FFFu];
+#pragma unroll
+  for (int j = 0; j < NW; ++j) s = j < nj ? fma(-R.f[j], v[j], s) : s;
+  s *= R.di;
+  ring[r & mask] = s;
+  y[r] = s;
+}
+// The forward (L y = t) or, UP, backward (L^T x = y) sweep over all levels in one
+// work-group.  A level's results stay in an LDS ring of mask + 1 rows that
+// holds every row the next levels gather (the host checks reach + width), so a
+// level costs an LDS gather, the row's products and a barrier on LDS alone: the
+// factor entries of the level after next are on their way, the first slot of its
+// rows two levels before them, and the level bounds lie in LDS.  Bound by
+// that chain for narrow levels and by one CU's loads (100 bytes a row) for wide
+// ones: 7,056 rows in 86 levels take 53 us (a launch per level: 330 us), 66,885
+// rows in 173 levels 180 us (950 us).  The rows beyond one per thread load as
+// they come.
+template <bool UP, int NW>
+__global__ __launch_bounds__(1024) void k_sweep_levels(int nlev, const int *__restrict__ lev, int n, LevSweep S,
+                                                       const double *__restrict__ F,
+                                                       const double *__restrict__ dinv, const double *tin, double *y,
+                                                       int mask, const int *__restrict__ done) {
+  extern __shared__ double ring[];
+  int *bound = (int *)(ring + mask + 1);
+  if (done && *done) return;
+  const int tid = threadIdx.x;
+  for (int i = tid; i <= nlev; i += blockDim.x) bound[i] = lev[i];
+  __syncthreads();
+  // bounds of the l-th level swept (empty past the last) and this thread's row in it (n: none)
+  auto bounds = [&](int l) {
+    const int k = min(max(UP ? nlev - 1 - l : l, 0), nlev - 1);
+    return make_int2(bound[k], l < nlev ? bound[k + 1] : 0);
+  };
+  auto row = [&](int2 b) { return b.x + tid < b.y ? b.x + tid : n; };
+  LevRow<NW> R[2];
+  uint32_t Q[2];
+  int2 B[2], cur[2];
+  int rr[2], rm[2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    cur[p] = bounds(p);
+    rr[p] = row(cur[p]);
+    if (rr[p] < n) lev_load(R[p], S.q0[rr[p]], S, n, F, dinv, tin, rr[p]);
+    rm[p] = row(bounds(2 + p));
+    Q[p] = rm[p] < n ? S.q0[rm[p]] : 0u;
+    B[p] = bounds(4 + p);
+  }
+  for (int l0 = 0; l0 < nlev; l0 += 2) {
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int l = l0 + p;
+      if (l >= nlev) break;
+      if (rr[p] < n) lev_solve(R[p], ring, mask, y, rr[p]);
+      rr[p] = rm[p];
+      if (rr[p] < n) lev_load(R[p], Q[p], S, n, F, dinv, tin, rr[p]);
+      rm[p] = row(B[p]);
+      if (rm[p] < n) Q[p] = S.q0[rm[p]];
+      B[p] = bounds(l + 6);
+      if (cur[p].y - cur[p].x > (int)blockDim.x)
+        for (int r = cur[p].x + tid + blockDim.x; r < cur[p].y; r += blockDim.x) {
+          LevRow<NW> X;
+          lev_load(X, S.q0[r], S, n, F, dinv, tin, r);
+          lev_solve(X, ring, mask, y, r);
+        }
+      cur[p] = bounds(l + 2);
+      // results pass between threads through the ring only: wait for LDS, not
+      // for the loads under way
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    }
+  }
+}
+#define CG_INST_LEV(NW)                                                                                              \
+  template __global__ void k_sweep_levels<false, NW>(int, const int *, int, LevSweep, const double *, const double *, \
+                                                     const double *, double *, int, const int *);                     \
+  template __global__ void k_sweep_levels<true, NW>(int, const int *, int, LevSweep, const double *, const double *,  \
+                                                    const double *, double *, int, const int *);
+CG_INST_LEV(7)
+CG_INST_LEV(8)
+#undef CG_INST_LEV
+
+// dst[i] = src[idx[i]]
+__global__ void k_gather(int n, const int *__restrict__ idx, const double *__restrict__ src, double *__restrict__ dst) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) dst[i] = src[idx[i]];
 }
 
 #define CG_INST_SWEEP(FT, U)                                                                              \
@@ -965,13 +1172,7 @@ __global__ void k_bwd_list(ListLevel L, const int *__restrict__ rows, Sell sl, c
   CG_INST_SWEEP(FT, 4)                                                                                      \
   CG_INST_SWEEP(FT, 8)                                                                                      \
   CG_INST_SWEEP(FT, 12)                                                                                     \
-  CG_INST_SWEEP(FT, 16)                                                                                     \
-  template __global__ void k_ic_factor_list<FT>(ListLevel, const int *, Sell, PairList, const int *,        \
-                                                const double *, const uint8_t *, FT *, double *, int *);    \
-  template __global__ void k_fwd_list<FT>(ListLevel, const int *, Sell, const FT *, const double *,         \
-                                          const double *, double *, const int *);                          \
-  template __global__ void k_bwd_list<FT>(ListLevel, const int *, Sell, const FT *, const double *,          \
-                                          const double *, double *, const int *);
+  CG_INST_SWEEP(FT, 16)
 CG_INST_FT(float)
 CG_INST_FT(double)
 #undef CG_INST_FT

@@ -1,7 +1,7 @@
 // kernels.h -- gfx950 kernels of the CATHY subsurface Picard step.
 //
-// Device numbering: node ids are permuted at set-up (ordering NATURAL keeps
-// CATHY's, COLUMN3 groups whole soil columns by a 3-colouring of the
+// Device numbering: node ids are permuted at set-up (ordering NATURAL sorts
+// CATHY's by elimination level, COLUMN3 groups whole soil columns by a 3-colouring of the
 // surface mesh so IC(0) sweeps run column-parallel).  Every vector below is
 // in device numbering; the full CSR (rowptr/col, sorted columns) holds the
 // symmetric system matrix (FP64) and, in the same pattern, the IC(0) factor

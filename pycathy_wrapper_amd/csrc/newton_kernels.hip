@@ -251,13 +251,13 @@ __global__ __launch_bounds__(256) void k_ilu_factor_col3(ColDesc C, Sell sl, Pai
 // Crout ILU(0), natural order, one level: each row of the level computes
 // its lower slots in ascending order, then its diagonal.
 template <typename FT>
-__global__ void k_ilu_factor_list(ListLevel Lv, const int *__restrict__ rows, Sell sl, PairList pl,
+__global__ void k_ilu_factor_list(ListLevel Lv, Sell sl, PairList pl,
                                   const int *__restrict__ tpos, const double *__restrict__ A,
                                   const uint8_t *__restrict__ isdir, FT *__restrict__ F,
                                   double *__restrict__ dinv, int *nfall) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= Lv.cnt) return;
-  const int r = rows[Lv.off + t];
+  const int r = Lv.off + t;
   const RowPos rp = row_pos(sl, r);
   const int jd = sell_diag(sl, rp, r);
   const int base = sl.so[r >> 6] + (r & 63);
@@ -297,7 +297,7 @@ __global__ void k_ilu_factor_list(ListLevel Lv, const int *__restrict__ rows, Se
 #define CG_INST_ILU(FT)                                                                                  \
   template __global__ void k_ilu_factor_col3<FT>(ColDesc, Sell, PairList, const int *, const double *,     \
                                                  const uint8_t *, FT *, double *, int *);                  \
-  template __global__ void k_ilu_factor_list<FT>(ListLevel, const int *, Sell, PairList, const int *,      \
+  template __global__ void k_ilu_factor_list<FT>(ListLevel, Sell, PairList, const int *,                   \
                                                  const double *, const uint8_t *, FT *, double *, int *);
 CG_INST_ILU(float)
 CG_INST_ILU(double)
