@@ -29,8 +29,15 @@ namespace {
 
 constexpr int kMaxMembers = 512;
 
-// launch shapes of the batched kernels: groups per member
-enum Shape { kShRows = 0, kShRed, kShNnod, kShFlux, kShOne, kShVec, kShCol0, kNShape = kShCol0 + 4 };
+// launch shapes of the batched kernels: groups per member.  kShRows .. kShCol3
+// hold every member; the PCG's kernels run either over surface tiles
+// (kShTile.., members with Flow::tiles()) or colour by colour (kShSpmv ..
+// kShSweep3, the others).
+enum Shape {
+  kShRows = 0, kShRed, kShNnod, kShFlux, kShOne, kShCol0,
+  kShTile = kShCol0 + 4, kShTileRows, kShTileOne,
+  kShSpmv, kShVec, kShSweep0, kNShape = kShSweep0 + 4
+};
 
 int shape_groups(const Flow &f, int sh) {
   switch (sh) {
@@ -39,9 +46,14 @@ int shape_groups(const Flow &f, int sh) {
     case kShNnod: return grid_for(f.nnod);
     case kShFlux: return grid_for(f.nnod, kBlock, kMaxRedBlocks);
     case kShOne: return 1;
-    case kShVec: return std::min(grid_for(f.n), kVecGroups);
+    case kShTile: return f.tiles() ? f.ntile : 0;
+    case kShTileRows: return f.tiles() ? grid_for(f.n) : 0;
+    case kShTileOne: return f.tiles() ? 1 : 0;
+    case kShSpmv: return f.tiles() ? 0 : grid_for(f.n);
+    case kShVec: return f.tiles() ? 0 : std::min(grid_for(f.n), kVecGroups);
     default: {
-      const int c = sh - kShCol0;
+      if (sh >= kShSweep0 && f.tiles()) return 0;
+      const int c = sh >= kShSweep0 ? sh - kShSweep0 : sh - kShCol0;
       return c < (int)f.sched.cols.size() ? grid_for(f.sched.cols[c].nc, kChains) : 0;
     }
   }
@@ -55,7 +67,8 @@ struct Ensemble {
   bool f32 = true;
   int mr = 16, ncol = 0;
   int wfac[4] = {0, 0, 0, 0}, wf[4] = {0, 0, 0, 0}, wb[4] = {0, 0, 0, 0};
-  size_t sm_col[4] = {0, 0, 0, 0}, sm_fac[4] = {0, 0, 0, 0};
+  size_t sm_col[4] = {0, 0, 0, 0}, sm_fac[4] = {0, 0, 0, 0}, sm_tile = 0;
+  int rpt_tile = 1, thr_tile = 0;  // rows per thread and threads that cover every member's tiles
   bool fuse_last = false;
   DBuf<MemberDev> dargs;
   Pinned<MemberDev> hargs;
@@ -147,6 +160,11 @@ struct Ensemble {
       CG_REQUIRE(f.ftab_ok, who + "the IC(0) chain tables do not apply to this mesh");
       CG_REQUIRE(f.f32 == f32, who + "members differ in IC(0) factor precision");
       CG_REQUIRE((int)f.sched.cols.size() == ncol && ncol >= 1 && ncol <= 4, who + "members differ in colour count");
+      if (f.tiles_on) {
+        sm_tile = std::max(sm_tile, f.tile_smem());
+        rpt_tile = std::max(rpt_tile, f.tile_rpt);
+        thr_tile = std::max(thr_tile, f.tile_threads);
+      }
       for (int c = 0; c < ncol; ++c) {
         const ColDesc &C = f.sched.cols[c];
         CG_REQUIRE(sweep_window(C.nf) <= 12, who + "a row has more earlier-colour slots than the table factor takes");
@@ -187,7 +205,7 @@ struct Ensemble {
   }
 
   MemberDev member_dev(int j) const {
-    const Flow &f = *mem[j];
+    Flow &f = *mem[j];
     MemberDev d{};
     d.n = f.n;
     d.nnod = f.nnod;
@@ -222,15 +240,20 @@ struct Ensemble {
     d.row_surf = f.row_surf.p; d.surf_row = f.surf_row.p; d.refid = f.refid.p;
     d.volnod = f.volnod.p; d.snodi = f.snodi.p; d.pnodi = f.pnodi.p;
     d.scal = f.scal.p;
+    d.tiles = f.tile_set();
+    if (f.tiles_on) d.tpcg = f.tile_pcg();
     return d;
   }
 
   // ---------------------------------------------------- batched launches --
   template <typename K, typename... A>
-  void launch(K kern, int sh, size_t smem, A... args) {
+  void launch_b(K kern, int sh, size_t smem, int block, A... args) {
     if (gtot[sh] == 0) return;
-    hipLaunchKernelGGL(kern, dim3(gtot[sh]), dim3(kBlock), smem, st, tab(sh), nm, (const MemberDev *)dargs.p,
-                       args...);
+    hipLaunchKernelGGL(kern, dim3(gtot[sh]), dim3(block), smem, st, tab(sh), nm, (const MemberDev *)dargs.p, args...);
+  }
+  template <typename K, typename... A>
+  void launch(K kern, int sh, size_t smem, A... args) {
+    launch_b(kern, sh, smem, kBlock, args...);
   }
 
   template <typename FT>
@@ -247,7 +270,7 @@ struct Ensemble {
   }
   template <typename FT, bool LAST>
   void fwd_t(int c, int vin, int vout, int use_done) {
-    const int sh = kShCol0 + c;
+    const int sh = kShSweep0 + c;
     const size_t sm = (LAST ? 2 : 1) * sm_col[c];
     switch (wf[c]) {
       case 0: launch(kb_fwd_col3<FT, 0, LAST>, sh, sm, c, vin, vout, use_done); break;
@@ -259,7 +282,7 @@ struct Ensemble {
   }
   template <typename FT>
   void bwd_t(int c, int vio, int use_done) {
-    const int sh = kShCol0 + c;
+    const int sh = kShSweep0 + c;
     switch (wb[c]) {
       case 0: launch(kb_bwd_col3<FT, 0>, sh, sm_col[c], c, vio, use_done); break;
       case 4: launch(kb_bwd_col3<FT, 4>, sh, sm_col[c], c, vio, use_done); break;
@@ -281,7 +304,18 @@ struct Ensemble {
     if (f32) factor_t<float>();
     else factor_t<double>();
   }
+  template <int MODE>
+  void tile(int vin, int vout) {
+    if (f32) tile_t<float, MODE>(vin, vout);
+    else tile_t<double, MODE>(vin, vout);
+  }
+  template <typename FT, int MODE>
+  void tile_t(int vin, int vout) {
+    auto k = rpt_tile == 1 ? kb_tile<FT, MODE, 1> : kb_tile<FT, MODE, 2>;
+    launch_b(k, kShTile, sm_tile, thr_tile, vin, vout);
+  }
   void precond(int vin, int vout, int use_done) {
+    if (!use_done) tile<kTileSolve>(vin, vout);
     if (f32) precond_t<float>(vin, vout, use_done);
     else precond_t<double>(vin, vout, use_done);
   }
@@ -290,7 +324,9 @@ struct Ensemble {
   // the same launches and batch policy, one launch per kernel for all.
   // one PCG iteration for every member still iterating (graddp.f:1325-1377)
   void pcg_iteration() {
-    launch(kb_spmv_dot2, kShRows, 0);
+    launch(kb_spmv_beta, kShTileRows, 0);
+    tile<kTilePcg>(0, 0);
+    launch(kb_spmv_dot2, kShSpmv, 0);
     launch(kb_pcg_alpha, kShVec, 0);
     precond(kVecR, kVecZ, 1);
     launch(kb_dot, kShVec, 0);
@@ -347,6 +383,7 @@ struct Ensemble {
       }
       launched += batch;
       ++pcg_batches;
+      launch(kb_pcg_check, kShTileOne, 0);
       launch(kb_poll, kShOne, 0, dpoll.p);
       CG_HIP(hipMemcpyAsync(hpoll.p, dpoll.p, sizeof(double) * 3 * nm, hipMemcpyDeviceToHost, st));
       CG_HIP(hipStreamSynchronize(st));

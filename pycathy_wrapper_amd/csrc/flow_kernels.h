@@ -200,6 +200,7 @@ struct ListLevel {
 struct PcgScal {
   double xlung, pb, alpha, err, tol;
   int niter, imax;
+  int it;  // iterations finished (tile path only)
 };
 
 struct NormPart {
@@ -410,6 +411,48 @@ __global__ void k_sumsq_free(int n, const double *u, const uint8_t *isdir, doubl
 __global__ void k_copy(size_t n, const double *src, double *dst);
 __global__ void k_fill(size_t n, double v, double *dst);
 
+// ------------------------------------- the PCG over surface tiles (tiles.h) --
+// A tile's columns in LDS order: colour 0, 1, 2; within a colour those whose final
+// x is needed first (x0: the tile's own), and the tile's own first of all.
+struct TileDesc {
+  int off, row;      // first entry of the tile's columns in the table, of its rows in TileSet::rows
+  int n[3];          // columns of each colour whose forward sweep runs here
+  int x1;            // colour-1 columns whose backward sweep runs here (prefix)
+  int own[3];        // the tile's own columns of each colour (prefix)
+};
+// Table words per (plane type, column of the tile): six of 16-bit entries for the
+// slots of earlier colours, six for those of later colours, one with the
+// diagonal slot and the two counts.  Entry: (dk + 1) * (columns of the tile) + local
+// column, the LDS distance from the tile's first column one plane up (entries past
+// the count repeat the first, or name the row itself); word w of
+// plane type pt and column l of the tile at tab[((pt * kTileWords + w) * ntot) + off + l].
+constexpr int kTileWords = 13;
+constexpr int kTileSlots = 12;   // entries of colour 2 forward, colour 0 back
+constexpr int kTileSlots1 = 8;   // of colour 1
+struct TileSet {
+  const TileDesc *desc;
+  const int2 *rows;        // (row id, SELL position of its slot 0), tile by tile, [plane][column]
+  const uint32_t *tab;
+  int ntile, ntot;         // tiles, columns of all tiles
+  int threads;             // that share a phase's rows (a batched launch may have more)
+};
+struct TileCols {
+  ColDesc c[3];
+};
+
+// State of a PCG solve on tiles: search directions and residuals alternate
+// between two buffers (a tile reads its neighbours' old values while they write
+// new ones), picked by the iteration count on the device.
+struct TilePcg {
+  double *p[2], *r[2], *z, *B, *x;
+  double *part_pr, *part_pb, *part_bz, *part_rr;
+  const double *A, *dinv;
+  const uint8_t *isdir;
+  PcgScal *sc;
+  int *done;
+  int n;
+};
+
 // ------------------------------------------ batched ensemble launches --
 // Everything one member's Picard iteration and IC(0)-PCG read or write,
 // held in device memory per member (an array over the ensemble).  A batched
@@ -438,6 +481,8 @@ struct MemberDev {
   const int *row_surf, *surf_row, *refid;
   const double *volnod, *snodi, *pnodi;
   PcgScal *scal;
+  TileSet tiles;               // the PCG over surface tiles (ntile 0: not used)
+  TilePcg tpcg;
 };
 // vectors a batched sweep reads / writes
 enum SweepVec { kVecTnoti = 0, kVecPdiff, kVecR, kVecP, kVecZ };

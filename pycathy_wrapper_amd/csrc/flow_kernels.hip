@@ -1422,6 +1422,7 @@ __device__ __forceinline__ void pcg_init_body(Blk bk, int nparts, const double *
     sc->tol = tol;
     sc->imax = imax;
     sc->niter = 1;
+    sc->it = 0;
     sc->err = 0.0;
     *done = 0;
   }
