@@ -482,10 +482,7 @@ int cathy_gpu_flow3d_set_pnew(int64_t *handle, const double *pnew) {
   return guarded([&] {
     const std::shared_ptr<Flow> f = lookup(handle);
     CG_REQUIRE(pnew, "null argument");
-    std::vector<double> h(f->n);
-    for (int i = 0; i < f->n; ++i) h[f->perm[i]] = pnew[i];
-    f->pnew.upload(h, f->st);
-    CG_HIP(hipStreamSynchronize(f->st));
+    f->put_nodes(pnew, f->pnew.p);
     return 0;
   });
 }

@@ -171,6 +171,7 @@ struct Flow {
   int ftab_nch = 0;
   bool ftab_ok = false;
   DBuf<double> dbeta;
+  std::vector<double> h_arenod;
   DBuf<int> inc_ptr, inc, refid, row_surf, surf_row, bot_row;
   DBuf<uint32_t> incoff;
   DBuf<int4> enode;
@@ -252,6 +253,11 @@ struct Flow {
     double v;
   };
   Pinned<HostBox> hbox;
+  // nodal values in CATHY's order on their way to or from the caller: the
+  // permutation runs on the device, so the caller's array is the only host
+  // copy.  The lock keeps readers in different threads from each other's values.
+  DBuf<double> iob;
+  std::mutex io_mu;
 
   // host time / balance state (cathy_main.f)
   Params prm;
@@ -1401,7 +1407,8 @@ struct Flow {
     volnod.upload(a_volnod, st); kznod.upload(a_kz, st);
     refid.upload(hrefid, st); row_surf.upload(hrow_surf, st); surf_row.upload(hsurf_row, st);
     bot_row.upload(hbot_row, st);
-    arenod.upload(std::vector<double>(arenod_, arenod_ + nnod), st);
+    h_arenod.assign(arenod_, arenod_ + nnod);
+    arenod.upload(h_arenod, st);
     CG_HIP(hipStreamSynchronize(st));
   }
 
@@ -1415,8 +1422,33 @@ struct Flow {
     pond.alloc(1);
     hipLaunchKernelGGL(k_put_int, dim3(1), dim3(64), 0, st, pond.p, 0);
     atmpot.alloc(nnod); atmact.alloc(nnod); atmold.alloc(nnod); qbot.alloc(nnod);
+    iob.alloc(n);
     alloc_solver();
     CG_HIP(hipMemsetAsync(qnode.p, 0, sizeof(double) * n, st));
+  }
+  // Nodal values of the caller (CATHY's order) to device rows, and to a second array.
+  void put_nodes(const double *h, double *d, double *d2 = nullptr) {
+    std::lock_guard<std::mutex> lk(io_mu);
+    iob.upload(h, n, st);
+    hipLaunchKernelGGL(k_from_cathy, dim3(grid_for(n)), dim3(kBlock), 0, st, n, refid.p, iob.p, d, d2);
+    CG_HIP(hipStreamSynchronize(st));
+  }
+  // Device rows to the caller's array in CATHY's order.  Small meshes are permuted
+  // by the host, which takes less than the launch does: 4,851 nodes 13 us against 26,
+  // 26,896 27 / 34, 54,621 45 / 45, 131,000 96 / 76, 1,252,431 1010 / 712.
+  static constexpr int kHostOrderRows = 50000;
+  void get_nodes(const double *d, double *h) {
+    if (n <= kHostOrderRows) {
+      std::vector<double> v(n);
+      CG_HIP(hipMemcpyAsync(v.data(), d, sizeof(double) * n, hipMemcpyDeviceToHost, st));
+      CG_HIP(hipStreamSynchronize(st));
+      for (int i = 0; i < n; ++i) h[i] = v[perm[i]];
+      return;
+    }
+    std::lock_guard<std::mutex> lk(io_mu);
+    hipLaunchKernelGGL(k_to_cathy, dim3(grid_for(n)), dim3(kBlock), 0, st, n, refid.p, d, iob.p);
+    iob.download(h, n, st);
+    CG_HIP(hipStreamSynchronize(st));
   }
   // what SYMSLV needs: matrix, factor, PCG vectors and reduction scratch
   void alloc_solver() {
@@ -2120,17 +2152,24 @@ struct Flow {
     ksf = 0;
   }
   // sfinit.f:22-45: a seepage node at or above 1e-8 m of head starts as an
-  // exit node with PTIMEP = PNEW = 0 (hp: PNEW = PTIMEP by CATHY id order of
-  // device rows)
-  void sfinit(std::vector<double> &hp) {
+  // exit node with PTIMEP = PNEW = 0, on the device and in hp (psi: the heads
+  // given in CATHY's order; hp: those of the surface)
+  void sfinit(const double *psi, std::vector<double> &hp) {
     if (nsf_nodes == 0) return;
-    std::vector<int> e(nsf_nodes, 0);
-    for (int i = 0; i < nsf_nodes; ++i) {
-      const int r = perm[sf_node[i]];
-      if (hp[r] >= 1.0e-8) {
+    std::vector<int> e(nsf_nodes, 0), rows;
+    for (int i = 0; i < nsf_nodes; ++i)
+      if (psi[sf_node[i]] >= 1.0e-8) {
         e[i] = 1;
-        hp[r] = 0.0;
+        if (sf_node[i] < nnod) hp[sf_node[i]] = 0.0;
+        rows.push_back(perm[sf_node[i]]);
       }
+    if (!rows.empty()) {
+      DBuf<int> dr(rows.size());
+      dr.upload(rows, st);
+      for (double *x : {pnew.p, ptimep.p})
+        hipLaunchKernelGGL(k_set_rows, dim3(grid_for(rows.size())), dim3(kBlock), 0, st, (int)rows.size(), dr.p,
+                           (const double *)nullptr, 0.0, x);
+      CG_HIP(hipStreamSynchronize(st));
     }
     sfex.upload(e, st);
     sfexit.upload(e, st);
@@ -2558,9 +2597,7 @@ struct Flow {
     CG_REQUIRE(!atm_t.empty(), "forcing not set");
     CG_REQUIRE(atm_w == arow() && atm_v.size() == atm_t.size() * (size_t)arow(),
                "forcing records do not match HSPATM (set the parameters before the forcing)");
-    std::vector<double> h(n);
-    for (int i = 0; i < n; ++i) h[perm[i]] = ptimep_ref[i];
-    ptimep.upload(h, st);
+    put_nodes(ptimep_ref, ptimep.p, pnew.p);
     // inital.f:201-205: PONDING starts clear (IPOND = 0); INIT_SR (init_sr.f)
     hipLaunchKernelGGL(k_put_int, dim3(1), dim3(64), 0, st, pond.p, 0);
     if (rt) routing_reset();
@@ -2579,7 +2616,6 @@ struct Flow {
     iter = 1; nstep = 1; nitert = 0; itlin = 0; itrtot = 0; klsfai = 0;
     finished = 0; noback = 0; bckstp = 0;
     store1 = store2 = dstore = cdstor = cvin = cvout = vtot = cerras = caeras = 0.0;
-    CG_HIP(hipMemcpyAsync(pnew.p, ptimep.p, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
     // BCONE of the fixed-head and Neumann series at TIME = DELTAT (inital.f:160-181)
     CG_REQUIRE(!(lists_on() || veg_on) || prm.iopt == 1, "listed boundary conditions and root uptake need IOPT=1");
     alloc_lists();
@@ -2591,14 +2627,9 @@ struct Flow {
     atminp.assign((size_t)3 * w, 0.0);
     atm_next = 0; htiatm = 0;
     atmtim[0] = atmtim[1] = atmtim[2] = 0.0;
-    std::vector<double> hp(n);
-    pnew.download(hp.data(), n, st);
-    CG_HIP(hipStreamSynchronize(st));
     std::vector<int> fa(nnod, 0), fap(nnod, 0);
     std::vector<double> apot(nnod, 0.0), aact(nnod, 0.0), aold(nnod, 0.0);
-    std::vector<double> are(nnod);
-    arenod.download(are.data(), nnod, st);
-    CG_HIP(hipStreamSynchronize(st));
+    const std::vector<double> &are = h_arenod;
     double *a3 = atminp.data() + 2 * (size_t)w;
     double tin;
     auto rate_at = [&](int slot, int s) { return atminp[(size_t)slot * w + (w > 1 ? s : 0)]; };
@@ -2621,25 +2652,34 @@ struct Flow {
         apot[s] = rt * are[s];
       }
     }
-    sfinit(hp);                    // inital.f:226-229, ahead of ATMONE
-    std::vector<double> hpt = hp;  // PTIMEP == PNEW here
+    // surface heads PNEW, and PTIMEP, which is PNEW here
+    std::vector<double> hp(ptimep_ref, ptimep_ref + nnod);
+    sfinit(ptimep_ref, hp);        // inital.f:226-229, ahead of ATMONE
+    std::vector<double> hpt = hp;
     for (int s : h_atm_off) fa[s] = fap[s] = -1;  // atmone.f:87-109, ahead of the classification
+    bool moved = false;
     for (int s = 0; s < nnod; ++s) {
-      const int d = perm[s];
       if (fa[s] == -1) continue;
-      if (hp[d] >= prm.pondh_min) { fa[s] = 2; fap[s] = 2; continue; }
-      if (hp[d] >= 0.0 && apot[s] > 0.0) fa[s] = 1;
-      if (hpt[d] >= 0.0 && aold[s] > 0.0) fap[s] = 1;
-      if (hp[d] <= prm.pmin && apot[s] < 0.0) { hp[d] = prm.pmin; fa[s] = 1; }
-      if (hpt[d] <= prm.pmin && aold[s] < 0.0) { hpt[d] = prm.pmin; fap[s] = 1; }
+      if (hp[s] >= prm.pondh_min) { fa[s] = 2; fap[s] = 2; continue; }
+      if (hp[s] >= 0.0 && apot[s] > 0.0) fa[s] = 1;
+      if (hpt[s] >= 0.0 && aold[s] > 0.0) fap[s] = 1;
+      if (hp[s] <= prm.pmin && apot[s] < 0.0) { hp[s] = prm.pmin; fa[s] = 1; moved = true; }
+      if (hpt[s] <= prm.pmin && aold[s] < 0.0) { hpt[s] = prm.pmin; fap[s] = 1; moved = true; }
     }
-    ptimep.upload(hpt, st);
+    if (moved) {
+      std::lock_guard<std::mutex> lk(io_mu);
+      for (auto hd : {std::make_pair(&hpt, ptimep.p), std::make_pair(&hp, pnew.p)}) {
+        iob.upload(*hd.first, st);
+        hipLaunchKernelGGL(k_set_rows, dim3(grid_for(nnod)), dim3(kBlock), 0, st, nnod, surf_row.p, iob.p, 0.0,
+                           hd.second);
+      }
+      CG_HIP(hipStreamSynchronize(st));
+    }
     for (int s = 0; s < nnod; ++s) {
       if (fa[s] == 0) aact[s] = apot[s] >= 0.0 ? apot[s] : (1.0 - prm.scf) * apot[s];
       else aact[s] = 0.0;
       if (fap[s] == 1 || fap[s] == 2) aold[s] = 0.0;
     }
-    pnew.upload(hp, st);
     ifatm.upload(fa, st); ifatmp.upload(fap, st);
     atmpot.upload(apot, st); atmact.upload(aact, st); atmold.upload(aold, st);
     const int gn = grid_for(n);
@@ -3032,13 +3072,8 @@ struct Flow {
     if (vv) e_vv.download(vv, nt, st);
     if (ww) e_ww.download(ww, nt, st);
     CG_HIP(hipStreamSynchronize(st));
-    std::vector<double> h(n);
-    for (auto pr : {std::make_pair(&n_u, unod), std::make_pair(&n_v, vnod), std::make_pair(&n_w, wnod)}) {
-      if (!pr.second) continue;
-      pr.first->download(h.data(), n, st);
-      CG_HIP(hipStreamSynchronize(st));
-      for (int i = 0; i < n; ++i) pr.second[i] = h[perm[i]];
-    }
+    for (auto pr : {std::make_pair(&n_u, unod), std::make_pair(&n_v, vnod), std::make_pair(&n_w, wnod)})
+      if (pr.second) get_nodes(pr.first->p, pr.second);
   }
   int nzone_ = 0, maxstr_ = 0;
 
@@ -3089,15 +3124,9 @@ struct Flow {
   }
 
   void get_state(double *pn, double *swo, double *ck, int *fa) {
-    std::vector<double> h(n);
-    auto fetch = [&](const DBuf<double> &b, double *out) {
-      b.download(h.data(), n, st);
-      CG_HIP(hipStreamSynchronize(st));
-      for (int i = 0; i < n; ++i) out[i] = h[perm[i]];
-    };
-    if (pn) fetch(pnew, pn);
-    if (swo) fetch(sw, swo);
-    if (ck) fetch(ckrw, ck);
+    if (pn) get_nodes(pnew.p, pn);
+    if (swo) get_nodes(sw.p, swo);
+    if (ck) get_nodes(ckrw.p, ck);
     if (fa) {
       ifatm.download(fa, nnod, st);
       CG_HIP(hipStreamSynchronize(st));

@@ -348,6 +348,8 @@ struct LevSweep {
 template <bool UP, int NW>
 __global__ void k_sweep_levels(int nlev, const int *lev, int n, LevSweep S, const double *F, const double *dinv,
                                const double *tin, double *y, int mask, const int *done);
+__global__ void k_from_cathy(int n, const int *refid, const double *h, double *d, double *d2);
+__global__ void k_to_cathy(int n, const int *refid, const double *d, double *h);
 __global__ void k_gather(int n, const int *idx, const double *src, double *dst);
 
 __global__ void k_residual0(int n, Sell sl, const double *A, const double *x, const double *b,
