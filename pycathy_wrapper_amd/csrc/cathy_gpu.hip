@@ -32,13 +32,12 @@ std::shared_ptr<Flow> lookup(const int64_t *h) {
 
 void set_last_error(const std::string &m) { g_last_error = m; }
 
-// Device staging of the allocation-free EnKF analysis: W (nens x nens FP64)
-// then the members' read and write state pointers, for nens <= kEnkfMax.
+// Device staging of the allocation-free EnKF analysis, for nens <= kEnkfMax: the members'
+// state table and sums, W (nens x nens FP64), the members' state pointers.
 // One array per GPU, held until the process ends; every call on a GPU uses
 // its GPU's copy, so calls that overlap on one GPU race.
-constexpr size_t kScratchW = sizeof(double) * kEnkfMax * kEnkfMax;
-constexpr size_t kScratchTab = sizeof(double *) * kEnkfMax;
-constexpr size_t kScratchBytes = kScratchW + 2 * kScratchTab;
+constexpr size_t kScratchBytes =
+    (sizeof(AdoptDev) + sizeof(double) * (kAdoptSums + kEnkfMax) + sizeof(double *)) * kEnkfMax;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 // Device address of `scratch` on the current GPU, looked up once per GPU
@@ -60,10 +59,6 @@ static unsigned char *scratch_ptr() {
   return g_scratch[dev];
 }
 
-// X_a = X + X' W on the members' PNEW in place (then inflation about the
-// analysis mean), with W and the state pointer tables staged in device
-// memory the caller provides (dw: m*m doubles, dx / dxa: m pointers each);
-// every member then continues from its analysis state.
 using Members = std::array<std::shared_ptr<Flow>, kEnkfMax>;
 
 // The members of an analysis: initialised, distinct, on one mesh and node
@@ -86,25 +81,66 @@ static Members analysis_members(int m, int64_t *handles) {
 // register width of the member loops: the smallest of 8, 16, 32, 64 >= m
 static int member_width(int m) { return m <= 8 ? 8 : m <= 16 ? 16 : m <= 32 ? 32 : 64; }
 
-static void enkf_apply(int m, int64_t *handles, const double *w, double inflation, double *dw,
-                       const double **dx, double **dxa) {
+static std::array<Flow *, kEnkfMax> pointers(const Members &fl, int m) {
+  std::array<Flow *, kEnkfMax> p{};
+  for (int j = 0; j < m; ++j) p[j] = fl[j].get();
+  return p;
+}
+
+// What an analysis stages on the device in one upload: the members' table for
+// adopt_states, their state pointers, and the arrays added by the caller.  Offsets are
+// multiples of 8 bytes; the table's sums lie behind what is uploaded.
+struct Staging {
+  int m;
+  std::vector<unsigned char> h;
+  size_t tab, ptr;
+  Staging(const Members &fl, int m_) : m(m_) {
+    std::vector<AdoptDev> t;
+    std::vector<double *> x;
+    for (int j = 0; j < m; ++j) {
+      t.push_back(fl[j]->adopt_dev());
+      x.push_back(fl[j]->pnew.p);
+    }
+    tab = add(t.data(), t.size());
+    ptr = add(x.data(), x.size());
+  }
+  template <typename T>
+  size_t add(const T *v, size_t cnt) {
+    const size_t off = h.size();
+    h.resize(off + (sizeof(T) * cnt + 7) / 8 * 8);
+    std::memcpy(h.data() + off, v, sizeof(T) * cnt);
+    return off;
+  }
+  size_t bytes() const { return h.size() + sizeof(double) * kAdoptSums * m; }
+  void upload(unsigned char *ws, hipStream_t s) const {
+    CG_HIP(hipMemcpyAsync(ws, h.data(), h.size(), hipMemcpyHostToDevice, s));
+  }
+};
+
+// X_a = X + X' W on the members' PNEW in place (then inflation about the
+// analysis mean), staged in ws of the caller's (null: the leading member's); every
+// member then continues from its analysis state.
+static void enkf_apply(int m, int64_t *handles, const double *w, double inflation, unsigned char *ws) {
   for (int j = 0; j < m * m; ++j) CG_REQUIRE(std::isfinite(w[j]), "non-finite analysis weight");
   Members fl = analysis_members(m, handles);
   Flow *f0 = fl[0].get();
-  std::array<const double *, kEnkfMax> hx;
-  std::array<double *, kEnkfMax> hxa;
-  for (int j = 0; j < m; ++j) {
-    hx[j] = fl[j]->pnew.p;
-    hxa[j] = fl[j]->pnew.p;  // in place: each thread reads its row of every member before writing
-  }
   hipStream_t s = f0->st;
-  CG_HIP(hipMemcpyAsync(dx, hx.data(), sizeof(double *) * m, hipMemcpyHostToDevice, s));
-  CG_HIP(hipMemcpyAsync(dxa, hxa.data(), sizeof(double *) * m, hipMemcpyHostToDevice, s));
-  CG_HIP(hipMemcpyAsync(dw, w, sizeof(double) * m * m, hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(k_enkf_update, dim3(grid_for(f0->n)), dim3(kBlock), 0, s, f0->n, m, dx, dw, inflation, dxa);
+  Staging sg(fl, m);
+  const size_t ow = sg.add(w, (size_t)m * m);
+  if (!ws) ws = f0->analysis_ws(sg.bytes());
+  sg.upload(ws, s);
+  double *const *dx = (double *const *)(ws + sg.ptr);  // in place: each thread reads its row of every member first
+  const double *const *dxr = (const double *const *)dx;
+  const double *dw = (const double *)(ws + ow);
+  const dim3 g((f0->n + 63) / 64), b(64);
+  switch (member_width(m)) {
+    case 8: hipLaunchKernelGGL(k_enkf_update<8>, g, b, 0, s, f0->n, m, dxr, dw, inflation, dx); break;
+    case 16: hipLaunchKernelGGL(k_enkf_update<16>, g, b, 0, s, f0->n, m, dxr, dw, inflation, dx); break;
+    case 32: hipLaunchKernelGGL(k_enkf_update<32>, g, b, 0, s, f0->n, m, dxr, dw, inflation, dx); break;
+    default: hipLaunchKernelGGL(k_enkf_update<64>, g, b, 0, s, f0->n, m, dxr, dw, inflation, dx); break;
+  }
   CG_HIP(hipGetLastError());
-  CG_HIP(hipStreamSynchronize(s));
-  for (int j = 0; j < m; ++j) fl[j]->adopt_state();
+  adopt_states(pointers(fl, m).data(), m, s, (AdoptDev *)(ws + sg.tab), (double *)(ws + sg.h.size()), false);
 }
 
 }  // namespace cg
@@ -291,10 +327,7 @@ int cathy_gpu_enkf_update(const int *nens, int64_t *handles, const double *w, co
     CG_REQUIRE(nens && handles && w && inflation, "null argument");
     const int m = *nens;
     CG_REQUIRE(m >= 2 && m <= kEnkfMax, "ensemble size out of range (2..64)");
-    DBuf<const double *> dx(m);
-    DBuf<double *> dxa(m);
-    DBuf<double> dw((size_t)m * m);
-    enkf_apply(m, handles, w, *inflation, dw.p, dx.p, dxa.p);
+    enkf_apply(m, handles, w, *inflation, nullptr);
     return 0;
   });
 }
@@ -305,11 +338,7 @@ int cathy_gpu_enkf_update_noalloc(const int *nens, int64_t *handles, const doubl
     const int m = *nens;
     CG_REQUIRE(m >= 2 && m <= kEnkfMax,
                "ensemble size out of range (2..64): the allocation-free analysis stages at most 64 members");
-    unsigned char *base = scratch_ptr();
-    double *dw = reinterpret_cast<double *>(base);
-    const double **dx = reinterpret_cast<const double **>(base + kScratchW);
-    double **dxa = reinterpret_cast<double **>(base + kScratchW + kScratchTab);
-    enkf_apply(m, handles, w, *inflation, dw, dx, dxa);
+    enkf_apply(m, handles, w, *inflation, scratch_ptr());
     return 0;
   });
 }
@@ -331,35 +360,29 @@ static void enkf_localized_apply(int m, int64_t *handles, int mo, const double *
   Flow *f0 = fl[0].get();
   const int n = f0->n;
   hipStream_t st = f0->st;
-  std::array<const double *, kEnkfMax> hx;
-  std::array<double *, kEnkfMax> hxa;
-  for (int j = 0; j < m; ++j) hx[j] = hxa[j] = fl[j]->pnew.p;
-  DBuf<const double *> dx(m);
-  DBuf<double *> dxa(m);
-  DBuf<double> ds((size_t)mo * m), dinv((size_t)mo * m), dloc, dnxy, doxy;
-  DBuf<int> dip(n), drz, doz;
-  dx.upload(hx.data(), m, st);
-  dxa.upload(hxa.data(), m, st);
-  ds.upload(s, (size_t)mo * m, st);
-  dinv.upload(invd, (size_t)mo * m, st);
-  dip.upload(f0->iperm.data(), n, st);
+  Staging sg(fl, m);
+  const size_t os = sg.add(s, (size_t)mo * m), od = sg.add(invd, (size_t)mo * m);
+  size_t on = 0, oo = 0;
+  DBuf<double> dloc;
   if (loc) {
     dloc.alloc((size_t)n * mo);
     dloc.upload(loc, (size_t)n * mo, st);
   } else if (row_zone) {
-    drz.alloc(n);
-    doz.alloc(mo);
-    drz.upload(row_zone, n, st);
-    doz.upload(obs_zone, mo, st);
+    on = sg.add(row_zone, n);
+    oo = sg.add(obs_zone, mo);
   } else {
-    dnxy.alloc((size_t)2 * n);
-    doxy.alloc((size_t)2 * mo);
-    dnxy.upload(node_xy, (size_t)2 * n, st);
-    doxy.upload(obs_xy, (size_t)2 * mo, st);
+    on = sg.add(node_xy, (size_t)2 * n);
+    oo = sg.add(obs_xy, (size_t)2 * mo);
   }
-  const LocArgs a{n, m, mo, dx.p, dxa.p, ds.p, dinv.p, dip.p, dloc.p, dnxy.p, doxy.p, drz.p, doz.p,
+  unsigned char *ws = f0->analysis_ws(sg.bytes());
+  sg.upload(ws, st);
+  const bool xy = !loc && !row_zone;
+  const LocArgs a{n, m, mo, (const double *const *)(ws + sg.ptr), (double *const *)(ws + sg.ptr),
+                  (const double *)(ws + os), (const double *)(ws + od), f0->refid.p, dloc.p,
+                  xy ? (const double *)(ws + on) : nullptr, xy ? (const double *)(ws + oo) : nullptr,
+                  row_zone ? (const int *)(ws + on) : nullptr, row_zone ? (const int *)(ws + oo) : nullptr,
                   radius, inflation};
-  const dim3 g(grid_for(n)), b(kBlock);
+  const dim3 g((n + 63) / 64), b(256);  // four lanes a row
   switch (member_width(m)) {
     case 8: hipLaunchKernelGGL(k_enkf_localized<8>, g, b, 0, st, a); break;
     case 16: hipLaunchKernelGGL(k_enkf_localized<16>, g, b, 0, st, a); break;
@@ -367,8 +390,7 @@ static void enkf_localized_apply(int m, int64_t *handles, int mo, const double *
     default: hipLaunchKernelGGL(k_enkf_localized<64>, g, b, 0, st, a); break;
   }
   CG_HIP(hipGetLastError());
-  CG_HIP(hipStreamSynchronize(st));
-  for (int j = 0; j < m; ++j) fl[j]->adopt_state();
+  adopt_states(pointers(fl, m).data(), m, st, (AdoptDev *)(ws + sg.tab), (double *)(ws + sg.h.size()), false);
 }
 }  // namespace cg
 
@@ -443,30 +465,26 @@ int cathy_gpu_pf_resample(const int *nens, int64_t *handles, const int *idx, con
     Flow *f0 = fl[0].get();
     const int n = f0->n;
     hipStream_t st = f0->st;
+    Staging stg(fl, m);
     std::array<const double *, kEnkfMax> hs;
-    std::array<double *, kEnkfMax> hd;
-    for (int j = 0; j < m; ++j) {
-      hs[j] = fl[idx[j]]->pnew.p;
-      hd[j] = fl[j]->pnew.p;
-    }
-    DBuf<const double *> dsrc(m);
-    DBuf<double *> ddst(m);
-    DBuf<int> dip(n);
-    dsrc.upload(hs.data(), m, st);
-    ddst.upload(hd.data(), m, st);
-    dip.upload(f0->iperm.data(), n, st);
+    for (int j = 0; j < m; ++j) hs[j] = fl[idx[j]]->pnew.p;
+    const size_t osrc = stg.add(hs.data(), m);
+    unsigned char *ws = f0->analysis_ws(stg.bytes());
+    stg.upload(ws, st);
+    const double *const *dsrc = (const double *const *)(ws + osrc);
+    double *const *ddst = (double *const *)(ws + stg.ptr);
+    const int *dip = f0->refid.p;
     const dim3 g(grid_for(n)), b(kBlock);
     const double sg = *jitter_std;
     const uint64_t sd = (uint64_t)*seed;
     switch (member_width(m)) {
-      case 8: hipLaunchKernelGGL(k_pf_resample<8>, g, b, 0, st, n, m, dsrc.p, dip.p, sg, sd, ddst.p); break;
-      case 16: hipLaunchKernelGGL(k_pf_resample<16>, g, b, 0, st, n, m, dsrc.p, dip.p, sg, sd, ddst.p); break;
-      case 32: hipLaunchKernelGGL(k_pf_resample<32>, g, b, 0, st, n, m, dsrc.p, dip.p, sg, sd, ddst.p); break;
-      default: hipLaunchKernelGGL(k_pf_resample<64>, g, b, 0, st, n, m, dsrc.p, dip.p, sg, sd, ddst.p); break;
+      case 8: hipLaunchKernelGGL(k_pf_resample<8>, g, b, 0, st, n, m, dsrc, dip, sg, sd, ddst); break;
+      case 16: hipLaunchKernelGGL(k_pf_resample<16>, g, b, 0, st, n, m, dsrc, dip, sg, sd, ddst); break;
+      case 32: hipLaunchKernelGGL(k_pf_resample<32>, g, b, 0, st, n, m, dsrc, dip, sg, sd, ddst); break;
+      default: hipLaunchKernelGGL(k_pf_resample<64>, g, b, 0, st, n, m, dsrc, dip, sg, sd, ddst); break;
     }
     CG_HIP(hipGetLastError());
-    CG_HIP(hipStreamSynchronize(st));
-    for (int j = 0; j < m; ++j) fl[j]->adopt_state();
+    adopt_states(pointers(fl, m).data(), m, st, (AdoptDev *)(ws + stg.tab), (double *)(ws + stg.h.size()), false);
     return 0;
   });
 }

@@ -2252,12 +2252,18 @@ struct Flow {
   // restart from zero, free drainage writes the base rows, the listed
   // fluxes are added
   void neumann_apply(const double *ck) {
-    if (nx_cur > 0)
-      hipLaunchKernelGGL(k_set_rows, dim3(grid_for(nx_cur)), dim3(kBlock), 0, st, nx_cur, neu_rows.p,
-                         (const double *)nullptr, 0.0, qnode.p);
+    neumann_clear(st);
     free_drainage(ck);
+    neumann_add(st);
+  }
+  void neumann_clear(hipStream_t s) {
     if (nx_cur > 0)
-      hipLaunchKernelGGL(k_add_rows, dim3(grid_for(nx_cur)), dim3(kBlock), 0, st, nx_cur, neu_rows.p, neu_vals.p,
+      hipLaunchKernelGGL(k_set_rows, dim3(grid_for(nx_cur)), dim3(kBlock), 0, s, nx_cur, neu_rows.p,
+                         (const double *)nullptr, 0.0, qnode.p);
+  }
+  void neumann_add(hipStream_t s) {
+    if (nx_cur > 0)
+      hipLaunchKernelGGL(k_add_rows, dim3(grid_for(nx_cur)), dim3(kBlock), 0, s, nx_cur, neu_rows.p, neu_vals.p,
                          qnode.p);
   }
   // SHLPIC's PNEW(CONTP) = PRESC (shlpic.f:30-35)
@@ -3081,46 +3087,32 @@ struct Flow {
   // accepted step (PTIMEP = PNEW, Sw and kr at it, the storage baseline
   // of the mass balance reset; the previous-step history of the learned
   // start is dropped).
-  void adopt_state() {
-    CG_REQUIRE(initialised, "flow3d_init not called");
-    CG_HIP(hipMemcpyAsync(ptimep.p, pnew.p, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
-    hipLaunchKernelGGL(k_sw_kr, dim3(grid_for(n)), dim3(kBlock), 0, st, n, pnew.p, soil(), sw.p, ckrw.p);
-    CG_HIP(hipMemcpyAsync(ckrwp.p, ckrw.p, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
-    hipLaunchKernelGGL(k_sw_kr, dim3(grid_for(n)), dim3(kBlock), 0, st, n, ptimep.p, soil(), swtimep.p,
-                       (double *)nullptr);
-    store1 = device_sum_store();
-    store2 = store1;
-    dtprev = 0.0;
-    mbinit_fluxes();
-    CG_HIP(hipStreamSynchronize(st));
-  }
+  void adopt_state();
   // MBINIT (mbinit.f:28-58) at an adopted state: the previous step's
   // boundary fluxes become those a run started from this state begins
   // with -- no Dirichlet fluxes, the atmospheric fluxes ATMOLD at the
   // IFATMP = 0 nodes, and the Neumann fluxes Q (free drainage at the
   // state's kr, then the listed ones).  The cumulative totals go on.
-  void mbinit_fluxes() {
+  // sums: kb_adopt's.
+  void mbinit_fluxes(const double *sums) {
+    store1 = store2 = sums[0];
+    dtprev = 0.0;
     adinp = adoutp = ndinp = ndoutp = 0.0;
-    aninp = anoutp = 0.0;
-    std::vector<double> aold(nnod);
-    std::vector<int> fap(nnod);
-    atmold.download(aold.data(), nnod, st);
-    ifatmp.download(fap.data(), nnod, st);
-    CG_HIP(hipStreamSynchronize(st));
-    for (int s = 0; s < nnod; ++s)
-      if (fap[s] == 0) {
-        if (aold[s] > 0.0) aninp += aold[s]; else anoutp += aold[s];
-      }
-    nninp = nnoutp = 0.0;
-    neumann_apply(ckrw.p);
-    if (prm.free_drainage) {
-      std::vector<double> q(nnod);
-      qbot.download(q.data(), nnod, st);
-      CG_HIP(hipStreamSynchronize(st));
-      for (int s = 0; s < nnod; ++s) { if (q[s] > 0.0) nninp += q[s]; else nnoutp += q[s]; }
-    }
-    nninp += nx_in;
-    nnoutp += nx_out;
+    aninp = sums[1];
+    anoutp = sums[2];
+    nninp = sums[3] + nx_in;
+    nnoutp = sums[4] + nx_out;
+  }
+  AdoptDev adopt_dev() {
+    return AdoptDev{n, nnod, prm.free_drainage ? 1 : 0, soil(), pnew.p, volnod.p, pnodi.p, arenod.p, kznod.p,
+                    atmold.p, bot_row.p, ifatmp.p, ptimep.p, sw.p, ckrw.p, ckrwp.p, swtimep.p, qbot.p, qnode.p, P(0)};
+  }
+  // staging of an analysis led by this member (weights, tables, observations): grows to
+  // the largest asked of it and lives as long as the run
+  DBuf<unsigned char> an_ws;
+  unsigned char *analysis_ws(size_t bytes) {
+    if (an_ws.n < bytes) an_ws.alloc(bytes);
+    return an_ws.p;
   }
 
   void get_state(double *pn, double *swo, double *ck, int *fa) {
@@ -3133,6 +3125,33 @@ struct Flow {
     }
   }
 };
+
+// Members on one mesh continued from their PNEW, all in two launches and one wait on s
+// (the members' own streams are idle); tab and sums: device memory for m entries.
+// up: the table goes there by this call (else the caller has put it there).
+inline void adopt_states(Flow *const *fl, int m, hipStream_t s, AdoptDev *tab, double *sums, bool up) {
+  std::vector<AdoptDev> h;
+  if (up) {
+    for (int j = 0; j < m; ++j) h.push_back(fl[j]->adopt_dev());
+    CG_HIP(hipMemcpyAsync(tab, h.data(), sizeof(AdoptDev) * m, hipMemcpyHostToDevice, s));
+  }
+  // the listed Neumann nodes around the free drainage, as in neumann_apply
+  for (int j = 0; j < m; ++j) fl[j]->neumann_clear(s);
+  hipLaunchKernelGGL(kb_adopt, dim3(fl[0]->red_grid(fl[0]->n), m), dim3(kBlock), 0, s, (const AdoptDev *)tab);
+  for (int j = 0; j < m; ++j) fl[j]->neumann_add(s);
+  hipLaunchKernelGGL(kb_adopt_sums, dim3(kAdoptSums, m), dim3(kBlock), 0, s, (const AdoptDev *)tab, sums);
+  CG_HIP(hipGetLastError());
+  std::array<double, kAdoptSums * kEnkfMax> out;
+  CG_HIP(hipMemcpyAsync(out.data(), sums, sizeof(double) * kAdoptSums * m, hipMemcpyDeviceToHost, s));
+  CG_HIP(hipStreamSynchronize(s));
+  for (int j = 0; j < m; ++j) fl[j]->mbinit_fluxes(&out[(size_t)kAdoptSums * j]);
+}
+inline void Flow::adopt_state() {
+  CG_REQUIRE(initialised, "flow3d_init not called");
+  Flow *self = this;
+  unsigned char *ws = analysis_ws(sizeof(AdoptDev) + sizeof(double) * kAdoptSums);
+  adopt_states(&self, 1, st, (AdoptDev *)ws, (double *)(ws + sizeof(AdoptDev)), true);
+}
 
 // Flow of a handle (cathy_gpu_flow3d_create); throws on an unknown handle.
 std::shared_ptr<Flow> lookup(const int64_t *h);

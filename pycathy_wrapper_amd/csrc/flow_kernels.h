@@ -553,8 +553,23 @@ __global__ void k_bicg_check(int n, int nparts, const double *part_rr, const dou
                              int *done);
 __global__ void k_sw_only(int n, const double *psi, SoilSoA s, double *sw);
 constexpr int kEnkfMax = 64;  // members per analysis launch
+template <int NE>
 __global__ void k_enkf_update(int n, int nens, const double *const *X, const double *W, double alpha,
                               double *const *Xa);
+// One member's state and what a run continued from it starts with (kb_adopt):
+// PTIMEP, Sw and kr at PNEW, the free-drainage fluxes; sums: storage, atmospheric
+// inflow and outflow of the previous step, free-drainage inflow and outflow.
+constexpr int kAdoptSums = 5;
+struct AdoptDev {
+  int n, nnod, drain;
+  SoilSoA soil;
+  const double *pnew, *volnod, *pnodi, *arenod, *kznod, *atmold;
+  const int *bot_row, *ifatmp;
+  double *ptimep, *sw, *ckrw, *ckrwp, *swtimep, *qbot, *qnode;
+  double *part;  // kAdoptSums slots of kMaxRedBlocks
+};
+__global__ void kb_adopt(const AdoptDev *md);
+__global__ void kb_adopt_sums(const AdoptDev *md, double *sums);
 // the localised analysis: states X/Xa (device order, one pointer per
 // member), S and COV^-1 D (m x nens, row-major), device row -> CATHY row,
 // and either the dense localisation (CATHY rows x m) or node / observation

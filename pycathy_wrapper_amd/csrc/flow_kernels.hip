@@ -2198,27 +2198,97 @@ __global__ void k_fill(size_t n, double v, double *__restrict__ dst) {
 //   xa_j = x_j + sum_k (x_k - xbar) W(k, j),
 // then, for inflation alpha != 1 (enkf.py:316-318), xa = mean(xa) +
 // alpha (xa - mean(xa)).  One thread per row; the member values of the
-// row live in registers (N <= kEnkfMax).
-__global__ void k_enkf_update(int n, int nens, const double *const *__restrict__ X, const double *__restrict__ W,
-                              double alpha, double *const *__restrict__ Xa) {
+// row live in registers (NE >= nens, the rest masked).  Bound by the members' rows, in
+// and out, and the latency of few waves: 64 threads a group spread the rows of a small mesh
+// over the CUs.  16 members of
+// 26,896 nodes 52.7 -> 14.0 us (256 threads, the values in scratch memory before).
+template <int NE>
+__global__ __launch_bounds__(64) void k_enkf_update(int n, int nens, const double *const *__restrict__ X,
+                                                    const double *__restrict__ W, double alpha,
+                                                    double *const *__restrict__ Xa) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  double x[kEnkfMax], xa[kEnkfMax];
+  double x[NE], xa[NE];
   double mean = 0.0;
-  for (int k = 0; k < nens; ++k) {
-    x[k] = X[k][i];
-    mean += x[k];
-  }
+#pragma unroll
+  for (int k = 0; k < NE; ++k) x[k] = k < nens ? X[k][i] : 0.0;
+#pragma unroll
+  for (int k = 0; k < NE; ++k) mean += x[k];
   mean /= nens;
   double meana = 0.0;
-  for (int j = 0; j < nens; ++j) {
+#pragma unroll
+  for (int j = 0; j < NE; ++j) {
     double s = x[j];
-    for (int k = 0; k < nens; ++k) s = fma(x[k] - mean, W[(size_t)j * nens + k], s);
+    if (j < nens) {
+      const double *w = W + (size_t)j * nens;
+#pragma unroll
+      for (int k = 0; k < NE; ++k)
+        if (k < nens) s = fma(x[k] - mean, w[k], s);
+    }
     xa[j] = s;
     meana += s;
   }
   meana /= nens;
-  for (int j = 0; j < nens; ++j) Xa[j][i] = alpha == 1.0 ? xa[j] : meana + alpha * (xa[j] - meana);
+#pragma unroll
+  for (int j = 0; j < NE; ++j)
+    if (j < nens) Xa[j][i] = alpha == 1.0 ? xa[j] : meana + alpha * (xa[j] - meana);
+}
+template __global__ void k_enkf_update<8>(int, int, const double *const *, const double *, double, double *const *);
+template __global__ void k_enkf_update<16>(int, int, const double *const *, const double *, double, double *const *);
+template __global__ void k_enkf_update<32>(int, int, const double *const *, const double *, double, double *const *);
+template __global__ void k_enkf_update<64>(int, int, const double *const *, const double *, double, double *const *);
+
+// Members continued from a rewritten PNEW (flow.h adopt_states), blockIdx.y = member:
+// what k_sw_kr, k_store and k_free_drainage compute, in one pass over each state.
+// A bottom node's kr is computed again from its head, so no group waits for another's.
+// Bound by the rows of the members (one read, five written).  16 members of 26,896
+// nodes took nine launches, four waits and 100 us each; now 16.4 us for all.
+__global__ __launch_bounds__(kBlock) void kb_adopt(const AdoptDev *__restrict__ md) {
+  __shared__ double sh[kBlock / 64 + 2];
+  const AdoptDev d = md[blockIdx.y];
+  const int tid = blockIdx.x * blockDim.x + threadIdx.x, nt = gridDim.x * blockDim.x;
+  double sum[kAdoptSums] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  for (int i = tid; i < d.n; i += nt) {
+    const double psi = d.pnew[i];
+    const double se = dev_fvgse(psi, d.soil.psat[i], d.soil.vgn[i], d.soil.vgm[i]);
+    const double sw = d.soil.pnot[i] * se + d.soil.rmcp[i];
+    const double kr = dev_fvgkr(psi, se, d.soil.vgmr[i], d.soil.vgm[i]);
+    d.ptimep[i] = psi;
+    d.sw[i] = sw;
+    d.swtimep[i] = sw;
+    d.ckrw[i] = kr;
+    d.ckrwp[i] = kr;
+    sum[0] += sw * d.volnod[i] * d.pnodi[i];
+  }
+  for (int s = tid; s < d.nnod; s += nt) {
+    if (d.ifatmp[s] == 0) {
+      const double q = d.atmold[s];
+      if (q > 0.0) sum[1] += q; else sum[2] += q;
+    }
+    if (d.drain) {
+      const int r = d.bot_row[s];
+      const double psi = d.pnew[r];
+      const double se = dev_fvgse(psi, d.soil.psat[r], d.soil.vgn[r], d.soil.vgm[r]);
+      const double kr = dev_fvgkr(psi, se, d.soil.vgmr[r], d.soil.vgm[r]);
+      const double q = -1.0 * d.arenod[s] * kr * d.kznod[r];
+      d.qbot[s] = q;
+      d.qnode[r] = q;
+      if (q > 0.0) sum[3] += q; else sum[4] += q;
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < kAdoptSums; ++u) {
+    const double t = block_sum<kBlock>(sum[u], sh);
+    if (threadIdx.x == 0) d.part[(size_t)u * kMaxRedBlocks + blockIdx.x] = t;
+  }
+}
+// one group per member and sum
+__global__ __launch_bounds__(kBlock) void kb_adopt_sums(const AdoptDev *__restrict__ md, double *__restrict__ sums) {
+  __shared__ double sh[kBlock / 64 + 2];
+  const AdoptDev &d = md[blockIdx.y];
+  const int nb = min((d.n + kBlock - 1) / kBlock, kMaxRedBlocks);
+  const double t = reduce_partials<kBlock>(d.part + (size_t)blockIdx.x * kMaxRedBlocks, nb, sh);
+  if (threadIdx.x == 0) sums[blockIdx.y * kAdoptSums + blockIdx.x] = t;
 }
 
 // Gaspari-Cohn weight of distance d for radius L (DA/localisation.py:
@@ -2237,27 +2307,52 @@ __device__ __forceinline__ double gaspari_cohn(double d, double L) {
 // S(j,k) at s[j*nens + k], invD likewise; L(ri,j) from loc[ri*m + j], or
 // 1 where row ri and observation j lie in one zone and 0 elsewhere, or the
 // Gaspari-Cohn weight of the (x, y) distance from node ri to observation
-// j.  Then inflation about the analysis mean.  Member
-// values stay in registers (NE >= nens, the rest masked); every row of
-// every member is read before the thread writes, so the update is in place.
+// j.  Then inflation about the analysis mean.  Every row of every member is read
+// before its threads write, so the update is in place.
+// Four lanes per row, each with a quarter of the members in registers (NE >= nens, the
+// rest zero) and every fourth observation's L, which costs more than the products
+// it weighs (a root and divisions); the dot products are summed over the quad by
+// DPP.  S and invD pass through LDS, kLocLds values each at a time.  Bound by
+// FP64 latency and issue: one thread per row (106 groups on 256 CUs, every L by every
+// thread) took 380 us for 24 members of 26,896 nodes, this 45.6 us.
+__device__ __forceinline__ double quad_xor(double v, bool two) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  return two ? __hiloint2double(__builtin_amdgcn_mov_dpp(hi, 0x4E, 0xF, 0xF, true),
+                                __builtin_amdgcn_mov_dpp(lo, 0x4E, 0xF, 0xF, true))
+             : __hiloint2double(__builtin_amdgcn_mov_dpp(hi, 0xB1, 0xF, 0xF, true),
+                                __builtin_amdgcn_mov_dpp(lo, 0xB1, 0xF, 0xF, true));
+}
+// the quad's sum, the same bits in its four lanes
+__device__ __forceinline__ double quad_sum(double v) {
+  v += quad_xor(v, false);
+  return v + quad_xor(v, true);
+}
+template <int J>
+__device__ __forceinline__ double quad_lane(double v) {
+  return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), J * 0x55, 0xF, 0xF, true),
+                          __builtin_amdgcn_mov_dpp(__double2loint(v), J * 0x55, 0xF, 0xF, true));
+}
+constexpr int kLocLds = 2048;
 template <int NE>
 __global__ __launch_bounds__(256) void k_enkf_localized(LocArgs a) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.n) return;
-  const int nens = a.nens;
+  constexpr int K = NE / 4, J = kLocLds / NE;  // members per lane, observations per LDS fill
+  __shared__ double2 ls[kLocLds / 2], ld[kLocLds / 2];
+  const int q = threadIdx.x & 3, nens = a.nens, k0 = q * K;
+  const int row = blockIdx.x * (blockDim.x / 4) + (threadIdx.x >> 2);
+  const bool on = row < a.n;
+  const int i = on ? row : a.n - 1;
   const int ri = a.iperm[i];
-  double xp[NE], dx[NE];
+  double x[K], xp[K], dx[K];
   double mean = 0.0;
 #pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    xp[k] = k < nens ? a.X[k][i] : 0.0;
-    mean += xp[k];
-  }
-  mean /= nens;
+  for (int u = 0; u < K; ++u) x[u] = k0 + u < nens ? a.X[k0 + u][i] : 0.0;
 #pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    xp[k] = k < nens ? xp[k] - mean : 0.0;
-    dx[k] = 0.0;
+  for (int u = 0; u < K; ++u) mean += x[u];
+  mean = quad_sum(mean) / nens;
+#pragma unroll
+  for (int u = 0; u < K; ++u) {
+    xp[u] = k0 + u < nens ? x[u] - mean : 0.0;
+    dx[u] = 0.0;
   }
   double px = 0.0, py = 0.0;
   const int zi = a.row_zone ? a.row_zone[ri] : 0;
@@ -2266,41 +2361,64 @@ __global__ __launch_bounds__(256) void k_enkf_localized(LocArgs a) {
     py = a.node_xy[2 * (size_t)ri + 1];
   }
   const double nm1 = (double)(nens - 1);
-  bool hit = false;  // zones: an observation in the row's zone
-  for (int j = 0; j < a.m; ++j) {
-    const double *sj = a.s + (size_t)j * nens, *dj = a.invd + (size_t)j * nens;
-    double c = 0.0;
-#pragma unroll
-    for (int k = 0; k < NE; ++k)
-      if (k < nens) c = fma(xp[k], sj[k], c);
-    c = c / nm1;
-    double l;
-    if (a.loc) {
-      l = a.loc[(size_t)ri * a.m + j];
-    } else if (a.row_zone) {
-      const bool in = a.obs_zone[j] == zi;
-      hit = hit || in;
-      l = in ? 1.0 : 0.0;
-    } else {
-      const double ex = a.obs_xy[2 * j] - px, ey = a.obs_xy[2 * j + 1] - py;
-      l = gaspari_cohn(sqrt(ex * ex + ey * ey), a.radius);
+  double hit = 0.0;  // zones: an observation in the row's zone
+  for (int j0 = 0; j0 < a.m; j0 += J) {
+    const int cnt = min(J, a.m - j0);
+    __syncthreads();
+    for (int e = threadIdx.x; e < kLocLds; e += blockDim.x) {
+      const int j = e / NE, k = e % NE;
+      const bool in = j < cnt && k < nens;
+      ((double *)ls)[e] = in ? a.s[(size_t)(j0 + j) * nens + k] : 0.0;
+      ((double *)ld)[e] = in ? a.invd[(size_t)(j0 + j) * nens + k] : 0.0;
     }
-    const double cl = c * l;
+    __syncthreads();
+    for (int j = 0; j < cnt; j += 4) {
+      const int jq = j0 + min(j + q, cnt - 1);
+      double l;
+      if (a.loc) {
+        l = a.loc[(size_t)ri * a.m + jq];
+      } else if (a.row_zone) {
+        l = a.obs_zone[jq] == zi ? 1.0 : 0.0;
+        hit += l;
+      } else {
+        const double ex = a.obs_xy[2 * (size_t)jq] - px, ey = a.obs_xy[2 * (size_t)jq + 1] - py;
+        l = gaspari_cohn(sqrt(ex * ex + ey * ey), a.radius);
+      }
+      l /= nm1;
+      auto one = [&](int jj, double lj) {
+        const double2 *s2 = ls + ((size_t)jj * NE + k0) / 2, *d2 = ld + ((size_t)jj * NE + k0) / 2;
+        double c = 0.0;
 #pragma unroll
-    for (int k = 0; k < NE; ++k)
-      if (k < nens) dx[k] = fma(cl, dj[k], dx[k]);
+        for (int u = 0; u < K / 2; ++u) {
+          const double2 v = s2[u];
+          c = fma(xp[2 * u], v.x, c);
+          c = fma(xp[2 * u + 1], v.y, c);
+        }
+        const double cl = quad_sum(c) * lj;
+#pragma unroll
+        for (int u = 0; u < K / 2; ++u) {
+          const double2 v = d2[u];
+          dx[2 * u] = fma(cl, v.x, dx[2 * u]);
+          dx[2 * u + 1] = fma(cl, v.y, dx[2 * u + 1]);
+        }
+      };
+      one(j, quad_lane<0>(l));
+      if (j + 1 < cnt) one(j + 1, quad_lane<1>(l));
+      if (j + 2 < cnt) one(j + 2, quad_lane<2>(l));
+      if (j + 3 < cnt) one(j + 3, quad_lane<3>(l));
+    }
   }
-  if (a.row_zone && !hit) return;  // a zone with no observation is not analysed
+  if (!on || (a.row_zone && quad_sum(hit) == 0.0)) return;  // a zone with no observation is not analysed
   double meana = 0.0;
 #pragma unroll
-  for (int k = 0; k < NE; ++k) {
-    dx[k] = k < nens ? a.X[k][i] + dx[k] : 0.0;  // x_a
-    meana += dx[k];
+  for (int u = 0; u < K; ++u) {
+    dx[u] = k0 + u < nens ? x[u] + dx[u] : 0.0;  // x_a
+    meana += dx[u];
   }
-  meana /= nens;
+  meana = quad_sum(meana) / nens;
 #pragma unroll
-  for (int k = 0; k < NE; ++k)
-    if (k < nens) a.Xa[k][i] = a.alpha == 1.0 ? dx[k] : meana + a.alpha * (dx[k] - meana);
+  for (int u = 0; u < K; ++u)
+    if (k0 + u < nens) a.Xa[k0 + u][i] = a.alpha == 1.0 ? dx[u] : meana + a.alpha * (dx[u] - meana);
 }
 template __global__ void k_enkf_localized<8>(LocArgs);
 template __global__ void k_enkf_localized<16>(LocArgs);
