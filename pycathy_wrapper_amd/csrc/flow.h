@@ -2353,7 +2353,8 @@ struct Flow {
     R->nptr.upload(ptr, st); R->nlist.upload(list, st);
     for (DBuf<double> *b : {&R->ovflnod, &R->ovflp, &R->pondnod}) b->alloc(nnod);
     R->ovflcel.alloc(ng); R->pondcel.alloc(ng); R->coarse.alloc(ncoarse_);
-    R->state.alloc((size_t)10 * ng); R->sav.alloc((size_t)4 * ng); R->pst.alloc((size_t)4 * ng);
+    R->state.alloc((size_t)10 * ng + (size_t)kRouteWork * link.ncell);
+    R->sav.alloc((size_t)4 * ng); R->pst.alloc((size_t)4 * ng);
     R->cu_ak.alloc(2); R->err.alloc(1);
     CG_HIP(hipStreamSynchronize(st));
     rt = std::move(R);

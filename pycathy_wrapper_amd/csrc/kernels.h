@@ -71,6 +71,13 @@ struct SoilSoA {
   const double *psat, *vgn, *vgm, *vgn1, *vgnr, *vgmr, *vgpsn, *pnot, *rmcp, *snodi, *pnodi;
 };
 
+// Barrier for values in LDS alone: loads and stores of global memory stay under way.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // ------------------------------------------------- block reductions --
 // MI355X dispatches the work-groups of a launch round-robin over its 8
 // XCDs (group g runs on XCD g % 8), each XCD with its own L2.  xcd_group

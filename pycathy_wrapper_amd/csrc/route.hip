@@ -9,11 +9,11 @@
 // QOI_SN order.  The host assigns each cell a level (1 + the deepest level
 // among the cells that feed it) and lists each cell's feeders in QOI_SN
 // order, branch 1 before 2.  One work-group routes one ensemble member:
-// level by level, each thread gathers its cell's inflow from the feeders'
+// level by level, two lanes gather a cell's inflow from the feeders'
 // outflows in that order (the reference's summation order, so the inflow
-// is bitwise the reference's for the same outflows), routes both branches
-// and stores them; a barrier separates the levels.  ALTEZZE follows over
-// every grid cell, with its own cell-type array (the reference's time loop
+// is bitwise the reference's for the same outflows), route a branch each
+// and store it; a barrier separates the levels.  ALTEZZE follows in a launch of its own
+// over every grid cell, with its own cell-type array (the reference's time loop
 // passes CELTYPE, which is zero everywhere, so by default every cell takes
 // the volume balance).  CU_MAX / AK_MAX keep the reference's rule (the last
 // branch in visiting order whose CU is >= the running maximum, starting
@@ -28,6 +28,7 @@
 
 #include "cathy_gpu.h"
 #include "common.h"
+#include "kernels.h"
 #include "route_link.h"
 
 namespace cg {
@@ -39,7 +40,8 @@ enum RouteParam { kW1, kW2, kEpl1, kEpl2, kCk1, kCk2, kEq1, kEq2, kEb1, kEb2, kD
 // DTM grids given to cathy_gpu_route_create, in argument order
 enum DtmGrid { gW1, gW2, gSlope1, gSlope2, gEpl1, gEpl2, gKs1, gKs2, gWs1, gWs2, gB1, gY1, gNrc, kNGrid };
 
-constexpr int kRouteBlock = 512;
+constexpr int kRouteBlock = 512;               // two lanes a cell
+constexpr int kRouteSlots = 7168;                  // outflows held in LDS at a time (56 KB)
 // A cell is fed by at most its 4 cardinal neighbours' W_1 branches and its
 // 4 diagonal neighbours' W_2 branches.
 constexpr int kMaxFeed = 8;
@@ -66,6 +68,11 @@ struct RouteDev {
   const int *key;           // [ncell] 2 * QOI_SN position
   const int *pred;          // [ncell][kMaxFeed] feeders in order: grid index * 2 + branch (0: W_1,
                             // 1: W_2), then -1
+  // A branch's outflow has one reader: it stays in an LDS slot from its level to
+  // the reader's, or, where all slots are taken, in memory alone (-1).
+  const int *slot;          // [ncell][2] of each branch's outflow
+  const int *loc;           // [ncell][kMaxFeed] of each feeder's
+  const int *late;          // [nlev + 1] 1: a cell of the level has a feeder in memory alone
   const double *prm;        // [kNParam][ncell]
   int numres;
   ResDev res;
@@ -95,14 +102,23 @@ McConst mc_const(double local_slope, double ks, double w, double b1, double y1) 
   return c;
 }
 
+// Value of lane J of each pair, in its two lanes.
+template <int J>
+__device__ __forceinline__ int pair_lane(int v) {
+  return __builtin_amdgcn_mov_dpp(v, J ? 0xF5 : 0xA0, 0xF, 0xF, true);
+}
+template <int J>
+__device__ __forceinline__ double pair_lane(double v) {
+  return __hiloint2double(pair_lane<J>(__double2hiint(v)), pair_lane<J>(__double2loint(v)));
+}
+
 // MC (mc.f:8-63): coefficients of one branch and its outflow.
 __device__ __forceinline__ double mc_outflow(double ck0, double eq, double eb, double dh0, double epl,
                                              double deltat, double q_in_kk, double q_in_kkp1, double q_out_kk,
-                                             double q_overland, double &cu, double &ak) {
+                                             double q_overland, double &cu, double &ck) {
   double qc = 1.0 / 3.0 * (q_in_kk + q_in_kkp1 + q_out_kk);
   if (qc <= 1.0e-05) qc = 1.0e-05;
-  const double ck = ck0 * pow(qc, eq);
-  ak = ck / epl;
+  ck = ck0 * pow(qc, eq);
   cu = ck * deltat / epl;
   double dh = pow(qc, eb) / dh0;
   if (dh < (1.0 - cu)) dh = 1.0 - cu;
@@ -189,109 +205,172 @@ __device__ __forceinline__ bool cu_beats(double cu, int key, const CuBest &b) {
   return cu > b.cu || (cu == b.cu && key > b.key);
 }
 
-__global__ __launch_bounds__(kRouteBlock) void k_route(
-    RouteDev d, double deltat, double dx, double dy, const double *__restrict__ sw_all,
-    const double *__restrict__ qin_kk_all, const double *__restrict__ qout_kk1_all,
-    const double *__restrict__ qout_kk2_all, const double *__restrict__ vol_kk_all, double *qin_kkp1_all,
-    double *qout1_all, double *qout2_all, double *__restrict__ vol_kkp1_all, double *__restrict__ h_all,
-    double *__restrict__ cu_ak, const double *__restrict__ hpool_kk_all, double *__restrict__ hpool_kkp1_all,
-    int *__restrict__ err) {
+// What a branch's routing needs of the old levels, in level order ([member][k][branch]; the
+// inflow so far [member][k]): everything that does not depend on the inflow
+// comes out of the serial chain of k_route.  One thread a cell.
+// kRouteWork arrays of ncell doubles: 2 each of q_overland, q_in_kk, q_out_kk, 1 of q_in, 1
+// unused (members start on 16 bytes).
+__global__ __launch_bounds__(256) void k_route_prep(RouteDev d, const double *__restrict__ sw,
+                                                    const double *__restrict__ qin_kk,
+                                                    const double *__restrict__ qout_kk1,
+                                                    const double *__restrict__ qout_kk2,
+                                                    const double *__restrict__ qin, double *__restrict__ pre_all) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x, n = d.ncell;
+  if (k >= n) return;
+  const size_t c = (size_t)blockIdx.y * d.ngrid + d.cell[k];
+  double *pre = pre_all + (size_t)blockIdx.y * kRouteWork * n;
+  const double nrc = d.prm[kNrc * n + k], swc = sw[c] / nrc, qi = qin_kk[c];
+  double2 qov, qik, qok;
+  const double w1 = d.prm[kW1 * n + k], w2 = d.prm[kW2 * n + k];
+  const double cr1 = 1.0 / d.prm[kEpl1 * n + k], cr2 = 1.0 / d.prm[kEpl2 * n + k];
+  qov.x = swc * w1 * cr1;
+  qov.y = swc * w2 * cr2;
+  qik.x = qi * w1 / nrc;
+  qik.y = qi * w2 / nrc;
+  qok.x = qout_kk1[c] / nrc;
+  qok.y = qout_kk2[c] / nrc;
+  ((double2 *)pre)[k] = qov;
+  ((double2 *)pre)[n + k] = qik;
+  ((double2 *)pre)[2 * (size_t)n + k] = qok;
+  pre[6 * (size_t)n + k] = qin[c];
+}
+
+// One routing step of one member by one work-group, level by level.
+//
+// Bound: the levels are a serial chain (413 of 98 cells on average at 201x201), each
+// of them a gather of outflows, two powers and half a dozen divisions one after the
+// other, and a barrier: 2.8 us.  Two lanes take a cell, one a branch; each fetches four of the
+// eight feeders from LDS, where an outflow stays until its reader's level.  All
+// else is loaded two levels ahead, across barriers that wait for LDS alone.  Eight
+// members of 201x201 cells 2470 -> 1150 us (one thread a cell, every load in its level and
+// the depths by the same group before).  Four lanes a cell, one power each: 1240; with
+// feeders beyond eight levels read from memory, which nearly every level has: 1270.
+struct RouteIds {
+  int c, key, slot;
+  int4 src, loc;  // the lane's four feeders
+};
+struct RouteVal {
+  double w, nrc, epl, ck0, eq, eb, dh0, qov, qik, qok, qin;
+};
+template <bool RES>
+__global__ __launch_bounds__(kRouteBlock) void k_route(RouteDev d, double deltat, const double *__restrict__ sw_all,
+                                                       const double *__restrict__ pre_all, double *qin_kkp1_all,
+                                                       double *qout1_all, double *qout2_all,
+                                                       double *__restrict__ cu_ak,
+                                                       const double *__restrict__ hpool_kk_all,
+                                                       double *__restrict__ hpool_kkp1_all, int *__restrict__ err) {
+  __shared__ double held[kRouteSlots];
   const size_t off = (size_t)blockIdx.x * d.ngrid;
-  const double *sw = sw_all + off, *qin_kk = qin_kk_all + off;
-  const double *qout_kk[2] = {qout_kk1_all + off, qout_kk2_all + off};
-  double *qin = qin_kkp1_all + off;
-  double *qout[2] = {qout1_all + off, qout2_all + off};
-  const double *hpool_kk = d.numres ? hpool_kk_all + (size_t)blockIdx.x * d.numres : nullptr;
-  double *hpool = d.numres ? hpool_kkp1_all + (size_t)blockIdx.x * d.numres : nullptr;
+  const int br = threadIdx.x & 1, n = d.ncell;
+  const double *pre = pre_all + (size_t)blockIdx.x * kRouteWork * n;
+  double *qin = qin_kkp1_all + off, *q1 = qout1_all + off, *q2 = qout2_all + off;
+  double *qout = br ? q2 : q1;
+  const double *hpool_kk = RES ? hpool_kk_all + (size_t)blockIdx.x * d.numres : nullptr;
+  double *hpool = RES ? hpool_kkp1_all + (size_t)blockIdx.x * d.numres : nullptr;
   __shared__ int s_err;
   if (threadIdx.x == 0) s_err = 0;
   __syncthreads();
-  CuBest best{0.0, 0.0, -1};
-  int kbeg = d.lev_ptr[0], kend = d.lev_ptr[1];
-  for (int lv = 0; lv < d.nlev; ++lv) {
-    const int knext = lv + 2 <= d.nlev ? d.lev_ptr[lv + 2] : 0;  // consumed after the barrier
-    for (int k = kbeg + (int)threadIdx.x; k < kend; k += blockDim.x) {
-      const int c = d.cell[k];
-      // the feeder slots, then all their outflows, as two batches of loads
-      // (empty slots read entry 0); the sum runs over the feeders in order
-      int src[kMaxFeed];
-#pragma unroll
-      for (int u = 0; u < kMaxFeed; ++u) src[u] = d.pred[(size_t)k * kMaxFeed + u];
-      double vin[kMaxFeed];
-#pragma unroll
-      for (int u = 0; u < kMaxFeed; ++u) {
-        const int sidx = src[u] >= 0 ? src[u] : 0;
-        vin[u] = qout[sidx & 1][sidx >> 1];
-      }
-      double q_in = qin[c];
-#pragma unroll
-      for (int u = 0; u < kMaxFeed; ++u)
-        if (src[u] >= 0) q_in = q_in + vin[u];
-      const double *P = d.prm;
-      const int n = d.ncell;
-      const double nrc = P[kNrc * n + k];
-      const double swc = sw[c] / nrc;
-      const int rflag = d.numres ? d.res.rflag[k] : 0;
-      for (int br = 0; br < 2; ++br) {
-        const double w = P[(kW1 + br) * n + k];
-        if (w == 0) continue;
-        if (rflag & (1 << br)) {  // route.f:101-126: through the reservoir, no NRC scaling of the outflow
-          const int r = d.res.rid[k];
-          double q, h;
-          if (!serbatoio(d.res, r, qin_kk[c] * w / nrc, q_in * w / nrc, hpool_kk[r], deltat, swc, q, h)) {
-            s_err = 1;
-            q = h = 0.0;
-          }
-          if (q < 0.0) q = 0.0;
-          if (rflag & (4 << br)) hpool[r] = h;
-          qout[br][c] = q;
-          continue;
-        }
-        const double epl = P[(kEpl1 + br) * n + k];
-        const double cr = 1.0 / epl;
-        const double q_overland = swc * w * cr;
-        const double qi_kk = qin_kk[c] * w / nrc;
-        const double qo_kk = qout_kk[br][c] / nrc;
-        const double qi_kkp1 = q_in * w / nrc;
-        double cu, ak;
-        double q = mc_outflow(P[(kCk1 + br) * n + k], P[(kEq1 + br) * n + k], P[(kEb1 + br) * n + k],
-                              P[(kDh1 + br) * n + k], epl, deltat, qi_kk, qi_kkp1, qo_kk, q_overland, cu, ak);
-        if (q < 0.0) q = 0.0;
-        qout[br][c] = q * nrc;
-        const int key = d.key[k] + br;
-        if (cu >= 0.0 && cu_beats(cu, key, best)) best = CuBest{cu, ak, key};
-      }
-      qin[c] = q_in;
+  CuBest best{0.0, 0.0, -1};  // ak: CK / EPL of the best branch
+  const int step = (int)blockDim.x >> 1, mine = (int)threadIdx.x >> 1;
+  const double *P = d.prm;
+  auto flow = [&](int src) { return ((src & 1) ? q2 : q1)[src >> 1]; };
+  auto ids = [&](int k, int end) {
+    RouteIds I{0, 0, -1, make_int4(-1, -1, -1, -1), make_int4(0, 0, 0, 0)};
+    if (k < end) {
+      I.c = d.cell[k];
+      I.key = d.key[k];
+      I.slot = d.slot[2 * (size_t)k + br];
+      I.src = ((const int4 *)d.pred)[(size_t)k * 2 + br];
+      I.loc = ((const int4 *)d.loc)[(size_t)k * 2 + br];
     }
-    __syncthreads();
-    kbeg = kend;
-    kend = knext;
+    return I;
+  };
+  auto vals = [&](int k, int end) {
+    RouteVal V{};
+    if (k < end) {
+      V.w = P[(kW1 + br) * n + k];
+      V.nrc = P[kNrc * n + k];
+      V.epl = P[(kEpl1 + br) * n + k];
+      V.ck0 = P[(kCk1 + br) * n + k];
+      V.eq = P[(kEq1 + br) * n + k];
+      V.eb = P[(kEb1 + br) * n + k];
+      V.dh0 = P[(kDh1 + br) * n + k];
+      V.qov = pre[2 * (size_t)k + br];
+      V.qik = pre[2 * ((size_t)n + k) + br];
+      V.qok = pre[2 * (2 * (size_t)n + k) + br];
+      V.qin = pre[6 * (size_t)n + k];
+    }
+    return V;
+  };
+  // the cell of the quad: its inflow, and the lane's branch
+  auto route = [&](int k, const RouteIds &I, const RouteVal &V) {
+    auto feed = [&](int src, int loc) {
+      if (src < 0) return 0.0;
+      return loc >= 0 ? held[loc] : flow(src);
+    };
+    const int4 e = I.src;
+    const double v0 = feed(e.x, I.loc.x), v1 = feed(e.y, I.loc.y), v2 = feed(e.z, I.loc.z), v3 = feed(e.w, I.loc.w);
+    double q_in = V.qin;  // the feeders in order
+    auto add = [&](int src, double v) { q_in = src >= 0 ? q_in + v : q_in; };
+    add(pair_lane<0>(e.x), pair_lane<0>(v0));
+    add(pair_lane<0>(e.y), pair_lane<0>(v1));
+    add(pair_lane<0>(e.z), pair_lane<0>(v2));
+    add(pair_lane<0>(e.w), pair_lane<0>(v3));
+    add(pair_lane<1>(e.x), pair_lane<1>(v0));
+    add(pair_lane<1>(e.y), pair_lane<1>(v1));
+    add(pair_lane<1>(e.z), pair_lane<1>(v2));
+    add(pair_lane<1>(e.w), pair_lane<1>(v3));
+    if (br == 0) qin[I.c] = q_in;
+    if (V.w == 0) return;
+    const double qi_kkp1 = q_in * V.w / V.nrc;
+    const int rflag = RES ? d.res.rflag[k] : 0;
+    double out;
+    if (RES && (rflag & (1 << br))) {  // route.f:101-126: through the reservoir, no NRC scaling of the outflow
+      const int r = d.res.rid[k];
+      double h;
+      if (!serbatoio(d.res, r, V.qik, qi_kkp1, hpool_kk[r], deltat, sw_all[off + I.c] / V.nrc, out, h)) {
+        s_err = 1;
+        out = h = 0.0;
+      }
+      if (out < 0.0) out = 0.0;
+      if (rflag & (4 << br)) hpool[r] = h;
+    } else {
+      double cu, ck;
+      double q = mc_outflow(V.ck0, V.eq, V.eb, V.dh0, V.epl, deltat, V.qik, qi_kkp1, V.qok, V.qov, cu, ck);
+      if (q < 0.0) q = 0.0;
+      out = q * V.nrc;
+      const int key = I.key + br;
+      if (cu >= 0.0 && cu_beats(cu, key, best)) best = CuBest{cu, ck / V.epl, key};
+    }
+    qout[I.c] = out;
+    if (I.slot >= 0) held[I.slot] = out;
+  };
+  auto lev = [&](int l) { return d.lev_ptr[min(l, d.nlev)]; };
+  int l0 = lev(0), l1 = lev(1), l2 = lev(2), l3 = lev(3);
+  RouteIds I0 = ids(l0 + mine, l1), I1 = ids(l1 + mine, l2);
+  RouteVal V0 = vals(l0 + mine, l1), V1 = vals(l1 + mine, l2);
+  int late = d.late[min(1, d.nlev)];
+  for (int lv = 0; lv < d.nlev; ++lv) {
+    const int l4 = lev(lv + 4), late2 = d.late[min(lv + 2, d.nlev)];
+    const RouteIds I2 = ids(l2 + mine, l3);
+    const RouteVal V2 = vals(l2 + mine, l3);
+    if (l0 + mine < l1) route(l0 + mine, I0, V0);
+    for (int k = l0 + mine + step; k < l1; k += step) route(k, ids(k, l1), vals(k, l1));
+    if (late) __syncthreads();  // the next level reads outflows from memory
+    else lds_barrier();
+    late = late2;
+    I0 = I1; V0 = V1;
+    I1 = I2; V1 = V2;
+    l0 = l1; l1 = l2; l2 = l3; l3 = l4;
   }
+  __syncthreads();
   // route.f:133-137, 244-246: the outflows into unrouted cells, in the
   // order the reference adds them
-  if (d.nsink) {
-    if (threadIdx.x == 0)
-      for (int u = 0; u < d.nsink; ++u) {
-        const int src = d.sink[2 * u], tgt = d.sink[2 * u + 1];
-        qin[tgt] = qin[tgt] + qout[src & 1][src >> 1];
-      }
-    __syncthreads();
-  }
-  // ALTEZZE (altezze.f:33-105) over every grid cell; reservoir and lake
-  // depths only where the caller's type array asks for them
-  for (int c = threadIdx.x; c < d.ngrid; c += blockDim.x) {
-    const int alt = d.res.alt ? d.res.alt[c] : -1;
-    if (alt >= 0) {  // reservoir outlet (depth clamped below at 0) or lake cell (positive depths only)
-      const double hw = hpool[alt >> 1] - d.res.elevation[c];
-      h_all[off + c] = (alt & 1) ? (hw > 0.0 ? hw : 0.0) : (hw < 0 ? 0.0 : hw);
-      continue;
+  if (threadIdx.x == 0)
+    for (int u = 0; u < d.nsink; ++u) {
+      const int src = d.sink[2 * u], tgt = d.sink[2 * u + 1];
+      qin[tgt] = qin[tgt] + flow(src);
     }
-    const double dv = (qin_kk[c] + qin[c]) / 2 * deltat + sw[c] * deltat -
-                      (qout_kk[0][c] + qout_kk[1][c]) / 2 * deltat - (qout[0][c] + qout[1][c]) / 2 * deltat;
-    const double v = vol_kk_all[off + c] + dv;
-    vol_kkp1_all[off + c] = v >= 0.0 ? v : 0.0;
-    h_all[off + c] = v >= 0.0 ? v / (dx * dy) : 0.0;
-  }
   // (CU, key) maximum over the work-group
   __shared__ double s_cu[kRouteBlock / 64], s_ak[kRouteBlock / 64];
   __shared__ int s_key[kRouteBlock / 64];
@@ -317,11 +396,49 @@ __global__ __launch_bounds__(kRouteBlock) void k_route(
   }
 }
 
+// ALTEZZE (altezze.f:33-105) over every grid cell; reservoir and lake depths
+// only where the caller's type array asks for them.  Its own launch (blockIdx.y =
+// member): bound by the arrays' bandwidth, which the routing's one group cannot reach.
+__global__ __launch_bounds__(256) void k_route_depth(
+    RouteDev d, double deltat, double dx, double dy, const double *__restrict__ sw, const double *__restrict__ qin_kk,
+    const double *__restrict__ qout_kk1, const double *__restrict__ qout_kk2, const double *__restrict__ vol_kk,
+    const double *__restrict__ qin, const double *__restrict__ qout1, const double *__restrict__ qout2,
+    double *__restrict__ vol_kkp1, double *__restrict__ h, const double *__restrict__ hpool_all) {
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= d.ngrid) return;
+  const size_t c = (size_t)blockIdx.y * d.ngrid + g;
+  const int alt = d.res.alt ? d.res.alt[g] : -1;
+  if (alt >= 0) {  // reservoir outlet (depth clamped below at 0) or lake cell (positive depths only)
+    const double hw = hpool_all[(size_t)blockIdx.y * d.numres + (alt >> 1)] - d.res.elevation[g];
+    h[c] = (alt & 1) ? (hw > 0.0 ? hw : 0.0) : (hw < 0 ? 0.0 : hw);
+    return;
+  }
+  const double dv = (qin_kk[c] + qin[c]) / 2 * deltat + sw[c] * deltat -
+                    (qout_kk1[c] + qout_kk2[c]) / 2 * deltat - (qout1[c] + qout2[c]) / 2 * deltat;
+  const double v = vol_kk[c] + dv;
+  vol_kkp1[c] = v >= 0.0 ? v : 0.0;
+  h[c] = v >= 0.0 ? v / (dx * dy) : 0.0;
+}
+
+// One step of m members on st; S: ten arrays of m x ngrid (the step's arguments in
+// order), pre: kRouteWork arrays of m x ncell, both of the caller.
+static void launch_step(const RouteDev &d, hipStream_t st, int m, double deltat, double dx, double dy, double *S,
+                        double *pre, double *cu_ak, const double *hpool_kk, double *hpool, int *err) {
+  const size_t g = (size_t)m * d.ngrid;
+  hipLaunchKernelGGL(k_route_prep, dim3((d.ncell + 255) / 256, m), dim3(256), 0, st, d, S, S + g, S + 2 * g,
+                     S + 3 * g, S + 5 * g, pre);
+  hipLaunchKernelGGL(d.numres ? k_route<true> : k_route<false>, dim3(m), dim3(kRouteBlock), 0, st, d, deltat, S,
+                     (const double *)pre, S + 5 * g, S + 6 * g, S + 7 * g, cu_ak, hpool_kk, hpool, err);
+  hipLaunchKernelGGL(k_route_depth, dim3((d.ngrid + 255) / 256, m), dim3(256), 0, st, d, deltat, dx, dy, S, S + g,
+                     S + 2 * g, S + 3 * g, S + 4 * g, S + 5 * g, S + 6 * g, S + 7 * g, S + 8 * g, S + 9 * g, hpool);
+  CG_HIP(hipGetLastError());
+}
+
 struct Route {
   int nrow = 0, ncol = 0, ncell = 0, ngrid = 0, nlev = 0, maxpred = 0;
   std::mutex mu;  // steps and reservoir set-up on one handle share its device buffers
   hipStream_t st = nullptr;
-  DBuf<int> lev_ptr, cell, key, pred, sink;
+  DBuf<int> lev_ptr, cell, key, pred, slot, loc, late, sink;
   int nsink = 0;
   DBuf<double> prm;
   // per-step state [member][ngrid]: 5 inputs, 4 in/out (volume_kkp1 keeps
@@ -343,7 +460,7 @@ struct Route {
   }
 
   RouteDev dev() const {
-    return RouteDev{ncell, ngrid, nlev, lev_ptr.p, cell.p, key.p, pred.p, prm.p, numres,
+    return RouteDev{ncell, ngrid, nlev, lev_ptr.p, cell.p, key.p, pred.p, slot.p, loc.p, late.p, prm.p, numres,
                     ResDev{maxres, r_nha.p, r_hres.p, r_ares.p, r_soglia.p, r_fondo.p, r_rid.p, r_rflag.p,
                            typed ? r_alt.p : nullptr, r_elev.p},
                     nsink, sink.p};
@@ -392,12 +509,7 @@ void route_substep(const RouteLink &l, hipStream_t st, double deltat, double dx,
   Route *r = static_cast<Route *>(l.route);
   CG_REQUIRE(r->numres == 0, "the coupled step routes networks without reservoirs");
   std::lock_guard<std::mutex> lk(r->mu);
-  const size_t g = r->ngrid;
-  double *S = state;
-  hipLaunchKernelGGL(k_route, dim3(1), dim3(kRouteBlock), 0, st, r->dev(), deltat, dx, dy, S, S + g, S + 2 * g,
-                     S + 3 * g, S + 4 * g, S + 5 * g, S + 6 * g, S + 7 * g, S + 8 * g, S + 9 * g, cu_ak,
-                     (const double *)nullptr, (double *)nullptr, err);
-  CG_HIP(hipGetLastError());
+  launch_step(r->dev(), st, 1, deltat, dx, dy, state, state + 10 * (size_t)r->ngrid, cu_ak, nullptr, nullptr, err);
 }
 }  // namespace cg
 
@@ -468,7 +580,7 @@ int cathy_gpu_route_create(int64_t *handle, const int *nrow, const int *ncol, co
     for (int l = 0; l < nlev; ++l) lev_ptr[l + 1] += lev_ptr[l];
     std::vector<int> slot(lev_ptr.begin(), lev_ptr.end() - 1), of(n);
     for (int p = 0; p < n; ++p) of[p] = slot[level[p]]++;
-    std::vector<int> cell(n), key(n), pred((size_t)n * kMaxFeed, -1);
+    std::vector<int> cell(n), key(n), pred((size_t)n * kMaxFeed, -1), loc((size_t)n * kMaxFeed, -1), late(nlev + 1, 0);
     std::vector<double> prm((size_t)kNParam * n);
     int maxpred = 0;
     std::vector<int> by_k(n);
@@ -499,6 +611,25 @@ int cathy_gpu_route_create(int64_t *handle, const int *nrow, const int *ncol, co
       for (size_t u = 0; u < feeders[p].size() && u < (size_t)kMaxFeed; ++u) pred[(size_t)k * kMaxFeed + u] = feeders[p][u];
     }
     CG_REQUIRE(maxpred <= kMaxFeed, "a cell has more than 8 feeders");
+    // LDS slots of the outflows: taken in their level, free again after their reader's
+    std::vector<int> slots((size_t)2 * n, -1), free_slots(kRouteSlots);
+    for (int u = 0; u < kRouteSlots; ++u) free_slots[u] = kRouteSlots - 1 - u;
+    std::vector<uint8_t> read((size_t)2 * n, 0);
+    for (int f : pred)
+      if (f >= 0) read[2 * (size_t)of[pos[f >> 1]] + (f & 1)] = 1;
+    for (int l = 0; l < nlev; ++l) {
+      for (int q = 2 * lev_ptr[l]; q < 2 * lev_ptr[l + 1]; ++q)
+        if (read[q] && !free_slots.empty()) {
+          slots[q] = free_slots.back();
+          free_slots.pop_back();
+        }
+      for (size_t u = (size_t)lev_ptr[l] * kMaxFeed; u < (size_t)lev_ptr[l + 1] * kMaxFeed; ++u)
+        if (pred[u] >= 0) {
+          loc[u] = slots[2 * (size_t)of[pos[pred[u] >> 1]] + (pred[u] & 1)];
+          if (loc[u] >= 0) free_slots.push_back(loc[u]);
+          else late[l] = 1;
+        }
+    }
     auto r = std::make_unique<Route>();
     r->nrow = nr;
     r->ncol = nc;
@@ -520,6 +651,9 @@ int cathy_gpu_route_create(int64_t *handle, const int *nrow, const int *ncol, co
     r->cell.upload(cell, r->st);
     r->key.upload(key, r->st);
     r->pred.upload(pred, r->st);
+    r->slot.upload(slots, r->st);
+    r->loc.upload(loc, r->st);
+    r->late.upload(late, r->st);
     r->prm.upload(prm, r->st);
     r->nsink = (int)sinks.size() / 2;
     if (r->nsink) r->sink.upload(sinks, r->st);
@@ -665,7 +799,7 @@ int cathy_gpu_route_step(int64_t *handle, const int *nmember, const double *delt
     const size_t len = (size_t)m * r->ngrid;
     const size_t lres = (size_t)m * r->numres;
     if (m > r->cap_members) {
-      r->state.alloc(10 * (size_t)m * r->ngrid);
+      r->state.alloc((10 * (size_t)r->ngrid + kRouteWork * (size_t)r->ncell) * m);
       r->cu_ak.alloc(2 * (size_t)m);
       r->err.alloc(m);
       r->hpool.alloc(2 * std::max<size_t>(lres, 1));
@@ -682,10 +816,8 @@ int cathy_gpu_route_step(int64_t *handle, const int *nmember, const double *delt
       CG_HIP(hipMemcpyAsync(r->hpool.p + lres, h_pool_kkp1_vec, lres * sizeof(double), hipMemcpyHostToDevice,
                             r->st));
     }
-    hipLaunchKernelGGL(k_route, dim3(m), dim3(kRouteBlock), 0, r->st, r->dev(), *deltat, *delta_x, *delta_y,
-                       S, S + len, S + 2 * len, S + 3 * len, S + 4 * len, S + 5 * len, S + 6 * len, S + 7 * len,
-                       S + 8 * len, S + 9 * len, r->cu_ak.p, r->hpool.p, r->hpool.p + lres, r->err.p);
-    CG_HIP(hipGetLastError());
+    launch_step(r->dev(), r->st, m, *deltat, *delta_x, *delta_y, S, S + 10 * len, r->cu_ak.p, r->hpool.p, r->hpool.p + lres,
+                r->err.p);
     double *out[5] = {q_in_kkp1_sn, q_out_kkp1_sn_1, q_out_kkp1_sn_2, volume_kkp1_sn, h_water_kkp1_sn};
     for (int a = 0; a < 5; ++a)
       CG_HIP(hipMemcpyAsync(out[a], S + (5 + a) * len, len * sizeof(double), hipMemcpyDeviceToHost, r->st));

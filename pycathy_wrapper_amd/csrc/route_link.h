@@ -10,6 +10,8 @@
 
 namespace cg {
 
+constexpr int kRouteWork = 8;  // doubles a substep needs per routed cell
+
 struct RouteLink {
   std::shared_ptr<void> keep;  // holds the routing handle while linked
   void *route = nullptr;
@@ -24,7 +26,7 @@ RouteLink route_link(const int64_t *handle);
 // st.  state: SURFACE_WATER_SN, Q_IN_KK_SN, Q_OUT_KK_SN_1, Q_OUT_KK_SN_2,
 // VOLUME_KK_SN, Q_IN_KKP1_SN, Q_OUT_KKP1_SN_1, Q_OUT_KKP1_SN_2,
 // VOLUME_KKP1_SN, H_WATER_KKP1_SN, each ngrid doubles by I_BASIN - 1, in
-// that order, contiguous.  cu_ak[2]: CU_MAX (out), AK_MAX (in, replaced
+// that order, contiguous, then room for kRouteWork * ncell doubles.  cu_ak[2]: CU_MAX (out), AK_MAX (in, replaced
 // where a branch sets it).  err[1]: 0.
 void route_substep(const RouteLink &l, hipStream_t st, double deltat, double dx, double dy, double *state,
                    double *cu_ak, int *err);

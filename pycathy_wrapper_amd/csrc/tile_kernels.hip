@@ -286,13 +286,6 @@ __device__ __forceinline__ void tile_chain(double *v, int nloc, const double *a,
   }
 }
 
-// Barrier for values in LDS alone: loads and stores of global memory stay under way.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // RPT: rows of a phase per thread (the host checks that every phase fits).
 template <typename FT, int MODE, int RPT>
 __device__ __forceinline__ void tile_body(Blk bk, double *smem, const TileSet &T, const TileCols &C,
