@@ -3073,14 +3073,14 @@ struct Flow {
     }
     hipLaunchKernelGGL(k_vel3d, dim3(grid_for(nt)), dim3(kBlock), 0, st, nt, enode.p, pnew.p, ckrw.p, vtab.p,
                        e_uu.p, e_vv.p, e_ww.p);
-    hipLaunchKernelGGL(k_vnod3d, dim3(grid_for(n)), dim3(kBlock), 0, st, n, inc_ptr.p, inc.p, e_uu.p, e_vv.p,
+    hipLaunchKernelGGL(k_vnod3d, dim3(grid_for(n)), dim3(kBlock), 0, st, n, inc_ptr.p, inc.p, refid.p, e_uu.p, e_vv.p,
                        e_ww.p, n_u.p, n_v.p, n_w.p);
     if (uu) e_uu.download(uu, nt, st);
     if (vv) e_vv.download(vv, nt, st);
     if (ww) e_ww.download(ww, nt, st);
-    CG_HIP(hipStreamSynchronize(st));
     for (auto pr : {std::make_pair(&n_u, unod), std::make_pair(&n_v, vnod), std::make_pair(&n_w, wnod)})
-      if (pr.second) get_nodes(pr.first->p, pr.second);
+      if (pr.second) pr.first->download(pr.second, n, st);
+    CG_HIP(hipStreamSynchronize(st));
   }
   int nzone_ = 0, maxstr_ = 0;
 

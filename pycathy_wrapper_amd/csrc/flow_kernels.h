@@ -596,7 +596,7 @@ __global__ void k_pf_resample(int n, int nens, const double *const *src, const i
                               uint64_t seed, double *const *dst);
 __global__ void k_vel3d(int nt, const int4 *enode, const double *pnew, const double *ckrw, const double *vt,
                         double *uu, double *vv, double *ww);
-__global__ void k_vnod3d(int n, const int *inc_ptr, const int *inc, const double *uu, const double *vv,
+__global__ void k_vnod3d(int n, const int *inc_ptr, const int *inc, const int *refid, const double *uu, const double *vv,
                          const double *ww, double *unod, double *vnod, double *wnod);
 
 }  // namespace cg
