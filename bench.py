@@ -290,8 +290,11 @@ def reference_baseline(args, members: int, max_steps: int, seconds: float) -> di
         for p in procs:
             p.stdout.readline()
         for p in procs:
-            p.stdin.write("go\n")
-            p.stdin.flush()
+            try:
+                p.stdin.write("go\n")
+                p.stdin.flush()
+            except BrokenPipeError:  # ended already (no reference build here): reported below
+                pass
         out = []
         for p in procs:
             o, _ = p.communicate(timeout=900)
