@@ -240,10 +240,10 @@ struct Flow {
   DBuf<double> part;  // partial sums, kSlots slots of kMaxRedBlocks
   DBuf<int> ipart;
   DBuf<PcgScal> scal;
-  DBuf<int> flags;  // [0] PCG done, [1] IC(0) breakdown count
+  DBuf<int> flags;  // [0] solver done, [1] IC(0) breakdown count
   DBuf<double> res;
   std::vector<double> h_res;
-  // what the host polls, in pinned memory: the solver's done flag and
+  // what the host polls, in pinned memory: BiCGSTAB's done flag, the solvers'
   // scalars, MASBAL's reduced values, single sums
   struct HostBox {
     int done;
@@ -1646,7 +1646,7 @@ struct Flow {
     DBuf<double> fa(fw), fb(fw);
     CG_HIP(hipMemsetAsync(fa.p, 0, fw * sizeof(double), st));
     int *done = flags.p;
-    CG_HIP(hipMemsetAsync(done, 0, sizeof(int), st));
+    CG_HIP(hipMemsetAsync(&scal.p->stop, 0, sizeof(int), st));
     const int Gs = grid_for(n, kBlock);
     const FacTab fts{(spmv_transposed && ftab_ok && sell().coded && maxrow <= kUnroll) ? ftab.p : nullptr, ftab_nch};
     std::vector<hipEvent_t> ev(4 * (size_t)nrep);
@@ -1655,7 +1655,7 @@ struct Flow {
       hipLaunchKernelGGL(k_copy, dim3((unsigned)((fw + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, fw, fa.p, fb.p);
       for (int h = 0; h < 2; ++h)
         hipExtLaunchKernelGGL(k_spmv_dot2, dim3(Gs), dim3(kBlock), 0, st, ev[4 * i + 2 * h], ev[4 * i + 2 * h + 1], 0,
-                              n, sell(), fts, A.p, p.p, r.p, Bv.p, P(1), P(2), done);
+                              n, sell(), fts, A.p, p.p, r.p, Bv.p, P(1), P(2), scal.p, done);
     }
     CG_HIP(hipStreamSynchronize(st));
     double cold = 0.0, warm = 0.0;
@@ -1699,17 +1699,17 @@ struct Flow {
           } else {
             hipLaunchKernelGGL(k_spmv_beta, dim3(Gs), dim3(kBlock), 0, st, sell(), fts, tile_pcg(), ntile);
           }
-          tile_apply<kTilePcg>(nullptr, z.p, done);
+          tile_apply<kTilePcg>(nullptr, z.p, nullptr);
           continue;
         }
         if (prof) {
           // the dispatch packet's own start/end timestamps (kernel time only)
           hipEvent_t e0 = next_event(), e1 = next_event();
           hipExtLaunchKernelGGL(k_spmv_dot2, dim3(Gs), dim3(kBlock), 0, st, e0, e1, 0, n, sell(), fts, A.p, p.p,
-                                r.p, Bv.p, P(1), P(2), done);
+                                r.p, Bv.p, P(1), P(2), scal.p, done);
         } else {
           hipLaunchKernelGGL(k_spmv_dot2, dim3(Gs), dim3(kBlock), 0, st, n, sell(), fts, A.p, p.p, r.p, Bv.p,
-                             P(1), P(2), done);
+                             P(1), P(2), scal.p, done);
         }
         hipLaunchKernelGGL(k_pcg_alpha, dim3(Gr), dim3(kBlock), 0, st, n, Gs, P(1), P(2), Bv.p, p.p, isdir.p,
                            r.p, pdiff.p, P(3), scal.p, done);
@@ -1719,11 +1719,10 @@ struct Flow {
       }
       launched += batch;
       if (tiles()) hipLaunchKernelGGL(k_pcg_check, dim3(1), dim3(256), 0, st, tile_pcg(), ntile);
-      CG_HIP(hipMemcpyAsync(&hbox.p->done, done, sizeof(int), hipMemcpyDeviceToHost, st));
       CG_HIP(hipMemcpyAsync(&hbox.p->pcg, scal.p, sizeof(PcgScal), hipMemcpyDeviceToHost, st));
       CG_HIP(hipStreamSynchronize(st));
-      h_done = hbox.p->done;
       hs = hbox.p->pcg;
+      h_done = hs.stop;
       if (prof) {
         // launches after convergence exit at once; count only the live ones
         const int executed = h_done ? hs.niter : hs.niter - 1;  // bodies run so far

@@ -197,10 +197,16 @@ struct ListLevel {
   int off, cnt;
 };
 
+// Scalars of a PCG solve.  How it ends: the launch that takes the stopping test
+// (k_pcg_beta, k_spmv_beta, k_pcg_check) stores `stop`.  The launch after it
+// (k_spmv_dot2, k_tile) returns on `stop` and copies it to the done flag, on which
+// all others return.  So no launch of several work-groups stores the flag that its own groups
+// return on, and all waves of a group pass its barriers or none does.  The host polls `stop`.
 struct PcgScal {
   double xlung, pb, alpha, err, tol;
   int niter, imax;
-  int it;  // iterations finished (tile path only)
+  int it;    // iterations finished (tile path only)
+  int stop;  // the stopping test has been met
 };
 
 struct NormPart {
@@ -359,13 +365,13 @@ __global__ void k_residual0(int n, Sell sl, const double *A, const double *x, co
 // upper slot (the assembled matrix is bitwise symmetric), so HBM serves
 // about one triangle and the last-level cache the other.
 __global__ void k_spmv_dot2(int n, Sell sl, FacTab ft, const double *A, const double *p, const double *r,
-                            double *B, double *part_pr, double *part_pb, const int *done);
+                            double *B, double *part_pr, double *part_pb, const PcgScal *sc, int *done);
 __global__ void k_pcg_alpha(int n, int nparts, const double *part_pr, const double *part_pb, const double *B,
                             const double *p, const uint8_t *isdir, double *r, double *x, double *part_rr,
                             PcgScal *sc, const int *done);
 __global__ void k_dot(int n, const double *u, const double *v, double *part, const int *done);
 __global__ void k_pcg_beta(int n, int nparts, const double *part_bz, const double *part_rr, const double *z,
-                           double *p, PcgScal *sc, int *done);
+                           double *p, PcgScal *sc, const int *done);
 __global__ void k_pcg_init(int nparts, const double *part, PcgScal *sc, int *done, double tol, int imax);
 __global__ void k_update_pnew(int n, const double *pdiff, const int *row_surf, const int *ifatm,
                               const double *pold, double *pnew);

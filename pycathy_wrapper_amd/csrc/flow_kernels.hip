@@ -1305,8 +1305,11 @@ __global__ void k_residual0(int n, Sell sl, const double *__restrict__ A, const 
 __device__ __forceinline__ void spmv_dot2_body(Blk bk, int n, Sell sl, FacTab ft, const double *__restrict__ A, const double *__restrict__ p,
                             const double *__restrict__ r, double *__restrict__ B,
                             double *__restrict__ part_pr, double *__restrict__ part_pb,
-                            const int *__restrict__ done) {
-  if (*done) return;
+                            const PcgScal *__restrict__ sc, int *__restrict__ done) {
+  if (sc->stop) {  // see PcgScal
+    if (bk.b == 0 && threadIdx.x == 0) *done = 1;
+    return;
+  }
   __shared__ double sh[2 * (kBlock / 64)];
   double apr = 0.0, apb = 0.0;
   const int i = bk.b * blockDim.x + threadIdx.x;
@@ -1326,8 +1329,8 @@ __device__ __forceinline__ void spmv_dot2_body(Blk bk, int n, Sell sl, FacTab ft
 __global__ void k_spmv_dot2(int n, Sell sl, FacTab ft, const double *__restrict__ A, const double *__restrict__ p,
                             const double *__restrict__ r, double *__restrict__ B,
                             double *__restrict__ part_pr, double *__restrict__ part_pb,
-                            const int *__restrict__ done) {
-  spmv_dot2_body(self_xcd_blk(), n, sl, ft, A, p, r, B, part_pr, part_pb, done);
+                            const PcgScal *__restrict__ sc, int *__restrict__ done) {
+  spmv_dot2_body(self_xcd_blk(), n, sl, ft, A, p, r, B, part_pr, part_pb, sc, done);
 }
 
 // alpha from the SpMV partials (every group sums them in the same fixed
@@ -1400,7 +1403,7 @@ __global__ void k_dot(int n, const double *__restrict__ u, const double *__restr
 // beta, p = z + beta p, err and the stopping test (graddp.f:1348-1377).
 __device__ __forceinline__ void pcg_beta_body(Blk bk, int n, int nparts, const double *__restrict__ part_bz,
                            const double *__restrict__ part_rr, const double *__restrict__ z,
-                           double *__restrict__ p, PcgScal *sc, int *done) {
+                           double *__restrict__ p, PcgScal *sc, const int *__restrict__ done) {
   if (*done) return;
   __shared__ double sh[2 * (kBlock / 64)];
   const double2 crr = reduce_partials2<kBlock>(part_bz, part_rr, nparts, sh);
@@ -1420,13 +1423,13 @@ __device__ __forceinline__ void pcg_beta_body(Blk bk, int n, int nparts, const d
     if (err > sc->tol && sc->niter < sc->imax) {
       sc->niter += 1;
     } else {
-      *done = 1;
+      sc->stop = 1;
     }
   }
 }
 __global__ void k_pcg_beta(int n, int nparts, const double *__restrict__ part_bz,
                            const double *__restrict__ part_rr, const double *__restrict__ z,
-                           double *__restrict__ p, PcgScal *sc, int *done) {
+                           double *__restrict__ p, PcgScal *sc, const int *__restrict__ done) {
   pcg_beta_body(self_blk(), n, nparts, part_bz, part_rr, z, p, sc, done);
 }
 
@@ -1441,6 +1444,7 @@ __device__ __forceinline__ void pcg_init_body(Blk bk, int nparts, const double *
     sc->imax = imax;
     sc->niter = 1;
     sc->it = 0;
+    sc->stop = 0;
     sc->err = 0.0;
     *done = 0;
   }
@@ -2696,7 +2700,8 @@ __global__ void kb_pcg_init(const int *start, int nmem, const MemberDev *md) {
 }
 __global__ void kb_spmv_dot2(const int *start, int nmem, const MemberDev *md) {
   CG_BATCH_HEAD
-  spmv_dot2_body(bk, d.n, d.sl, d.fts, d.A, d.p, d.r, d.Bv, slot_part(d, 1), slot_part(d, 2), d.flags);
+  spmv_dot2_body(bk, d.n, d.sl, d.fts, d.A, d.p, d.r, d.Bv, slot_part(d, 1), slot_part(d, 2), d.scal,
+                 d.flags);
 }
 __global__ void kb_pcg_alpha(const int *start, int nmem, const MemberDev *md) {
   CG_BATCH_HEAD
@@ -2711,12 +2716,12 @@ __global__ void kb_pcg_beta(const int *start, int nmem, const MemberDev *md) {
   CG_BATCH_HEAD
   pcg_beta_body(bk, d.n, d.g_vec, slot_part(d, 4), slot_part(d, 3), d.z, d.p, d.scal, d.flags);
 }
-// out[3m..3m+2] = done flag, iterations, last relative residual of member m
+// out[3m..3m+2] = stop flag, iterations, last relative residual of member m
 __global__ void kb_poll(const int *start, int nmem, const MemberDev *md, double *out) {
   CG_BATCH_HEAD
   (void)bk;
   if (threadIdx.x == 0) {
-    out[3 * m_] = (double)d.flags[0];
+    out[3 * m_] = (double)d.scal->stop;
     out[3 * m_ + 1] = (double)d.scal->niter;
     out[3 * m_ + 2] = d.scal->err;
   }

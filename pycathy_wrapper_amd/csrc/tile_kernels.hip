@@ -102,7 +102,7 @@ __device__ __forceinline__ PcgTest pcg_test(const TilePcg &P, const Partials<1> 
 // formed for the row and for each neighbour it gathers (the same fma
 // everywhere), B = A p and partial (p, r), (p, B).  Joins k_pcg_beta to k_spmv_dot2
 // for one more gather per entry.  The scalars a launch reads (it) are written by the
-// other launch of the iteration, those it writes (niter, err, done) it does
+// other launch of the iteration, those it writes (niter, err, stop) it does
 // not read.  Bound: the dependent loads (slice offset, column code, neighbour)
 // on small meshes, in flight together with the partials; the gathers on large ones.
 // 7.9 us at 4,851 nodes, 16.9 at 214,221, 12.9 at 8 x 26,896 (k_spmv_dot2 and
@@ -163,7 +163,7 @@ __device__ __forceinline__ void spmv_beta_body(Blk bk, const Sell &sl, const Fac
     const PcgTest t = pcg_test(P, q, it, sh);
     if (bk.b == 0 && threadIdx.x == 0) {
       P.sc->err = t.err;
-      if (t.stop) *P.done = 1;
+      if (t.stop) P.sc->stop = 1;
     }
     if (t.stop) return;
     beta = t.beta;
@@ -198,12 +198,12 @@ __global__ __launch_bounds__(kBlock) void k_spmv_beta(Sell sl, FacTab ft, TilePc
 // The stopping test of the last iteration of a launch batch, before the host reads
 // the flag (the next batch's first launch would take it again, alike).
 __device__ __forceinline__ void pcg_check_body(const TilePcg &P, int ntile) {
-  if (*P.done) return;
+  if (P.sc->stop) return;
   __shared__ double sh[16];
   const PcgTest t = pcg_test(P, partials_load<1>(P.part_bz, P.part_rr, ntile), P.sc->it, sh);
   if (threadIdx.x == 0) {
     P.sc->err = t.err;
-    if (t.stop) *P.done = 1;
+    if (t.stop) P.sc->stop = 1;
     else P.sc->niter = P.sc->it + 1;
   }
 }
@@ -286,16 +286,20 @@ __device__ __forceinline__ void tile_chain(double *v, int nloc, const double *a,
   }
 }
 
-// RPT: rows of a phase per thread (the host checks that every phase fits).
+// RPT: rows of a phase per thread (the host checks that every phase fits).  flag: the
+// launch returns where it is set (null: never).
 template <typename FT, int MODE, int RPT>
 __device__ __forceinline__ void tile_body(Blk bk, double *smem, const TileSet &T, const TileCols &C,
                                           const FT *__restrict__ F, const TilePcg &P, const double *__restrict__ in,
-                                          double *out, const int *done) {
+                                          double *out, const int *flag) {
   __shared__ double sh[2 * kTileThreads / 64];
-  const int stopped = done ? *done : 0;
+  const int stopped = flag ? *flag : 0;
   const TileDesc d = T.desc[bk.b];
   const int body = MODE == kTilePcg ? P.sc->niter : 0;  // written by this iteration's first launch
-  if (stopped) return;
+  if (stopped) {
+    if (MODE == kTilePcg && bk.b == 0 && threadIdx.x == 0) *P.done = 1;  // the flag read is sc->stop (see PcgScal)
+    return;
+  }
   const int len = C.c[0].len, kl = len - 1, tid = threadIdx.x, nt = T.threads;
   const int off1 = d.n[0], off2 = d.n[0] + d.n[1], nloc = off2 + d.n[2];
   double *V = smem, *W = smem + nloc * len;  // y / x by [plane][column]; coefficients of a phase
@@ -513,7 +517,7 @@ template <typename FT, int MODE, int RPT>
 __global__ __launch_bounds__(kTileThreads) void k_tile(TileSet T, TileCols C, const FT *F, TilePcg P,
                                                        const double *in, double *out, const int *done) {
   extern __shared__ double smem[];
-  tile_body<FT, MODE, RPT>(self_xcd_blk(), smem, T, C, F, P, in, out, done);
+  tile_body<FT, MODE, RPT>(self_xcd_blk(), smem, T, C, F, P, in, out, MODE == kTilePcg ? &P.sc->stop : done);
 }
 #define CG_INST_TILE(FT, MODE)                                                                                       \
   template __global__ void k_tile<FT, MODE, 1>(TileSet, TileCols, const FT *, TilePcg, const double *, double *, const int *); \
@@ -541,7 +545,7 @@ __global__ __launch_bounds__(kTileThreads) void kb_tile(const int *start, int nm
   CG_TILE_HEAD
   const FT *F = sizeof(FT) == 4 ? (const FT *)d.F32 : (const FT *)d.F64;
   const TileCols C{{d.col[0], d.col[1], d.col[2]}};
-  if (MODE == kTilePcg) tile_body<FT, MODE, RPT>(bk, smem, d.tiles, C, F, d.tpcg, nullptr, d.z, d.flags);
+  if (MODE == kTilePcg) tile_body<FT, MODE, RPT>(bk, smem, d.tiles, C, F, d.tpcg, nullptr, d.z, &d.tpcg.sc->stop);
   else tile_body<FT, MODE, RPT>(bk, smem, d.tiles, C, F, d.tpcg, member_vec(d, vin), member_vec(d, vout), nullptr);
 }
 #define CG_INST_BTILE(FT, MODE)                                                          \
