@@ -78,7 +78,6 @@ struct DBuf {
   ~DBuf() { release(); }
   void alloc(size_t count) {
     release();
-    n = count;
     if (count) {
       hipError_t e = hipMalloc(&p, count * sizeof(T));
       if (e != hipSuccess) {
@@ -86,6 +85,7 @@ struct DBuf {
         throw Error(-3, "hipMalloc of " + std::to_string(count * sizeof(T)) + " bytes failed");
       }
     }
+    n = count;  // after a failure 0: callers grow a buffer by comparing with it
   }
   void release() {
     if (p) (void)hipFree(p);

@@ -3066,9 +3066,9 @@ struct Flow {
         t[15] = permy[ix];
         t[16] = permz[ix];
       }
-      vtab.upload(h, st);
       for (DBuf<double> *b : {&e_uu, &e_vv, &e_ww}) b->alloc(nt);
       for (DBuf<double> *b : {&n_u, &n_v, &n_w}) b->alloc(n);
+      vtab.upload(h, st);  // last: its presence stands for all of them
     }
     hipLaunchKernelGGL(k_vel3d, dim3(grid_for(nt)), dim3(kBlock), 0, st, nt, enode.p, pnew.p, ckrw.p, vtab.p,
                        e_uu.p, e_vv.p, e_ww.p);

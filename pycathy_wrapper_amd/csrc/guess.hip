@@ -770,6 +770,7 @@ void GuessNet::ensure(int ncol) {
   CG_REQUIRE(ncol > 0, "guess net: no columns");
   if (ncol <= cap) return;
   const size_t pos = (size_t)ncol * Lp;
+  cap = 0;  // should an allocation fail
   xs.alloc(pos * kGuessIn);
   y32.alloc(pos);
   ts.alloc(pos);
@@ -841,10 +842,8 @@ void GuessNet::gradient(const unsigned short *x, const int *idx, const float *t,
   int nloss;
   if (fused()) {
     const int G = std::min(tiles(ncol), kTrainGroups);
-    if (part.n < (size_t)G * kPartSize) {
-      part.alloc((size_t)G * kPartSize);
-      lossp.alloc(G);
-    }
+    if (part.n < (size_t)G * kPartSize) part.alloc((size_t)G * kPartSize);
+    if (lossp.n < (size_t)G) lossp.alloc(G);
     hipLaunchKernelGGL(k_gfused<true>, dim3(G), dim3(512), 0, st, fused_net(*this), ncol, Lp, L, idx, x, t, inv,
                        (float *)nullptr, lossp.p, part.p);
     nloss = gp.nsplit = G;
@@ -1038,6 +1037,7 @@ int cathy_gpu_guess_load(int64_t *net, const int64_t *nsamp, const uint16_t *x, 
     auto g = guess_lookup(*net);
     std::lock_guard<std::mutex> lk(g->mu);
     const size_t pos = (size_t)*nsamp * g->Lp;
+    g->nsamp = 0;  // no training set should an allocation fail
     g->X.alloc(pos * kGuessIn);
     g->T.alloc(pos);
     g->X.upload(x, pos * kGuessIn, g->st);

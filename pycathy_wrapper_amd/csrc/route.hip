@@ -799,6 +799,7 @@ int cathy_gpu_route_step(int64_t *handle, const int *nmember, const double *delt
     const size_t len = (size_t)m * r->ngrid;
     const size_t lres = (size_t)m * r->numres;
     if (m > r->cap_members) {
+      r->cap_members = 0;  // should an allocation fail
       r->state.alloc((10 * (size_t)r->ngrid + kRouteWork * (size_t)r->ncell) * m);
       r->cu_ak.alloc(2 * (size_t)m);
       r->err.alloc(m);
