@@ -2577,7 +2577,7 @@ __global__ void k_vel3d(int nt, const int4 *__restrict__ enode, const double *__
 // vnod3d.f:17-32: nodal means over the incident elements, summed in element order.
 // Bound by the latency of the element lists and of the values behind them: eight
 // elements' loads go out together.  214,221 nodes 303 us one element at a time, 114 us now.
-// The means go to CATHY's node order (refid).
+// The means go to CATHY's node order (refid) or stay in row order (null).
 __global__ void k_vnod3d(int n, const int *__restrict__ inc_ptr, const int *__restrict__ inc,
                          const int *__restrict__ refid, const double *__restrict__ uu,
                          const double *__restrict__ vv, const double *__restrict__ ww, double *__restrict__ unod,
@@ -2586,7 +2586,7 @@ __global__ void k_vnod3d(int n, const int *__restrict__ inc_ptr, const int *__re
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= n) return;
   double su = 0.0, sv = 0.0, sw = 0.0;
-  const int i0 = inc_ptr[r], i1 = inc_ptr[r + 1], o = refid[r];
+  const int i0 = inc_ptr[r], i1 = inc_ptr[r + 1], o = refid ? refid[r] : r;
   for (int i = i0; i < i1; i += U) {
     int e[U];
     double a[U], b[U], c[U];

@@ -1,13 +1,22 @@
 /* The HIP calls of libcathy_gpu.so on host memory, for tests without a GPU
  * (LD_PRELOAD): allocations and copies work, launches do nothing.
  * hip_stub_fail(k) lets the k-th allocation from now fail (0: the next);
- * hip_stub_live() counts the device allocations held. */
+ * hip_stub_live() counts the device allocations held, hip_stub_copies(p) the
+ * copies made to p. */
 #include <stdlib.h>
 #include <string.h>
 
 static int fail_at = -1, live = 0;
 void hip_stub_fail(int k) { fail_at = k; }
 int hip_stub_live(void) { return live; }
+
+static void *copied[4096];
+static int ncopied = 0;
+int hip_stub_copies(void *p) {
+  int c = 0;
+  for (int i = 0; i < ncopied && i < 4096; ++i) c += copied[i] == p;
+  return c;
+}
 
 int hipMalloc(void **p, size_t n) {
   if (fail_at >= 0 && fail_at-- == 0) { *p = 0; return 2; /* hipErrorOutOfMemory */ }
@@ -21,6 +30,7 @@ int hipHostFree(void *p) { free(p); return 0; }
 int hipMemcpyAsync(void *d, const void *s, size_t n, int k, void *st) {
   (void)k; (void)st;
   if (n && (!d || !s)) return 1; /* hipErrorInvalidValue */
+  copied[ncopied++ % 4096] = d;
   memcpy(d, s, n);
   return 0;
 }

@@ -84,3 +84,27 @@ def test_velocity_linear_head_on_device():
     assert np.allclose(vel["uu"], -kr * kx * a, rtol=1e-7, atol=0)
     assert np.allclose(vel["vv"], -kr * ky * b, rtol=1e-7, atol=0)
     assert np.allclose(vel["ww"], kr * kz * g, rtol=1e-7, atol=0)
+
+
+@pytest.mark.parametrize("rows,cols,layers,order", [
+    (1, 1, 1, 1), (9, 8, 5, 0), (49, 49, 19, 1), (49, 50, 20, 1), (49, 50, 20, 0), (60, 50, 20, 3)])
+def test_nodal_means_in_the_callers_order(rows, cols, layers, order):
+    """Meshes on either side of the 50,000 nodes up to which the host puts the
+    nodal means in CATHY's order: the mean of the device's own element values
+    in element order, bit for bit."""
+    from pycathy_wrapper_amd import gpu as G
+    from test_gpu_tiles import _problem
+    pr = _problem(rows, cols, layers, 1)
+    m = pr.mesh
+    f = G.FlowGPU(pr, order)
+    try:
+        f.set_pnew(pr.psi0 + 0.2 * np.random.default_rng(rows).standard_normal(m.n))
+        vel = f.velocity()
+    finally:
+        f.close()
+    t = np.asarray(m.tetra)[:, :4].ravel()
+    cnt = np.bincount(t, minlength=m.n)
+    for e, nod in (("uu", "unod"), ("vv", "vnod"), ("ww", "wnod")):
+        s = np.zeros(m.n)
+        np.add.at(s, t, np.repeat(vel[e], 4))
+        assert np.any(s != 0.0) and np.array_equal(vel[nod], s / cnt), nod
