@@ -587,6 +587,16 @@ int cathy_gpu_flow3d_spmv_bytes(int64_t *handle, double *bytes);
  * per-chain codes of the extruded mesh (else read per slot), and the
  * number of slots whose code failed the set-up check (0). */
 int cathy_gpu_flow3d_layout(int64_t *handle, int64_t *out6);
+/* How the preconditioner runs: out3 = surface tiles the solver uses (0:
+ * launches per colour or level), rows of a tile's phase per thread, threads
+ * of a tile. */
+int cathy_gpu_flow3d_tiles(int64_t *handle, int *out3);
+/* The preconditioner of the last linear solve on a vector, z = M^-1 t (N
+ * values each, CATHY order): (L L^T)^-1 in Picard runs, U^-1 L^-1 in Newton
+ * runs.  *launches: 0 as the solver runs it, 1 by the launches per colour or
+ * level.  A diagnostic; no state of the run changes. */
+int cathy_gpu_flow3d_precond(int64_t *handle, const int *launches,
+                             const double *t, double *z);
 /* Copy kernel over NBYTES (read NBYTES, write NBYTES), REPS launches;
  * average ms per launch.  Calibrates HBM counters. */
 int cathy_gpu_calib_copy(const int64_t *nbytes, const int *reps,

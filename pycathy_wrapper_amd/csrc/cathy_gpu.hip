@@ -544,6 +544,26 @@ int cathy_gpu_flow3d_layout(int64_t *handle, int64_t *out6) {
   });
 }
 
+int cathy_gpu_flow3d_tiles(int64_t *handle, int *out3) {
+  return guarded([&] {
+    const std::shared_ptr<Flow> f = lookup(handle);
+    CG_REQUIRE(out3, "null argument");
+    out3[0] = f->tiles() ? f->ntile : 0;
+    out3[1] = f->tiles() ? f->tile_rpt : 0;
+    out3[2] = f->tiles() ? f->tile_threads : 0;
+    return 0;
+  });
+}
+
+int cathy_gpu_flow3d_precond(int64_t *handle, const int *launches, const double *t, double *z) {
+  return guarded([&] {
+    const std::shared_ptr<Flow> f = lookup(handle);
+    CG_REQUIRE(launches && t && z, "null argument");
+    f->precond_nodes(*launches != 0, t, z);
+    return 0;
+  });
+}
+
 int cathy_gpu_calib_copy(const int64_t *nbytes, const int *reps, double *ms_per_launch) {
   return guarded([&] {
     CG_REQUIRE(nbytes && reps && ms_per_launch && *nbytes >= 8 && *reps >= 1, "bad argument");

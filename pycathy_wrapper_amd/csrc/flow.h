@@ -1863,6 +1863,37 @@ struct Flow {
     return hs.niter;
   }
 
+  // z = M^-1 t of the last solve on nodal values in CATHY's order, as the solver runs
+  // it or by the colour or level launches.  Uses vectors that every solve writes first.
+  void precond_nodes(bool launches, const double *t, double *zout) {
+    const bool newton = prm.iopt == 2;
+    CG_REQUIRE(initialised && c_pcg > 0 && (!newton || newton_ready),
+               "the preconditioner belongs to a solve: none has run");
+    put_nodes(t, Bv.p);
+    if (!launches && newton) {
+      ilu_fwd(Bv.p, b_z1.p, nullptr);
+      ilu_bwd(b_z1.p, z.p, nullptr);
+    } else if (!launches) {
+      precond_apply(Bv.p, z.p, nullptr);
+    } else if (f32) {
+      precond_launches<float>(newton, F32.p);
+    } else {
+      precond_launches<double>(newton, F64.p);
+    }
+    CG_HIP(hipGetLastError());
+    get_nodes(z.p, zout);
+  }
+
+  template <typename FT>
+  void precond_launches(bool newton, const FT *F) {
+    if (newton) {
+      ilu_fwd_t<FT>(F, Bv.p, b_z1.p, nullptr);
+      ilu_bwd_t<FT>(F, b_z1.p, z.p, nullptr);
+    } else {
+      precond_apply_t<FT>(F, Bv.p, z.p, nullptr);
+    }
+  }
+
   // One Newton iteration (newton.f).
   void newton_iteration(double &err) {
     alloc_newton();

@@ -382,6 +382,23 @@ class FlowGPU:
         return dict(n=int(out[0]), nnz=int(out[1]), nnz_sell=int(out[2]), maxrow=int(out[3]),
                     coded=int(out[4]), code_mismatch=int(out[5]))
 
+    def tiles(self) -> dict:
+        """Surface tiles the solver runs over (0: launches per colour or
+        level), rows of a phase per thread and threads of a tile."""
+        out = np.zeros(3, dtype=np.int32)
+        _check(lib().cathy_gpu_flow3d_tiles(C.byref(self.h), _p(out)), "tiles")
+        return dict(tiles=int(out[0]), rows_per_thread=int(out[1]), threads=int(out[2]))
+
+    def precond(self, t, launches: bool = False) -> np.ndarray:
+        """The last solve's preconditioner on a vector (N, CATHY order), as the
+        solver runs it or by the launches per colour or level."""
+        t = np.ascontiguousarray(t, dtype=np.float64)
+        if t.shape != (self.n,):
+            raise ValueError("one value per node")
+        z = np.zeros(self.n)
+        _check(lib().cathy_gpu_flow3d_precond(C.byref(self.h), _i(1 if launches else 0), _p(t), _p(z)), "precond")
+        return z
+
     def close(self):
         if getattr(self, "h", None) is not None and self.h.value:
             lib().cathy_gpu_flow3d_destroy(C.byref(self.h))

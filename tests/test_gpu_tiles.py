@@ -12,6 +12,11 @@ tolerance's other side.  psi's bound is that of test_gpu_parity.  (Newton on
 90x90x22 is no test of this: its first BiCGSTAB solve is marginal, 1,132
 iterations with chain-major rows where the oracle, the natural and both other column
 orderings step back.)
+
+Each case asserts that it runs on tiles, with the rows per thread it is there for,
+and that chain-major rows do not.  The preconditioner itself is compared on one
+flow: z of the tiles against z of the colour launches with the same factor.
+Lockstep members on tiles equal their solo runs bit for bit, in both precisions.
 """
 from __future__ import annotations
 
@@ -47,6 +52,15 @@ def _problem(rows, cols, layers, iopt):
                       CF.hillslope_small_params(iopt=iopt), 0)
 
 
+TWO_ROWS = {(12, 12, 28), (12, 12, 40), (9, 9, 63), (90, 90, 22)}   # meshes whose phases take two rows per thread
+
+
+def _on_tiles(f, rows, cols, layers):
+    """The flow runs on tiles, as many rows per thread as the mesh is a test of."""
+    t = f.tiles()
+    return t["tiles"] >= 1 and t["rows_per_thread"] == (2 if (rows, cols, layers) in TWO_ROWS else 1)
+
+
 @pytest.mark.parametrize("rows,cols,layers,iopt,fp64", [
     (1, 1, 1, 1, False), (1, 30, 2, 1, False), (4, 4, 3, 1, False), (1, 12, 5, 1, True), (5, 4, 3, 2, False),
     (3, 40, 1, 2, False), (9, 31, 5, 1, True), (24, 25, 15, 1, False), (12, 12, 40, 1, False), (12, 12, 40, 2, True),
@@ -62,6 +76,7 @@ def test_tiles_match_oracle_and_colour_launches(gpu, oracle, rows, cols, layers,
     try:
         for f in flows:
             f.factor_fp64(fp64)
+        assert _on_tiles(flows[0], rows, cols, layers) and flows[1].tiles()["tiles"] == 0
         for _ in range(2 if m.n < 50000 else 1):
             _, so = run.step()
             st = [f.advance()[1] for f in flows]
@@ -73,4 +88,64 @@ def test_tiles_match_oracle_and_colour_launches(gpu, oracle, rows, cols, layers,
     finally:
         run.close()
         for f in flows:
+            f.close()
+
+
+# z of the tiles and z of the colour launches differ by the rounding of FP64 sums alone:
+# five phases of at most 14 products and a recurrence down a column of 64 levels at
+# 2^-53 each, 5 * 80 * 1.1e-16 (measured: 2e-16).  A wrong halo value shows at the size
+# of z's entries.
+Z_TOL = 5e-14
+
+
+@pytest.mark.parametrize("rows,cols,layers,iopt,fp64", [
+    (1, 1, 1, 1, False), (1, 30, 2, 1, False), (5, 4, 3, 2, False), (24, 25, 15, 1, False), (24, 25, 15, 2, False),
+    (12, 12, 40, 1, False), (12, 12, 40, 2, False), (9, 9, 63, 1, False), (90, 90, 22, 1, False)])
+def test_the_tiles_precondition_as_the_colour_launches(gpu, rows, cols, layers, iopt, fp64):
+    pr = _problem(rows, cols, layers, iopt)
+    f = gpu.FlowGPU(pr, gpu.ORDER_COLUMN3)
+    try:
+        f.factor_fp64(fp64)
+        assert _on_tiles(f, rows, cols, layers)
+        with pytest.raises(gpu.CathyGpuError, match="none has run"):
+            f.precond(np.zeros(pr.mesh.n))
+        f.advance()
+        rng = np.random.default_rng(rows)
+        for t in (rng.standard_normal(pr.mesh.n), np.eye(1, pr.mesh.n, pr.mesh.n // 2)[0]):
+            z, zl = f.precond(t), f.precond(t, launches=True)
+            assert np.any(z != 0.0) and np.all(np.isfinite(z))
+            assert np.max(np.abs(z - zl)) <= Z_TOL * np.max(np.abs(zl))
+    finally:
+        f.close()
+
+
+@pytest.mark.parametrize("fp64", [False, True])
+@pytest.mark.parametrize("sizes", [((12, 12, 28), (12, 12, 28)), ((24, 25, 15), (9, 31, 5)),
+                                   ((12, 12, 28), (4, 4, 3), (24, 25, 15))])
+def test_lockstep_on_tiles_matches_solo_runs(gpu, sizes, fp64):
+    """Members with one and two rows per thread in one launch, each its solo run's bits."""
+    probs = [_problem(*sz, 1) for sz in sizes]
+    for k, pr in enumerate(probs):
+        pr.psi0 = pr.psi0 - 0.01 * k
+    flows = [gpu.FlowGPU(pr, gpu.ORDER_COLUMN3) for pr in probs]
+    for f, sz in zip(flows, sizes):
+        f.factor_fp64(fp64)
+        assert _on_tiles(f, *sz)
+    ens = gpu.EnsembleGPU(flows)
+    try:
+        rc, taken, stats = ens.advance(2)
+        assert np.all(rc == 0) and np.all(taken == 2)
+        psi = [f.psi() for f in flows]
+    finally:
+        ens.close()
+        for f in flows:
+            f.close()
+    for pr, st, ps in zip(probs, stats, psi):
+        f = gpu.FlowGPU(pr, gpu.ORDER_COLUMN3)
+        try:
+            f.factor_fp64(fp64)
+            for s in st:
+                assert f.advance()[1] == s
+            assert np.array_equal(f.psi(), ps)
+        finally:
             f.close()
