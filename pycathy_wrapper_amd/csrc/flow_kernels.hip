@@ -711,12 +711,12 @@ __device__ __forceinline__ void fwd_col3_body(Blk bk, double *smem, ColDesc C, S
       // slot max(jp - 1, 0) and are masked (see sell_row_dot)
       const int jl = max(jp - 1, 0);
       int c[NW > 0 ? NW : 1];
-      float f[NW > 0 ? NW : 1];
+      FT f[NW > 0 ? NW : 1];
       double yv[NW > 0 ? NW : 1];
       // slots past the window read index 0 (a broadcast where the whole
       // wave is past it) and are masked
 #pragma unroll
-      for (int j = 0; j < NW; ++j) f[j] = (float)F[j < jp ? base + 64 * j : 0];
+      for (int j = 0; j < NW; ++j) f[j] = F[j < jp ? base + 64 * j : 0];
       sell_cols_window(sl, rp, base, 0, jl, c);
 #pragma unroll
       for (int j = 0; j < NW; ++j) yv[j] = y[j < jp ? c[j] : 0];
@@ -814,12 +814,12 @@ __device__ __forceinline__ void bwd_col3_body(Blk bk, double *smem, ColDesc C, S
       // entry j is slot min(js + 1 + j, len - 1), masked past len
       const int jl = len - 1;
       int c[NW > 0 ? NW : 1];
-      float f[NW > 0 ? NW : 1];
+      FT f[NW > 0 ? NW : 1];
       double xv[NW > 0 ? NW : 1];
       // slots past the row read index 0 (a broadcast where the whole wave
       // is past it) and are masked
 #pragma unroll
-      for (int j = 0; j < NW; ++j) f[j] = (float)F[j0 + j < len ? base + 64 * (j0 + j) : 0];
+      for (int j = 0; j < NW; ++j) f[j] = F[j0 + j < len ? base + 64 * (j0 + j) : 0];
       sell_cols_window(sl, rp, base, j0, jl, c);
 #pragma unroll
       for (int j = 0; j < NW; ++j) xv[j] = x[j0 + j < len ? c[j] : 0];

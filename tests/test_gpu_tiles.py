@@ -99,8 +99,8 @@ Z_TOL = 5e-14
 
 
 @pytest.mark.parametrize("rows,cols,layers,iopt,fp64", [
-    (1, 1, 1, 1, False), (1, 30, 2, 1, False), (5, 4, 3, 2, False), (24, 25, 15, 1, False), (24, 25, 15, 2, False),
-    (12, 12, 40, 1, False), (12, 12, 40, 2, False), (9, 9, 63, 1, False), (90, 90, 22, 1, False)])
+    (1, 1, 1, 1, False), (1, 30, 2, 1, True), (5, 4, 3, 2, False), (24, 25, 15, 1, False), (24, 25, 15, 2, True),
+    (12, 12, 40, 1, True), (12, 12, 40, 2, False), (9, 9, 63, 1, False), (90, 90, 22, 1, False)])
 def test_the_tiles_precondition_as_the_colour_launches(gpu, rows, cols, layers, iopt, fp64):
     pr = _problem(rows, cols, layers, iopt)
     f = gpu.FlowGPU(pr, gpu.ORDER_COLUMN3)
