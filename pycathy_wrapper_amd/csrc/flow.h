@@ -722,13 +722,21 @@ struct Flow {
   DBuf<uint32_t> t_tab;
   DBuf<double> p2, r2;
   // Meshes the tiles serve: columns plane by plane in three colours, and either a
-  // tile per CU at most or few nodes; beyond, five launches stream the factor
-  // faster than the tiles, which read it two to three times.  A pass of one time step,
-  // five launches / tiles: 214,221 nodes 8.90 / 7.35 ms, 120x120 cells of 18 layers
-  // (one tile per CU) 4.65 / 3.97, of 24 layers 13.2 / 11.7; but more than one per
-  // CU, 120x120x18 at 49 columns a tile 4.76 / 4.99, 200x200x8 5.69 / 6.02.  The
-  // FP64 factor doubles what is read again: 100x100x20 9.20 / 8.68, 120x120x24
-  // 13.6 / 13.9.
+  // tile per CU at most, or up to 250,000 nodes and one row per thread.  A pass of one time
+  // step, five launches / tiles, ms:
+  //   a tile per CU     115x115 cells of 10 layers 3.93 / 2.72, 126x126x14 4.02 / 3.23,
+  //                     120x120x18 4.65 / 3.97, 120x120x24 13.2 / 11.7
+  //   more, one row     130x130x8 (270 tiles) 3.51 / 3.08, 150x150x5 (357) 4.51 / 2.97,
+  //                     200x200x2 (634) 4.66 / 3.14, 135x135x12 (289) 4.95 / 4.78,
+  //                     150x150x9 4.28 / 3.91, 170x170x7 (459) 5.46 / 4.75, 200x200x5
+  //                     4.96 / 4.39, 220x220x4 (764) 5.20 / 3.86; Newton 150x150x9 7.8 / 7.2
+  //   and two rows      128x128x13 (261) 4.14 / 4.25, 130x130x13 (270) 3.82 / 3.98, FP64
+  //                     3.85 / 5.46: the tiles beyond one per CU wait for a second round
+  //   above 250,000     200x200x8 5.69 / 6.02: reading the factor two to three times costs more
+  //                     than the launches.
+  // Only surfaces of more than 16,000 columns need more than one tile per CU.  The FP64 factor
+  // doubles what is read again: 100x100x20 9.20 / 8.68, 150x150x9 4.35 / 4.14, but
+  // 120x120x24 13.6 / 13.9.
   static constexpr int kTileMaxRows = 250000, kTileGroups = 256;
   bool tiles() const { return tiles_on && (f32 || n <= kTileMaxRows); }
   bool tiles_wanted(int ncolr) const { return ncolr == 3 && row_tile() == 0 && n <= 2 * kTileMaxRows; }
@@ -766,9 +774,9 @@ struct Flow {
   // Columns per tile: a tile per CU, from 25 columns (below, the columns around a
   // tile outweigh it) to 64 (above, a phase outgrows the LDS a work-group may
   // take); fewer where columns are so deep that a phase's rows outgrow a
-  // work-group.  No tiles where a large mesh needs more than one tile per CU.
+  // work-group.
   void cut_tiles() {
-    bool fits = false;
+    bool fits = false, one_row = false;
     for (int size = std::min(64, std::max(25, (nnod + 247) / 248)); size >= 9 && !fits; size = size * 7 / 8) {
       cut_tiles_of(size);
       std::vector<std::vector<int>> mem(ntile);
@@ -780,8 +788,9 @@ struct Flow {
         cols = std::max({cols, (int)mem[t].size(), (int)T.set[0].size(), (int)T.set[1].size(), (int)T.set[2].size()});
       }
       fits = (long long)cols * (nstr + 1) <= 2 * kTileThreads;
+      one_row = (long long)cols * (nstr + 1) <= kTileThreads;
     }
-    if (fits && (ntile <= kTileGroups || n <= kTileMaxRows)) return;
+    if (fits && (ntile <= kTileGroups || (n <= kTileMaxRows && one_row))) return;
     tile_of.clear();
     ntile = 0;
   }
