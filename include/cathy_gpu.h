@@ -571,6 +571,9 @@ int cathy_gpu_ensemble_set_graphs(int64_t *ens, const int *on);
 /* out5: members, Picard rounds, PCG polls, PCG launch batches and graph
  * captures of the last advance. */
 int cathy_gpu_ensemble_info(int64_t *ens, int64_t *out5);
+/* Rounds of the last advance in which every member ran over surface tiles
+ * (cathy_gpu_flow3d_tiles). */
+int cathy_gpu_ensemble_tile_rounds(int64_t *ens, int64_t *out);
 int cathy_gpu_ensemble_destroy(int64_t *ens);
 
 /* ------------------------------------------------------------------ *
@@ -587,10 +590,11 @@ int cathy_gpu_flow3d_spmv_bytes(int64_t *handle, double *bytes);
  * per-chain codes of the extruded mesh (else read per slot), and the
  * number of slots whose code failed the set-up check (0). */
 int cathy_gpu_flow3d_layout(int64_t *handle, int64_t *out6);
-/* How the preconditioner runs: out3 = surface tiles the solver uses (0:
- * launches per colour or level), rows of a tile's phase per thread, threads
- * of a tile. */
-int cathy_gpu_flow3d_tiles(int64_t *handle, int *out3);
+/* How the solver runs on this mesh: out4 = its surface tiles (0: launches per
+ * colour or level), rows of a tile's phase per thread, threads of a tile, and
+ * whether the last solve ran over the tiles (it takes the launches per colour,
+ * to the same bits, while many rows are being advanced on the GPU). */
+int cathy_gpu_flow3d_tiles(int64_t *handle, int *out4);
 /* The preconditioner of the last linear solve on a vector, z = M^-1 t (N
  * values each, CATHY order): (L L^T)^-1 in Picard runs, U^-1 L^-1 in Newton
  * runs.  *launches: 0 as the solver runs it, 1 by the launches per colour or

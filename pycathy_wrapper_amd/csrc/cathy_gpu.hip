@@ -544,13 +544,14 @@ int cathy_gpu_flow3d_layout(int64_t *handle, int64_t *out6) {
   });
 }
 
-int cathy_gpu_flow3d_tiles(int64_t *handle, int *out3) {
+int cathy_gpu_flow3d_tiles(int64_t *handle, int *out4) {
   return guarded([&] {
     const std::shared_ptr<Flow> f = lookup(handle);
-    CG_REQUIRE(out3, "null argument");
-    out3[0] = f->tiles() ? f->ntile : 0;
-    out3[1] = f->tiles() ? f->tile_rpt : 0;
-    out3[2] = f->tiles() ? f->tile_threads : 0;
+    CG_REQUIRE(out4, "null argument");
+    out4[0] = f->tiles() ? f->ntile : 0;
+    out4[1] = f->tiles() ? f->tile_rpt : 0;
+    out4[2] = f->tiles() ? f->tile_threads : 0;
+    out4[3] = f->over_tiles() ? 1 : 0;
     return 0;
   });
 }

@@ -31,12 +31,12 @@ constexpr int kMaxMembers = 512;
 
 // launch shapes of the batched kernels: groups per member.  kShRows .. kShCol3
 // hold every member; the PCG's kernels run either over surface tiles
-// (kShTile.., members with Flow::tiles()) or colour by colour (kShSpmv ..
-// kShSweep3, the others).
+// (kShTile.., members with Flow::over_tiles()) or colour by colour (kShSpmv ..
+// kShSweep3, the others; their dots by tile, kShDots, where the mesh has tiles).
 enum Shape {
   kShRows = 0, kShRed, kShNnod, kShFlux, kShOne, kShCol0,
   kShTile = kShCol0 + 4, kShTileRows, kShTileOne,
-  kShSpmv, kShVec, kShSweep0, kNShape = kShSweep0 + 4
+  kShSpmv, kShVec, kShDot, kShDots, kShSweep0, kNShape = kShSweep0 + 4
 };
 
 int shape_groups(const Flow &f, int sh) {
@@ -46,13 +46,15 @@ int shape_groups(const Flow &f, int sh) {
     case kShNnod: return grid_for(f.nnod);
     case kShFlux: return grid_for(f.nnod, kBlock, kMaxRedBlocks);
     case kShOne: return 1;
-    case kShTile: return f.tiles() ? f.ntile : 0;
-    case kShTileRows: return f.tiles() ? grid_for(f.n) : 0;
-    case kShTileOne: return f.tiles() ? 1 : 0;
-    case kShSpmv: return f.tiles() ? 0 : grid_for(f.n);
-    case kShVec: return f.tiles() ? 0 : std::min(grid_for(f.n), kVecGroups);
+    case kShTile: return f.over_tiles() ? f.ntile : 0;
+    case kShTileRows: return f.over_tiles() ? grid_for(f.n) : 0;
+    case kShTileOne: return f.over_tiles() ? 1 : 0;
+    case kShSpmv: return f.over_tiles() ? 0 : grid_for(f.n);
+    case kShVec: return f.over_tiles() ? 0 : std::min(grid_for(f.n), kVecGroups);
+    case kShDot: return f.tiles() ? 0 : std::min(grid_for(f.n), kVecGroups);
+    case kShDots: return f.tiles() && f.crowded ? f.ntile : 0;
     default: {
-      if (sh >= kShSweep0 && f.tiles()) return 0;
+      if (sh >= kShSweep0 && f.over_tiles()) return 0;
       const int c = sh >= kShSweep0 ? sh - kShSweep0 : sh - kShCol0;
       return c < (int)f.sched.cols.size() ? grid_for(f.sched.cols[c].nc, kChains) : 0;
     }
@@ -80,7 +82,10 @@ struct Ensemble {
   DBuf<int> dact;
   Pinned<int> hact;
   std::vector<char> active, tab_active;
+  int kind = 0;  // of the members on the colour launches: none on a mesh with tiles, all, some
+  std::vector<char> crowding, tab_crowded;  // Flow::crowded of each member when the tables were built
   // statistics of the last advance
+  long tile_rounds = 0;  // rounds in which every member ran over tiles
   long rounds = 0, polls = 0, pcg_batches = 0, graph_captures = 0;
   // HIP graphs of a round's fixed launch sequences: pre-solve (Picard
   // assembly, factor, PCG start), one PCG batch of `g_follow` iterations,
@@ -200,7 +205,12 @@ struct Ensemble {
       gtot[sh] = t[nm];
     }
     CG_HIP(hipMemcpyAsync(dtab.p, htab.p, sizeof(int) * kNShape * (nm + 1), hipMemcpyHostToDevice, st));
+    bool plain = false, tiled = false;
+    for (int j = 0; j < nm; ++j)
+      if (active[j] && !mem[j]->over_tiles()) (mem[j]->tiles() ? tiled : plain) = true;
+    kind = tiled ? (plain ? 2 : 1) : 0;
     tab_active = active;
+    tab_crowded = crowding;
     drop_graphs();  // the grids change with the members taking part
   }
 
@@ -268,28 +278,29 @@ struct Ensemble {
       }
     }
   }
+  // f(KIND) of the members that run by the colour launches (see kb_fwd_col3)
+  template <typename F>
+  void by_kind(F &&f) {
+    if (kind == 0) f(std::integral_constant<int, 0>{});
+    else if (kind == 1) f(std::integral_constant<int, 1>{});
+    else f(std::integral_constant<int, 2>{});
+  }
   template <typename FT, bool LAST>
   void fwd_t(int c, int vin, int vout, int use_done) {
-    const int sh = kShSweep0 + c;
-    const size_t sm = (LAST ? 2 : 1) * sm_col[c];
-    switch (wf[c]) {
-      case 0: launch(kb_fwd_col3<FT, 0, LAST>, sh, sm, c, vin, vout, use_done); break;
-      case 4: launch(kb_fwd_col3<FT, 4, LAST>, sh, sm, c, vin, vout, use_done); break;
-      case 8: launch(kb_fwd_col3<FT, 8, LAST>, sh, sm, c, vin, vout, use_done); break;
-      case 12: launch(kb_fwd_col3<FT, 12, LAST>, sh, sm, c, vin, vout, use_done); break;
-      default: launch(kb_fwd_col3<FT, 16, LAST>, sh, sm, c, vin, vout, use_done); break;
-    }
+    Flow::with_window(wf[c], [&](auto nw) {
+      by_kind([&](auto kd) {
+        launch(kb_fwd_col3<FT, decltype(nw)::value, LAST, decltype(kd)::value>, kShSweep0 + c,
+               (LAST ? 2 : 1) * sm_col[c], c, vin, vout, use_done);
+      });
+    });
   }
   template <typename FT>
   void bwd_t(int c, int vio, int use_done) {
-    const int sh = kShSweep0 + c;
-    switch (wb[c]) {
-      case 0: launch(kb_bwd_col3<FT, 0>, sh, sm_col[c], c, vio, use_done); break;
-      case 4: launch(kb_bwd_col3<FT, 4>, sh, sm_col[c], c, vio, use_done); break;
-      case 8: launch(kb_bwd_col3<FT, 8>, sh, sm_col[c], c, vio, use_done); break;
-      case 12: launch(kb_bwd_col3<FT, 12>, sh, sm_col[c], c, vio, use_done); break;
-      default: launch(kb_bwd_col3<FT, 16>, sh, sm_col[c], c, vio, use_done); break;
-    }
+    Flow::with_window(wb[c], [&](auto nw) {
+      by_kind([&](auto kd) {
+        launch(kb_bwd_col3<FT, decltype(nw)::value, decltype(kd)::value>, kShSweep0 + c, sm_col[c], c, vio, use_done);
+      });
+    });
   }
   // z = (L L^T)^-1 t for every member (Flow::precond_apply_t)
   template <typename FT>
@@ -327,10 +338,11 @@ struct Ensemble {
     launch(kb_spmv_beta, kShTileRows, 0);
     tile<kTilePcg>(0, 0);
     launch(kb_spmv_dot2, kShSpmv, 0);
-    launch(kb_pcg_alpha, kShVec, 0);
+    by_kind([&](auto kd) { launch(kb_pcg_alpha<decltype(kd)::value>, kShVec, 0); });
     precond(kVecR, kVecZ, 1);
-    launch(kb_dot, kShVec, 0);
-    launch(kb_pcg_beta, kShVec, 0);
+    launch(kb_dot, kShDot, 0);
+    launch_b(rpt_tile == 1 ? kb_tile_dots<1> : kb_tile_dots<2>, kShDots, 0, thr_tile);
+    by_kind([&](auto kd) { launch(kb_pcg_beta<decltype(kd)::value>, kShVec, 0); });
   }
   // the Picard iteration up to the PCG loop: CHPIC0, BCPIC rows, the fused
   // assembly (picard.f:74-165), IC(0), x0 = M^-1 b, r, p = M^-1 r
@@ -426,7 +438,7 @@ struct Ensemble {
         for (int j = 0; j < e->nm; ++j) e->mem[j]->st = own[j];
       }
     } restore{this, own};
-    rounds = polls = pcg_batches = graph_captures = 0;
+    rounds = polls = pcg_batches = graph_captures = tile_rounds = 0;
     std::vector<int> niter(nm, 0), cont(nm, 0);
     for (int j = 0; j < nm; ++j) {
       rc[j] = 0;
@@ -440,10 +452,21 @@ struct Ensemble {
       active[j] = 1;
       f.step_begin();
     }
+    long rows = 0;
+    for (int j = 0; j < nm; ++j) rows += active[j] ? mem[j]->n : 0;
+    const RowsInFlight here(rows);
     tab_active.assign(nm, 2);  // forces the first table build
+    crowding.assign(nm, 0);
     while (std::find(active.begin(), active.end(), 1) != active.end()) {
       ++rounds;
-      if (active != tab_active) build_tables();
+      for (int j = 0; j < nm; ++j) {  // another group may have started or ended
+        if (active[j]) mem[j]->crowded = mem[j]->too_crowded(here.rows);
+        crowding[j] = mem[j]->crowded;
+      }
+      bool over = true;
+      for (int j = 0; j < nm; ++j) over = over && (!active[j] || mem[j]->over_tiles());
+      tile_rounds += over;
+      if (active != tab_active || crowding != tab_crowded) build_tables();
       for (int j = 0; j < nm; ++j)
         if (active[j]) hargs.p[j] = member_dev(j);
       CG_HIP(hipMemcpyAsync(dargs.p, hargs.p, sizeof(MemberDev) * nm, hipMemcpyHostToDevice, st));
@@ -549,6 +572,14 @@ int cathy_gpu_ensemble_info(int64_t *ens, int64_t *out5) {
     out5[2] = e->polls;
     out5[3] = e->pcg_batches;
     out5[4] = e->graph_captures;
+    return 0;
+  });
+}
+
+int cathy_gpu_ensemble_tile_rounds(int64_t *ens, int64_t *out) {
+  return guarded([&] {
+    CG_REQUIRE(out, "null argument");
+    *out = ens_lookup(ens)->tile_rounds;
     return 0;
   });
 }

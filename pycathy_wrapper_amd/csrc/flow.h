@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstring>
@@ -137,6 +138,17 @@ struct BcSeries {
 };
 
 // ------------------------------------------------------------------ Flow --
+// Rows of the runs that this process is advancing: a measure of how full the GPU is, from which a
+// solve takes one of two ways to the same bits (Flow::too_crowded).
+inline std::atomic<long> rows_in_flight{0};
+struct RowsInFlight {
+  const long rows;
+  explicit RowsInFlight(long r) : rows(r) { rows_in_flight += r; }
+  ~RowsInFlight() { rows_in_flight -= rows; }
+  RowsInFlight(const RowsInFlight &) = delete;
+  RowsInFlight &operator=(const RowsInFlight &) = delete;
+};
+
 struct Flow {
   int n = 0, nt = 0, ntri = 0, nnod = 0, nstr = 0, nnz = 0, ordering = 0, lump = 1;
   // the 3-colour column ordering; its rows in tiles of row_tile() chains
@@ -738,7 +750,30 @@ struct Flow {
   // doubles what is read again: 100x100x20 9.20 / 8.68, 150x150x9 4.35 / 4.14, but
   // 120x120x24 13.6 / 13.9.
   static constexpr int kTileMaxRows = 250000, kTileGroups = 256;
+  // The solver's tiles; over_tiles(): and the current solve runs on them.
   bool tiles() const { return tiles_on && (f32 || n <= kTileMaxRows); }
+  bool over_tiles() const { return tiles() && !crowded; }
+  // Whether the GPU is too full for tiles: they compute each row two to three times over,
+  // which costs nothing while CUs are idle.  rows: of the advances under way (RowsInFlight).  The
+  // same bits either way (tiles.h).  Member-steps/s in lockstep, colour launches / tiles:
+  //   n = 4,851    64 members 2,330 / 3,190, 192 (931,000 rows) 4,240 / 4,850
+  //   12,493       16 members 880 / 1,046, 32 (400,000) 1,424 / 1,409, 48 1,806 / 1,650
+  //   26,896       4 members 136 / 160, 8 (215,000) 186 / 179 (390 / 418 with fewer PCG iterations
+  //                a step), 16 280 / 225, 32 in groups of 8 421 / 281
+  //   63,257       3 members 148 / 156, 4 (253,000) 184 / 175
+  //   124,659      2 members (249,000) 81.7 / 78.7, 3 91 / 76
+  //   214,221      1 33.1 / 33.6, 2 52 / 42, 4 60 / 40, 8 in groups of 2 77.8 / 39.7
+  // Advances on streams of their own share four hardware queues, so at most four are under
+  // way at a moment: 26,896 nodes, 8 streams 116 / 163, 32 133 / 185; 214,221, 2 streams
+  // 58 / 48, 4 78.3 / 47.3.
+  // A mesh with tiles runs the colour launches 0 - 4% slower than they run without (its sums are
+  // by tile, k_tile_dots): 26,896 nodes, 32 members 424, 16 272; 214,221, 8 members 76.4.
+  static long tile_rows(int n) { return n < 8192 ? 900000 : (n < 16384 ? 400000 : 225000); }
+  bool too_crowded(long own) const {  // own: rows of this advance
+    const long rows = std::min(rows_in_flight.load(), 4 * own);
+    return rows > n && rows > tile_rows(n);
+  }
+  bool crowded = false;
   bool tiles_wanted(int ncolr) const { return ncolr == 3 && row_tile() == 0 && n <= 2 * kTileMaxRows; }
   // Columns of each colour a tile needs besides its own (mem): set[c] starts
   // with the own[c] of the tile, those up to x1 (colour 1) take the backward sweep.
@@ -861,6 +896,8 @@ struct Flow {
         std::sort(set[c].begin() + d.own[c], set[c].begin() + x, key);
         std::sort(set[c].begin() + x, set[c].end(), key);
         d.n[c] = (int)set[c].size();
+        for (int i = 1; i < d.own[c]; ++i)  // the own columns of a colour: neighbouring chains (k_tile_dots)
+          if (chain(set[c][i]) != chain(set[c][0]) + i) return;
         cols[t].insert(cols[t].end(), set[c].begin(), set[c].end());
       }
       d.off = ntot;
@@ -925,7 +962,7 @@ struct Flow {
     tiles_on = true;
   }
   TileSet tile_set() const {
-    return TileSet{t_desc.p, t_rows.p, t_tab.p, tiles_on ? ntile : 0, tile_ntot, tile_threads};
+    return TileSet{t_desc.p, t_rows.p, t_tab.p, tiles() ? ntile : 0, tile_ntot, tile_threads};
   }
   TilePcg tile_pcg(const double *diag = nullptr) {
     TilePcg P{};
@@ -934,6 +971,12 @@ struct Flow {
     P.part_pr = this->P(1); P.part_pb = this->P(2); P.part_bz = this->P(4); P.part_rr = this->P(3);
     P.A = A.p; P.dinv = diag ? diag : dinv.p; P.isdir = isdir.p; P.sc = scal.p; P.done = flags.p; P.n = n;
     return P;
+  }
+  // (B, z) and ||r||^2 by tile
+  void tile_dots() {
+    auto k = tile_rpt == 1 ? k_tile_dots<1> : k_tile_dots<2>;
+    hipLaunchKernelGGL(k, dim3(ntile), dim3(tile_threads), 0, st, tile_set(),
+                       TileCols{{sched.cols[0], sched.cols[1], sched.cols[2]}}, tile_pcg());
   }
   size_t tile_smem() const { return tile_lds(tile_nloc, tile_coef, nstr + 1); }
   // out = (L L^T)^-1 in, L^-1 in or L^-T in (diag: the inverse diagonal; null: dinv)
@@ -1519,25 +1562,33 @@ struct Flow {
                        double *out, const int *done) {
     const dim3 g(grid_for(C.nc, kChains)), b(256);
     const size_t sm = (LAST ? 2 : 1) * col_smem(C);
-    switch (sweep_window(C.nf)) {
-      case 0: hipLaunchKernelGGL((k_fwd_col3<FT, 0, LAST>), g, b, sm, st, C, sl, F, di, tin, out, done); break;
-      case 4: hipLaunchKernelGGL((k_fwd_col3<FT, 4, LAST>), g, b, sm, st, C, sl, F, di, tin, out, done); break;
-      case 8: hipLaunchKernelGGL((k_fwd_col3<FT, 8, LAST>), g, b, sm, st, C, sl, F, di, tin, out, done); break;
-      case 12: hipLaunchKernelGGL((k_fwd_col3<FT, 12, LAST>), g, b, sm, st, C, sl, F, di, tin, out, done); break;
-      default: hipLaunchKernelGGL((k_fwd_col3<FT, 16, LAST>), g, b, sm, st, C, sl, F, di, tin, out, done); break;
-    }
+    auto k = [&](auto nw) {
+      constexpr int NW = decltype(nw)::value;
+      auto f = tiles() ? k_fwd_col3<FT, NW, LAST, true> : k_fwd_col3<FT, NW, LAST, false>;
+      hipLaunchKernelGGL(f, g, b, sm, st, C, sl, F, di, tin, out, done);
+    };
+    with_window(sweep_window(C.nf), k);
   }
   template <typename FT>
   void launch_bwd_col3(const ColDesc &C, const Sell &sl, const FT *F, const double *di, const double *xin,
                        double *out, const int *done) {
     const dim3 g(grid_for(C.nc, kChains)), b(256);
     const size_t sm = col_smem(C);
-    switch (sweep_window(C.nb)) {
-      case 0: hipLaunchKernelGGL((k_bwd_col3<FT, 0>), g, b, sm, st, C, sl, F, di, xin, out, done); break;
-      case 4: hipLaunchKernelGGL((k_bwd_col3<FT, 4>), g, b, sm, st, C, sl, F, di, xin, out, done); break;
-      case 8: hipLaunchKernelGGL((k_bwd_col3<FT, 8>), g, b, sm, st, C, sl, F, di, xin, out, done); break;
-      case 12: hipLaunchKernelGGL((k_bwd_col3<FT, 12>), g, b, sm, st, C, sl, F, di, xin, out, done); break;
-      default: hipLaunchKernelGGL((k_bwd_col3<FT, 16>), g, b, sm, st, C, sl, F, di, xin, out, done); break;
+    auto k = [&](auto nw) {
+      constexpr int NW = decltype(nw)::value;
+      auto f = tiles() ? k_bwd_col3<FT, NW, true> : k_bwd_col3<FT, NW, false>;
+      hipLaunchKernelGGL(f, g, b, sm, st, C, sl, F, di, xin, out, done);
+    };
+    with_window(sweep_window(C.nb), k);
+  }
+  template <typename K>
+  static void with_window(int w, K &&k) {
+    switch (w) {
+      case 0: k(std::integral_constant<int, 0>{}); break;
+      case 4: k(std::integral_constant<int, 4>{}); break;
+      case 8: k(std::integral_constant<int, 8>{}); break;
+      case 12: k(std::integral_constant<int, 12>{}); break;
+      default: k(std::integral_constant<int, 16>{}); break;
     }
   }
   size_t fac_smem(const ColDesc &C) const {
@@ -1589,7 +1640,7 @@ struct Flow {
     }
   }
   void precond_apply(const double *tin, double *out, const int *done) {
-    if (tiles()) { tile_apply<kTileSolve>(tin, out, done); return; }
+    if (over_tiles()) { tile_apply<kTileSolve>(tin, out, done); return; }
     if (f32) precond_apply_t<float>(F32.p, tin, out, done);
     else precond_apply_t<double>(F64.p, tin, out, done);
   }
@@ -1683,6 +1734,8 @@ struct Flow {
   // SYMSLV on the current A / TNOTI: x = pdiff.  Returns NITER; err out.
   int pcg(double tol, int imax, double *err_out, int expect) {
     const int G = std::min(grid_for(n, kBlock), 1024);
+    const bool tiled = tiles();
+    crowded = too_crowded(n);
     factor();
     int *done = flags.p;
     precond_apply(tnoti.p, pdiff.p, nullptr);  // x0 = M^-1 b (symslv :4686)
@@ -1701,7 +1754,7 @@ struct Flow {
     PcgScal hs{};
     while (true) {
       for (int b = 0; b < batch; ++b) {
-        if (tiles()) {
+        if (over_tiles()) {
           if (prof) {
             hipEvent_t e0 = next_event(), e1 = next_event();
             hipExtLaunchKernelGGL(k_spmv_beta, dim3(Gs), dim3(kBlock), 0, st, e0, e1, 0, sell(), fts, tile_pcg(), ntile);
@@ -1720,14 +1773,16 @@ struct Flow {
           hipLaunchKernelGGL(k_spmv_dot2, dim3(Gs), dim3(kBlock), 0, st, n, sell(), fts, A.p, p.p, r.p, Bv.p,
                              P(1), P(2), scal.p, done);
         }
-        hipLaunchKernelGGL(k_pcg_alpha, dim3(Gr), dim3(kBlock), 0, st, n, Gs, P(1), P(2), Bv.p, p.p, isdir.p,
+        hipLaunchKernelGGL(tiled ? k_pcg_alpha<true> : k_pcg_alpha<false>, dim3(Gr), dim3(kBlock), 0, st, n, Gs, P(1), P(2), Bv.p, p.p, isdir.p,
                            r.p, pdiff.p, P(3), scal.p, done);
         precond_apply(r.p, z.p, done);
-        hipLaunchKernelGGL(k_dot, dim3(Gr), dim3(kBlock), 0, st, n, Bv.p, z.p, P(4), done);
-        hipLaunchKernelGGL(k_pcg_beta, dim3(Gr), dim3(kBlock), 0, st, n, Gr, P(4), P(3), z.p, p.p, scal.p, done);
+        if (tiled) tile_dots();
+        else hipLaunchKernelGGL(k_dot, dim3(Gr), dim3(kBlock), 0, st, n, Bv.p, z.p, P(4), done);
+        hipLaunchKernelGGL(tiled ? k_pcg_beta<true> : k_pcg_beta<false>, dim3(Gr), dim3(kBlock), 0, st, n,
+                           tiled ? ntile : Gr, P(4), P(3), z.p, p.p, scal.p, done);
       }
       launched += batch;
-      if (tiles()) hipLaunchKernelGGL(k_pcg_check, dim3(1), dim3(256), 0, st, tile_pcg(), ntile);
+      if (over_tiles()) hipLaunchKernelGGL(k_pcg_check, dim3(1), dim3(256), 0, st, tile_pcg(), ntile);
       CG_HIP(hipMemcpyAsync(&hbox.p->pcg, scal.p, sizeof(PcgScal), hipMemcpyDeviceToHost, st));
       CG_HIP(hipStreamSynchronize(st));
       hs = hbox.p->pcg;
@@ -1785,12 +1840,12 @@ struct Flow {
     }
   }
   void ilu_fwd(const double *tin, double *out, const int *done) {
-    if (tiles()) { tile_apply<kTileFwd>(tin, out, done); return; }
+    if (over_tiles()) { tile_apply<kTileFwd>(tin, out, done); return; }
     if (f32) ilu_fwd_t<float>(F32.p, tin, out, done);
     else ilu_fwd_t<double>(F64.p, tin, out, done);
   }
   void ilu_bwd(const double *xin, double *out, const int *done) {
-    if (tiles()) { tile_apply<kTileBwd>(xin, out, done, ones.p); return; }
+    if (over_tiles()) { tile_apply<kTileBwd>(xin, out, done, ones.p); return; }
     if (f32) ilu_bwd_t<float>(F32.p, xin, out, done);
     else ilu_bwd_t<double>(F64.p, xin, out, done);
   }
@@ -1821,6 +1876,7 @@ struct Flow {
   // NSYSLV with ISOLV=0 on the current A / TNOTI: x = pdiff.  Returns NITER.
   int bicgstab(double tol, int imax, double *err_out, int expect) {
     alloc_newton();
+    crowded = too_crowded(n);
     if (f32) ilu_factor_t<float>(F32.p);
     else ilu_factor_t<double>(F64.p);
     int *done = flags.p;
@@ -2817,6 +2873,7 @@ struct Flow {
   int advance(double *stv) {
     step_check();
     if (finished) return finished;
+    const RowsInFlight here(n);
     step_begin();
     while (true) {
       if (surf && rt) {  // label 100 of cathy_main.f: route a ponded surface, then POLD = PNEW on it

@@ -316,10 +316,10 @@ __global__ void k_ic_factor_col3t(ColDesc C, Sell sl, FacTab ft, const double *A
                                   double *dinv, int *nfall);
 // LAST: the colour has no later-colour neighbours, so its backward sweep
 // runs in the same launch and y holds the final x for its rows.
-template <typename FT, int NW, bool LAST>
+template <typename FT, int NW, bool LAST, bool SER>
 __global__ void k_fwd_col3(ColDesc C, Sell sl, const FT *F, const double *dinv, const double *tin, double *y,
                            const int *done);
-template <typename FT, int NW>
+template <typename FT, int NW, bool SER>
 __global__ void k_bwd_col3(ColDesc C, Sell sl, const FT *F, const double *dinv, const double *xin, double *x,
                            const int *done);
 // Gather window of the column sweeps: the smallest instantiated size that
@@ -366,10 +366,12 @@ __global__ void k_residual0(int n, Sell sl, const double *A, const double *x, co
 // about one triangle and the last-level cache the other.
 __global__ void k_spmv_dot2(int n, Sell sl, FacTab ft, const double *A, const double *p, const double *r,
                             double *B, double *part_pr, double *part_pb, const PcgScal *sc, int *done);
+template <bool TILED>
 __global__ void k_pcg_alpha(int n, int nparts, const double *part_pr, const double *part_pb, const double *B,
                             const double *p, const uint8_t *isdir, double *r, double *x, double *part_rr,
                             PcgScal *sc, const int *done);
 __global__ void k_dot(int n, const double *u, const double *v, double *part, const int *done);
+template <bool TILED>
 __global__ void k_pcg_beta(int n, int nparts, const double *part_bz, const double *part_rr, const double *z,
                            double *p, PcgScal *sc, const int *done);
 __global__ void k_pcg_init(int nparts, const double *part, PcgScal *sc, int *done, double tol, int imax);
@@ -489,7 +491,7 @@ struct MemberDev {
   const int *row_surf, *surf_row, *refid;
   const double *volnod, *snodi, *pnodi;
   PcgScal *scal;
-  TileSet tiles;               // the PCG over surface tiles (ntile 0: not used)
+  TileSet tiles;               // the PCG over surface tiles (ntile 0: a mesh not on tiles)
   TilePcg tpcg;
 };
 // vectors a batched sweep reads / writes
@@ -504,16 +506,18 @@ template <int MR>
 __global__ void kb_assemble_plan(const int *start, int nmem, const MemberDev *md);
 template <typename FT, int NW>
 __global__ void kb_ic_factor_col3t(const int *start, int nmem, const MemberDev *md, int c);
-template <typename FT, int NW, bool LAST>
+template <typename FT, int NW, bool LAST, int KIND>
 __global__ void kb_fwd_col3(const int *start, int nmem, const MemberDev *md, int c, int vin, int vout,
                             int use_done);
-template <typename FT, int NW>
+template <typename FT, int NW, int KIND>
 __global__ void kb_bwd_col3(const int *start, int nmem, const MemberDev *md, int c, int vio, int use_done);
 __global__ void kb_residual0(const int *start, int nmem, const MemberDev *md);
 __global__ void kb_pcg_init(const int *start, int nmem, const MemberDev *md);
 __global__ void kb_spmv_dot2(const int *start, int nmem, const MemberDev *md);
+template <int KIND>
 __global__ void kb_pcg_alpha(const int *start, int nmem, const MemberDev *md);
 __global__ void kb_dot(const int *start, int nmem, const MemberDev *md);
+template <int KIND>
 __global__ void kb_pcg_beta(const int *start, int nmem, const MemberDev *md);
 __global__ void kb_poll(const int *start, int nmem, const MemberDev *md, double *out);
 __global__ void kb_update_pnew(const int *start, int nmem, const MemberDev *md);

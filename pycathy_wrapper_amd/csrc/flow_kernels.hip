@@ -1,6 +1,6 @@
 // flow_kernels.hip -- gfx950 kernels of one Picard iteration and of the
 // IC(0)-PCG solve (device numbering, see kernels.h).
-#include "flow_kernels.h"
+#include "tiles.h"
 
 namespace cg {
 
@@ -684,7 +684,8 @@ __device__ __forceinline__ void chain_scan(double *b, double *a, int len, bool o
 // LAST (the final colour, whose rows couple to no later colour): pass 2
 // then runs the backward sweep L^T x = y of the same chains from LDS
 // (x_k = y_k/L_kk - u'_k x_k+1, as k_bwd_col3 forms it) and stores x.
-template <typename FT, int NW, bool LAST>
+// SER (meshes on surface tiles): the recurrences level by level, in k_tile's order.
+template <typename FT, int NW, bool LAST, bool SER>
 __device__ __forceinline__ void fwd_col3_body(Blk bk, double *smem, ColDesc C, Sell sl, const FT *__restrict__ F,
                                                   const double *__restrict__ dinv, const double *__restrict__ tin,
                                                   double *__restrict__ y, const int *__restrict__ done) {
@@ -737,6 +738,21 @@ __device__ __forceinline__ void fwd_col3_body(Blk bk, double *smem, ColDesc C, S
     }
   }
   __syncthreads();
+  if (SER) {
+    const int t = threadIdx.x, ls = chain_step(C);
+    if (t < kChains && t0 + t < C.nc) {
+      const int o = chain_lds(C, t, 0);
+      tile_chain<false, LAST>(T + o, ls, Lp + o, D + o, ls, C.len);
+      if (LAST) tile_chain<true, false>(T + o, ls, U + o, nullptr, ls, C.len);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < tot; i += blockDim.x) {
+      int k, t;
+      chain_elem(C, t0, i, k, t);
+      if (t < C.nc) y[col_row(C, t, k)] = T[i];
+    }
+    return;
+  }
   if (tot <= (int)blockDim.x) {
     // chains of at most blockDim.x / kChains levels: log-depth scans
     const int i = threadIdx.x;
@@ -776,17 +792,17 @@ __device__ __forceinline__ void fwd_col3_body(Blk bk, double *smem, ColDesc C, S
     }
   }
 }
-template <typename FT, int NW, bool LAST>
+template <typename FT, int NW, bool LAST, bool SER>
 __global__ __launch_bounds__(256) void k_fwd_col3(ColDesc C, Sell sl, const FT *__restrict__ F,
                                                   const double *__restrict__ dinv, const double *__restrict__ tin,
                                                   double *__restrict__ y, const int *__restrict__ done) {
   extern __shared__ double smem[];
-  fwd_col3_body<FT, NW, LAST>(self_xcd_blk(), smem, C, sl, F, dinv, tin, y, done);
+  fwd_col3_body<FT, NW, LAST, SER>(self_xcd_blk(), smem, C, sl, F, dinv, tin, y, done);
 }
 
 // Backward sweep L^T x = y (proddp, solscal-extended.f:4186-4197) on one
 // colour, in place: later colours are final; chains run from the base up.
-template <typename FT, int NW>
+template <typename FT, int NW, bool SER>
 __device__ __forceinline__ void bwd_col3_body(Blk bk, double *smem, ColDesc C, Sell sl, const FT *__restrict__ F,
                                                   const double *__restrict__ dinv, const double *xin, double *x,
                                                   const int *__restrict__ done) {
@@ -836,6 +852,20 @@ __device__ __forceinline__ void bwd_col3_body(Blk bk, double *smem, ColDesc C, S
     U[i] = k < kl ? (double)F[base + 64 * (jd + 1)] * di : 0.0;
   }
   __syncthreads();
+  if (SER) {
+    const int t = threadIdx.x, ls = chain_step(C);
+    if (t < kChains && t0 + t < C.nc) {
+      const int o = chain_lds(C, t, 0);
+      tile_chain<true, false>(T + o, ls, U + o, nullptr, ls, C.len);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < tot; i += blockDim.x) {
+      int k, t;
+      chain_elem(C, t0, i, k, t);
+      if (t < C.nc) x[col_row(C, t, k)] = T[i];
+    }
+    return;
+  }
   if (tot <= (int)blockDim.x) {
     const int i = threadIdx.x;
     int k, t;
@@ -858,12 +888,12 @@ __device__ __forceinline__ void bwd_col3_body(Blk bk, double *smem, ColDesc C, S
     }
   }
 }
-template <typename FT, int NW>
+template <typename FT, int NW, bool SER>
 __global__ __launch_bounds__(256) void k_bwd_col3(ColDesc C, Sell sl, const FT *__restrict__ F,
                                                   const double *__restrict__ dinv, const double *xin, double *x,
                                                   const int *__restrict__ done) {
   extern __shared__ double smem[];
-  bwd_col3_body<FT, NW>(self_xcd_blk(), smem, C, sl, F, dinv, xin, x, done);
+  bwd_col3_body<FT, NW, SER>(self_xcd_blk(), smem, C, sl, F, dinv, xin, x, done);
 }
 
 // ---- natural order: levels of the reference's elimination DAG.  The device
@@ -1169,13 +1199,14 @@ __global__ void k_to_cathy(int n, const int *__restrict__ refid, const double *_
   if (i < n) h[refid[i]] = d[i];
 }
 
-#define CG_INST_SWEEP(FT, U)                                                                              \
-  template __global__ void k_fwd_col3<FT, U, false>(ColDesc, Sell, const FT *, const double *,              \
-                                                    const double *, double *, const int *);                 \
-  template __global__ void k_fwd_col3<FT, U, true>(ColDesc, Sell, const FT *, const double *,               \
-                                                   const double *, double *, const int *);                  \
-  template __global__ void k_bwd_col3<FT, U>(ColDesc, Sell, const FT *, const double *, const double *,      \
-                                             double *, const int *);
+#define CG_INST_SWEEP_S(FT, U, S)                                                                         \
+  template __global__ void k_fwd_col3<FT, U, false, S>(ColDesc, Sell, const FT *, const double *,           \
+                                                       const double *, double *, const int *);              \
+  template __global__ void k_fwd_col3<FT, U, true, S>(ColDesc, Sell, const FT *, const double *,            \
+                                                      const double *, double *, const int *);               \
+  template __global__ void k_bwd_col3<FT, U, S>(ColDesc, Sell, const FT *, const double *, const double *,   \
+                                                double *, const int *);
+#define CG_INST_SWEEP(FT, U) CG_INST_SWEEP_S(FT, U, false) CG_INST_SWEEP_S(FT, U, true)
 #define CG_INST_FTAB(FT, W)                                                                               \
   template __global__ void k_ic_factor_col3t<FT, W>(ColDesc, Sell, FacTab, const double *, const uint8_t *, \
                                                     FT *, double *, int *);
@@ -1334,7 +1365,9 @@ __global__ void k_spmv_dot2(int n, Sell sl, FacTab ft, const double *__restrict_
 }
 
 // alpha from the SpMV partials (every group sums them in the same fixed
-// order); r -= alpha B; x += alpha p; partial r_free^2.
+// order); r -= alpha B; x += alpha p; partial r_free^2.  TILED: a mesh on surface tiles,
+// its sums in k_tile's order (r_free^2 by k_tile_dots).
+template <bool TILED>
 __device__ __forceinline__ void pcg_alpha_body(Blk bk, int n, int nparts, const double *__restrict__ part_pr,
                             const double *__restrict__ part_pb, const double *__restrict__ B,
                             const double *__restrict__ p, const uint8_t *__restrict__ isdir,
@@ -1342,7 +1375,8 @@ __device__ __forceinline__ void pcg_alpha_body(Blk bk, int n, int nparts, const 
                             PcgScal *sc, const int *__restrict__ done) {
   if (*done) return;
   __shared__ double sh[2 * (kBlock / 64)];
-  const double2 prb = reduce_partials2<kBlock>(part_pr, part_pb, nparts, sh);
+  const double2 prb = TILED ? partials_sum(partials_load<4>(part_pr, part_pb, nparts), sh)
+                            : reduce_partials2<kBlock>(part_pr, part_pb, nparts, sh);
   const double pr = prb.x, pb = prb.y;
   const double alfa = pr / pb;
   if (bk.b == 0 && threadIdx.x == 0) {
@@ -1356,28 +1390,34 @@ __device__ __forceinline__ void pcg_alpha_body(Blk bk, int n, int nparts, const 
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int iu = i + u * stride;
-      const double ri = r[iu] - alfa * B[iu];
+      const double ri = fma(-alfa, B[iu], r[iu]);
       r[iu] = ri;
-      x[iu] = x[iu] + alfa * p[iu];
-      if (!isdir[iu]) acc[u] += ri * ri;
+      x[iu] = fma(alfa, p[iu], x[iu]);
+      if (!TILED && !isdir[iu]) acc[u] += ri * ri;
     }
   }
   for (; i < n; i += stride) {
-    const double ri = r[i] - alfa * B[i];
+    const double ri = fma(-alfa, B[i], r[i]);
     r[i] = ri;
-    x[i] = x[i] + alfa * p[i];
-    if (!isdir[i]) acc[0] += ri * ri;
+    x[i] = fma(alfa, p[i], x[i]);
+    if (!TILED && !isdir[i]) acc[0] += ri * ri;
   }
+  if (TILED) return;
   double t = block_sum<kBlock>((acc[0] + acc[1]) + (acc[2] + acc[3]), sh);
   if (threadIdx.x == 0) part_rr[bk.b] = t;
 }
+template <bool TILED>
 __global__ void k_pcg_alpha(int n, int nparts, const double *__restrict__ part_pr,
                             const double *__restrict__ part_pb, const double *__restrict__ B,
                             const double *__restrict__ p, const uint8_t *__restrict__ isdir,
                             double *__restrict__ r, double *__restrict__ x, double *__restrict__ part_rr,
                             PcgScal *sc, const int *__restrict__ done) {
-  pcg_alpha_body(self_blk(), n, nparts, part_pr, part_pb, B, p, isdir, r, x, part_rr, sc, done);
+  pcg_alpha_body<TILED>(self_blk(), n, nparts, part_pr, part_pb, B, p, isdir, r, x, part_rr, sc, done);
 }
+template __global__ void k_pcg_alpha<false>(int, int, const double *, const double *, const double *, const double *,
+                                            const uint8_t *, double *, double *, double *, PcgScal *, const int *);
+template __global__ void k_pcg_alpha<true>(int, int, const double *, const double *, const double *, const double *,
+                                           const uint8_t *, double *, double *, double *, PcgScal *, const int *);
 
 // partial (B, z)
 __device__ __forceinline__ void dot_body(Blk bk, int n, const double *__restrict__ u, const double *__restrict__ v,
@@ -1401,21 +1441,23 @@ __global__ void k_dot(int n, const double *__restrict__ u, const double *__restr
 }
 
 // beta, p = z + beta p, err and the stopping test (graddp.f:1348-1377).
+template <bool TILED>
 __device__ __forceinline__ void pcg_beta_body(Blk bk, int n, int nparts, const double *__restrict__ part_bz,
                            const double *__restrict__ part_rr, const double *__restrict__ z,
                            double *__restrict__ p, PcgScal *sc, const int *__restrict__ done) {
   if (*done) return;
   __shared__ double sh[2 * (kBlock / 64)];
-  const double2 crr = reduce_partials2<kBlock>(part_bz, part_rr, nparts, sh);
+  const double2 crr = TILED ? partials_sum(partials_load<1>(part_bz, part_rr, nparts), sh)
+                            : reduce_partials2<kBlock>(part_bz, part_rr, nparts, sh);
   const double c = crr.x, rr = crr.y;
   const double beta = -c / sc->pb;
   const int stride = bk.nb * blockDim.x;
   int i = bk.b * blockDim.x + threadIdx.x;
   for (; i + 3 * stride < n; i += 4 * stride) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) p[i + u * stride] = z[i + u * stride] + beta * p[i + u * stride];
+    for (int u = 0; u < 4; ++u) p[i + u * stride] = fma(beta, p[i + u * stride], z[i + u * stride]);
   }
-  for (; i < n; i += stride) p[i] = z[i] + beta * p[i];
+  for (; i < n; i += stride) p[i] = fma(beta, p[i], z[i]);
   if (bk.b == 0 && threadIdx.x == 0) {
     const double xl = sc->xlung;
     const double err = xl > 0.0 ? sqrt(rr / xl) : sqrt(rr / n);
@@ -1427,11 +1469,16 @@ __device__ __forceinline__ void pcg_beta_body(Blk bk, int n, int nparts, const d
     }
   }
 }
+template <bool TILED>
 __global__ void k_pcg_beta(int n, int nparts, const double *__restrict__ part_bz,
                            const double *__restrict__ part_rr, const double *__restrict__ z,
                            double *__restrict__ p, PcgScal *sc, const int *__restrict__ done) {
-  pcg_beta_body(self_blk(), n, nparts, part_bz, part_rr, z, p, sc, done);
+  pcg_beta_body<TILED>(self_blk(), n, nparts, part_bz, part_rr, z, p, sc, done);
 }
+template __global__ void k_pcg_beta<false>(int, int, const double *, const double *, const double *, double *, PcgScal *,
+                                           const int *);
+template __global__ void k_pcg_beta<true>(int, int, const double *, const double *, const double *, double *, PcgScal *,
+                                          const int *);
 
 // XLUNG from k_residual0's partials; reset the iteration state.
 __device__ __forceinline__ void pcg_init_body(Blk bk, int nparts, const double *__restrict__ part, PcgScal *sc, int *done,
@@ -2655,26 +2702,39 @@ __global__ __launch_bounds__(256) void kb_ic_factor_col3t(const int *start, int 
   CG_BATCH_HEAD
   ic_factor_col3t_body<FT, NW>(bk, smem, d.col[c], d.sl, d.ft, d.A, d.isdir, fac_of<FT>(d), d.dinv, d.flags + 1);
 }
-template <typename FT, int NW, bool LAST>
+// KIND: the members launched are none of them (0), all of them (1) or some (2) on meshes with
+// surface tiles; one kernel for either kind needs more registers than the plain one (1.25M-node
+// members 2% slower).
+template <typename FT, int NW, bool LAST, int KIND>
 __global__ __launch_bounds__(256) void kb_fwd_col3(const int *start, int nmem, const MemberDev *md, int c, int vin,
                                                    int vout, int use_done) {
   extern __shared__ double smem[];
   CG_BATCH_HEAD
-  fwd_col3_body<FT, NW, LAST>(bk, smem, d.col[c], d.sl, fac_of<FT>(d), d.dinv, vec_of(d, vin), vec_of(d, vout),
-                              use_done ? d.flags : nullptr);
+  const int *done = use_done ? d.flags : nullptr;
+  if (KIND == 1 || (KIND == 2 && d.tiles.ntile))
+    fwd_col3_body<FT, NW, LAST, true>(bk, smem, d.col[c], d.sl, fac_of<FT>(d), d.dinv, vec_of(d, vin), vec_of(d, vout),
+                                      done);
+  else
+    fwd_col3_body<FT, NW, LAST, false>(bk, smem, d.col[c], d.sl, fac_of<FT>(d), d.dinv, vec_of(d, vin),
+                                       vec_of(d, vout), done);
 }
-template <typename FT, int NW>
+template <typename FT, int NW, int KIND>
 __global__ __launch_bounds__(256) void kb_bwd_col3(const int *start, int nmem, const MemberDev *md, int c, int vio,
                                                    int use_done) {
   extern __shared__ double smem[];
   CG_BATCH_HEAD
   double *x = vec_of(d, vio);
-  bwd_col3_body<FT, NW>(bk, smem, d.col[c], d.sl, fac_of<FT>(d), d.dinv, x, x, use_done ? d.flags : nullptr);
+  const int *done = use_done ? d.flags : nullptr;
+  if (KIND == 1 || (KIND == 2 && d.tiles.ntile))
+    bwd_col3_body<FT, NW, true>(bk, smem, d.col[c], d.sl, fac_of<FT>(d), d.dinv, x, x, done);
+  else bwd_col3_body<FT, NW, false>(bk, smem, d.col[c], d.sl, fac_of<FT>(d), d.dinv, x, x, done);
 }
-#define CG_INST_BATCH_SWEEP(FT, U)                                                                         \
-  template __global__ void kb_fwd_col3<FT, U, false>(const int *, int, const MemberDev *, int, int, int, int); \
-  template __global__ void kb_fwd_col3<FT, U, true>(const int *, int, const MemberDev *, int, int, int, int);  \
-  template __global__ void kb_bwd_col3<FT, U>(const int *, int, const MemberDev *, int, int, int);
+#define CG_INST_BATCH_SWEEP_K(FT, U, K)                                                                        \
+  template __global__ void kb_fwd_col3<FT, U, false, K>(const int *, int, const MemberDev *, int, int, int, int); \
+  template __global__ void kb_fwd_col3<FT, U, true, K>(const int *, int, const MemberDev *, int, int, int, int);  \
+  template __global__ void kb_bwd_col3<FT, U, K>(const int *, int, const MemberDev *, int, int, int);
+#define CG_INST_BATCH_SWEEP(FT, U) \
+  CG_INST_BATCH_SWEEP_K(FT, U, 0) CG_INST_BATCH_SWEEP_K(FT, U, 1) CG_INST_BATCH_SWEEP_K(FT, U, 2)
 #define CG_INST_BATCH_FT(FT)                                                                   \
   template __global__ void kb_ic_factor_col3t<FT, 0>(const int *, int, const MemberDev *, int);  \
   template __global__ void kb_ic_factor_col3t<FT, 4>(const int *, int, const MemberDev *, int);  \
@@ -2689,6 +2749,7 @@ CG_INST_BATCH_FT(float)
 CG_INST_BATCH_FT(double)
 #undef CG_INST_BATCH_FT
 #undef CG_INST_BATCH_SWEEP
+#undef CG_INST_BATCH_SWEEP_K
 
 __global__ void kb_residual0(const int *start, int nmem, const MemberDev *md) {
   CG_BATCH_HEAD
@@ -2703,19 +2764,35 @@ __global__ void kb_spmv_dot2(const int *start, int nmem, const MemberDev *md) {
   spmv_dot2_body(bk, d.n, d.sl, d.fts, d.A, d.p, d.r, d.Bv, slot_part(d, 1), slot_part(d, 2), d.scal,
                  d.flags);
 }
+template <int KIND>
 __global__ void kb_pcg_alpha(const int *start, int nmem, const MemberDev *md) {
   CG_BATCH_HEAD
-  pcg_alpha_body(bk, d.n, d.g_rows, slot_part(d, 1), slot_part(d, 2), d.Bv, d.p, d.isdir, d.r, d.pdiff,
-                 slot_part(d, 3), d.scal, d.flags);
+  if (KIND == 1 || (KIND == 2 && d.tiles.ntile))
+    pcg_alpha_body<true>(bk, d.n, d.g_rows, slot_part(d, 1), slot_part(d, 2), d.Bv, d.p, d.isdir, d.r, d.pdiff,
+                         slot_part(d, 3), d.scal, d.flags);
+  else
+    pcg_alpha_body<false>(bk, d.n, d.g_rows, slot_part(d, 1), slot_part(d, 2), d.Bv, d.p, d.isdir, d.r, d.pdiff,
+                          slot_part(d, 3), d.scal, d.flags);
 }
 __global__ void kb_dot(const int *start, int nmem, const MemberDev *md) {
   CG_BATCH_HEAD
   dot_body(bk, d.n, d.Bv, d.z, slot_part(d, 4), d.flags);
 }
+template <int KIND>
 __global__ void kb_pcg_beta(const int *start, int nmem, const MemberDev *md) {
   CG_BATCH_HEAD
-  pcg_beta_body(bk, d.n, d.g_vec, slot_part(d, 4), slot_part(d, 3), d.z, d.p, d.scal, d.flags);
+  if (KIND == 1 || (KIND == 2 && d.tiles.ntile))
+    pcg_beta_body<true>(bk, d.n, d.tiles.ntile, slot_part(d, 4), slot_part(d, 3), d.z, d.p, d.scal, d.flags);
+  else
+    pcg_beta_body<false>(bk, d.n, d.g_vec, slot_part(d, 4), slot_part(d, 3), d.z, d.p, d.scal, d.flags);
 }
+#define CG_INST_BATCH_VEC(K)                                                   \
+  template __global__ void kb_pcg_alpha<K>(const int *, int, const MemberDev *); \
+  template __global__ void kb_pcg_beta<K>(const int *, int, const MemberDev *);
+CG_INST_BATCH_VEC(0)
+CG_INST_BATCH_VEC(1)
+CG_INST_BATCH_VEC(2)
+#undef CG_INST_BATCH_VEC
 // out[3m..3m+2] = stop flag, iterations, last relative residual of member m
 __global__ void kb_poll(const int *start, int nmem, const MemberDev *md, double *out) {
   CG_BATCH_HEAD

@@ -16,71 +16,6 @@ __device__ __forceinline__ void put(T *p, int i, T v) {
   *(T *)((char *)p + (size_t)((uint32_t)i * (uint32_t)sizeof(T))) = v;
 }
 
-// Sums of two partial arrays in a fixed order by the first 256 threads of a
-// work-group of any size, in every thread (sh: 16 doubles).
-// U: partials per thread and array that are loaded without a wait between them.
-template <int U>
-struct Partials {
-  double a[U], b[U];
-};
-template <int U>
-__device__ __forceinline__ Partials<U> partials_load(const double *pa, const double *pb, int cnt) {
-  Partials<U> q{};
-  if (threadIdx.x < 256) {
-    int i = threadIdx.x;
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (i + 256 * u < cnt) {
-        q.a[u] = pa[i + 256 * u];
-        q.b[u] = pb[i + 256 * u];
-      }
-    for (i += 256 * U; i < cnt; i += 256) {
-      q.a[0] += pa[i];
-      q.b[0] += pb[i];
-    }
-  }
-  return q;
-}
-template <int U>
-__device__ __forceinline__ double2 partials_sum(const Partials<U> &q, double *sh) {
-  if (threadIdx.x < 256) {
-    double va = q.a[0], vb = q.b[0];
-#pragma unroll
-    for (int u = 1; u < U; ++u) {
-      va += q.a[u];
-      vb += q.b[u];
-    }
-    va = wave_sum(va);
-    vb = wave_sum(vb);
-    if ((threadIdx.x & 63) == 0) {
-      sh[2 * (threadIdx.x >> 6)] = va;
-      sh[2 * (threadIdx.x >> 6) + 1] = vb;
-    }
-  }
-  __syncthreads();
-  const double2 t = make_double2((sh[0] + sh[2]) + (sh[4] + sh[6]), (sh[1] + sh[3]) + (sh[5] + sh[7]));
-  __syncthreads();
-  return t;
-}
-// Block sums of two values, in thread 0 (sh: 2 * waves doubles).
-__device__ __forceinline__ double2 tile_sum2(double a, double b, double *sh) {
-  a = wave_sum(a);
-  b = wave_sum(b);
-  const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    sh[2 * w] = a;
-    sh[2 * w + 1] = b;
-  }
-  __syncthreads();
-  double2 t = make_double2(0.0, 0.0);
-  if (threadIdx.x == 0)
-    for (int k = 0; k < nw; ++k) {
-      t.x += sh[2 * k];
-      t.y += sh[2 * k + 1];
-    }
-  return t;
-}
-
 // The stopping test after iteration `it` (graddp.f:1348-1377) from its
 // partials; every work-group takes it alike.
 struct PcgTest {
@@ -235,55 +170,6 @@ struct TileRow {
 // tile's first column one plane up.
 __device__ __forceinline__ int tile_nbr(const uint32_t (&w)[kTileSlots / 2], int e, int above) {
   return above + (int)((w[e >> 1] >> (16 * (e & 1))) & 0xFFFFu);
-}
-
-// The recurrence v_k = b_k - a_k v_(k -+ 1) of one column in place (v: b in, v out,
-// planes nloc apart; a: planes cnt apart), k ascending or, UP, descending; SCALE
-// stores v_k d_k instead.  Eight levels' coefficients are in registers ahead of
-// the serial part: the LDS stores would otherwise hold back the loads.
-template <bool UP, bool SCALE>
-__device__ __forceinline__ void tile_chain(double *v, int nloc, const double *a, const double *d, int cnt, int len) {
-  const int sv = UP ? -nloc : nloc, sa = UP ? -cnt : cnt;
-  if (UP) {
-    v += (len - 1) * nloc;
-    a += (len - 1) * cnt;
-  }
-  double y = 0.0;
-  int k = 0;
-  for (; k + 8 <= len; k += 8) {
-    double b[8], c[8], e[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      b[u] = v[u * sv];
-      c[u] = a[u * sa];
-      if (SCALE) e[u] = d[u * sa];
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      y = fma(-c[u], y, b[u]);
-      v[u * sv] = SCALE ? y * e[u] : y;
-    }
-    v += 8 * sv;
-    a += 8 * sa;
-    if (SCALE) d += 8 * sa;
-  }
-  if (k < len) {  // the last levels: reads past the end stay on the last one
-    const int m = len - 1 - k;
-    double b[8], c[8], e[8];
-#pragma unroll
-    for (int u = 0; u < 7; ++u) {
-      const int q = min(u, m);
-      b[u] = v[q * sv];
-      c[u] = a[q * sa];
-      if (SCALE) e[u] = d[q * sa];
-    }
-#pragma unroll
-    for (int u = 0; u < 7; ++u) {
-      if (u > m) break;
-      y = fma(-c[u], y, b[u]);
-      v[u * sv] = SCALE ? y * e[u] : y;
-    }
-  }
 }
 
 // RPT: rows of a phase per thread (the host checks that every phase fits).  flag: the
@@ -529,6 +415,84 @@ CG_INST_TILES(double)
 #undef CG_INST_TILES
 #undef CG_INST_TILE
 
+// ---------------------- the dots of a tile's own rows, for the colour launches --
+// (B, z) and ||r||^2 by tile, by the thread and in the order k_tile takes them: a mesh on tiles
+// whose solve runs by the colour launches (Flow::crowded) sums the same partials, so the
+// two ways give the same bits.  Takes the place of k_dot.  A tile's own columns of a colour
+// are neighbouring chains, so their rows follow from the first.  Bound by latency: the values of all
+// items go out together (threads without a row read the tile's first).  16 x 26,896 nodes 9.8 us (k_dot 3.8);
+// phase after phase, with the rows read from the table, 11.7.
+template <int RPT>
+__device__ __forceinline__ void tile_dots_body(Blk bk, const TileSet &T, const TileCols &C, const TilePcg &P) {
+  __shared__ double sh[2 * kTileThreads / 64];
+  const int stopped = *P.done;
+  const TileDesc d = T.desc[bk.b];
+  if (stopped) return;
+  const int tid = threadIdx.x, nt = T.threads, len = C.c[0].len;
+  const int off1 = d.n[0], off2 = d.n[0] + d.n[1], nown = d.own[0] + d.own[1] + d.own[2];
+  // first own row of each colour (surface plane)
+  const int2 *rows = T.rows + d.row;
+  const int row0[3] = {d.own[0] > 0 ? rows[0].x : 0, d.own[1] > 0 ? rows[off1].x : 0,
+                       d.own[2] > 0 ? rows[off2].x : 0};
+  const int any = d.own[0] > 0 ? row0[0] : (d.own[1] > 0 ? row0[1] : row0[2]);
+  // phase c's items as k_tile's solve takes them (c = 3: its own rows)
+  int r[4][RPT];
+  bool on[4][RPT];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int cnt = c < 3 ? d.n[c] : nown, own = c < 3 ? d.own[c] : nown;
+    int k = cnt > 0 && tid < nt ? tid / cnt : len, l = cnt > 0 ? tid - k * cnt : 0;
+    const int dk = cnt > 0 ? nt / cnt : 0, dl = cnt > 0 ? nt - dk * cnt : 0;
+#pragma unroll
+    for (int u = 0; u < RPT; ++u) {
+      on[c][u] = k < len && l < own;
+      int row;
+      if (c < 3) row = row0[c] + k * C.c[c].nc + l;
+      else if (l < d.own[0]) row = row0[0] + k * C.c[0].nc + l;
+      else if (l < d.own[0] + d.own[1]) row = row0[1] + k * C.c[1].nc + l - d.own[0];
+      else row = row0[2] + k * C.c[2].nc + l - d.own[0] - d.own[1];
+      r[c][u] = on[c][u] ? row : any;
+      k += dk;
+      l += dl;
+      if (cnt > 0 && l >= cnt) {
+        l -= cnt;
+        k += 1;
+      }
+    }
+  }
+  double s[3][RPT], b[RPT], z[RPT], rr = 0.0, bz = 0.0;
+  uint8_t dir[3][RPT];
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+#pragma unroll
+    for (int u = 0; u < RPT; ++u) {
+      s[c][u] = at((const double *)P.r[0], r[c][u]);
+      dir[c][u] = at(P.isdir, r[c][u]);
+    }
+#pragma unroll
+  for (int u = 0; u < RPT; ++u) {
+    b[u] = at((const double *)P.B, r[3][u]);
+    z[u] = at((const double *)P.z, r[3][u]);
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+#pragma unroll
+    for (int u = 0; u < RPT; ++u) rr = on[c][u] && !dir[c][u] ? fma(s[c][u], s[c][u], rr) : rr;
+#pragma unroll
+  for (int u = 0; u < RPT; ++u) bz = on[3][u] ? fma(b[u], z[u], bz) : bz;
+  const double2 t = tile_sum2(bz, rr, sh);
+  if (tid == 0) {
+    P.part_bz[bk.b] = t.x;
+    P.part_rr[bk.b] = t.y;
+  }
+}
+template <int RPT>
+__global__ __launch_bounds__(kTileThreads) void k_tile_dots(TileSet T, TileCols C, TilePcg P) {
+  tile_dots_body<RPT>(self_xcd_blk(), T, C, P);
+}
+template __global__ void k_tile_dots<1>(TileSet, TileCols, TilePcg);
+template __global__ void k_tile_dots<2>(TileSet, TileCols, TilePcg);
+
 // ------------------------------------------ batched ensemble launches --
 #define CG_TILE_HEAD                                       \
   const int g_ = xcd_group();                              \
@@ -565,6 +529,13 @@ __global__ __launch_bounds__(256) void kb_pcg_check(const int *start, int nmem, 
   (void)bk;
   pcg_check_body(d.tpcg, d.tiles.ntile);
 }
+template <int RPT>
+__global__ __launch_bounds__(kTileThreads) void kb_tile_dots(const int *start, int nmem, const MemberDev *md) {
+  CG_TILE_HEAD
+  tile_dots_body<RPT>(bk, d.tiles, TileCols{{d.col[0], d.col[1], d.col[2]}}, d.tpcg);
+}
+template __global__ void kb_tile_dots<1>(const int *, int, const MemberDev *);
+template __global__ void kb_tile_dots<2>(const int *, int, const MemberDev *);
 #undef CG_TILE_HEAD
 
 }  // namespace cg

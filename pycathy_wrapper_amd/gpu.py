@@ -383,11 +383,12 @@ class FlowGPU:
                     coded=int(out[4]), code_mismatch=int(out[5]))
 
     def tiles(self) -> dict:
-        """Surface tiles the solver runs over (0: launches per colour or
-        level), rows of a phase per thread and threads of a tile."""
-        out = np.zeros(3, dtype=np.int32)
+        """The solver's surface tiles (0: launches per colour or level), rows
+        of a phase per thread, threads of a tile, and whether the last solve
+        ran over them (full GPUs take the launches, to the same bits)."""
+        out = np.zeros(4, dtype=np.int32)
         _check(lib().cathy_gpu_flow3d_tiles(C.byref(self.h), _p(out)), "tiles")
-        return dict(tiles=int(out[0]), rows_per_thread=int(out[1]), threads=int(out[2]))
+        return dict(tiles=int(out[0]), rows_per_thread=int(out[1]), threads=int(out[2]), last=bool(out[3]))
 
     def precond(self, t, launches: bool = False) -> np.ndarray:
         """The last solve's preconditioner on a vector (N, CATHY order), as the
@@ -452,6 +453,13 @@ class EnsembleGPU:
         _check(lib().cathy_gpu_ensemble_info(C.byref(self.h), _p(out)), "ensemble_info")
         return dict(members=int(out[0]), rounds=int(out[1]), polls=int(out[2]), pcg_batches=int(out[3]),
                     graph_captures=int(out[4]))
+
+    def tile_rounds(self) -> int:
+        """Rounds of the last advance in which every member ran over surface
+        tiles (``info()["rounds"]`` in all)."""
+        out = C.c_int64(0)
+        _check(lib().cathy_gpu_ensemble_tile_rounds(C.byref(self.h), C.byref(out)), "ensemble_tile_rounds")
+        return int(out.value)
 
     def close(self):
         if getattr(self, "h", None) is not None and self.h.value:

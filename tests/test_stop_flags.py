@@ -70,7 +70,7 @@ def test_the_others_are_launched_as_one_group(body, kernels):
         if k.startswith("kb_"):
             shapes = re.findall(r"launch\(" + k + r", (\w+),", text)
             assert shapes and set(shapes) == {"kShTileOne"}
-            assert re.search(r"case kShTileOne: return f\.tiles\(\) \? 1 : 0;", text)
+            assert re.search(r"case kShTileOne: return f\.over_tiles\(\) \? 1 : 0;", text)
         else:
             grids = re.findall(r"hipLaunchKernelGGL\(" + k + r", (dim3\([^)]*\))", text)
             assert grids and set(grids) == {"dim3(1)"}

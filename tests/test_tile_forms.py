@@ -22,7 +22,7 @@ for sz in sorted(small):
     assert T._on_tiles(f, *sz), (sz, f.tiles())
     assert f.tiles()["threads"] <= 1024 and f.tiles()["threads"] % 64 == 0
     c = G.FlowGPU(T._problem(*sz, 1), G.ORDER_COLUMN3C)
-    assert c.tiles() == dict(tiles=0, rows_per_thread=0, threads=0), sz
+    assert c.tiles() == dict(tiles=0, rows_per_thread=0, threads=0, last=False), sz
 assert len(small) > 8 and any(sz in T.TWO_ROWS for sz in small)
 """
 
