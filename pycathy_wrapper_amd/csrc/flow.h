@@ -40,6 +40,15 @@ struct Schedule {
   DBuf<uint32_t> q0[2], idx[2];  // LevSweep forward, backward
 };
 
+// Slot of column v among a row's len sorted columns (len: past the last smaller one, v or not).
+// Rows have some fifteen entries: counting takes no branch that depends on them, where a
+// binary search's were the larger part of a set-up.
+inline int row_slot(const int *c, int len, int v) {
+  int s = 0;
+  for (int i = 0; i < len; ++i) s += c[i] < v;
+  return s;
+}
+
 // Device numbering of the natural elimination order: rows sorted by
 // level(r) = 1 + max level of its lower neighbours, CATHY ids ascending within
 // a level.  Coupled rows keep their order, so the factor is the natural order's
@@ -1005,9 +1014,9 @@ struct Flow {
     for (const ColDesc &C : sched.cols) nch = std::max(nch, C.g0 + C.nc);
     constexpr int NB = kFacWords * 4;
     auto pos_in = [&](int row, int col) -> int {
-      const int *b = &hcol[hrp[row]], *e = &hcol[hrp[row + 1]];
-      const int *f = std::lower_bound(b, e, col);
-      return (f != e && *f == col) ? (int)(f - b) : -1;
+      const int *b = &hcol[hrp[row]];
+      const int len = hrp[row + 1] - hrp[row], k = row_slot(b, len, col);
+      return (k < len && b[k] == col) ? k : -1;
     };
     // the bytes row r (plane k of a colour whose planes lie sk rows apart) needs
     auto row_bytes = [&](int r, int k, int sk, uint8_t *out) -> bool {
@@ -1098,9 +1107,11 @@ struct Flow {
       std::fill(b, b + sizeof b, (uint8_t)0xFF);
       for (int j = 0; j < hsd[r]; ++j) {
         const int p = hrp[r] + j, c = hcol[p];
-        for (int a = 0; a < j; ++a) {
-          const int *e = &hcol[hrp[c + 1]], *f = std::lower_bound(&hcol[hrp[c]], e, hcol[hrp[r] + a]);
-          if (f != e && *f == hcol[hrp[r] + a]) b[j * (j - 1) / 2 + a] = (uint8_t)(f - &hcol[hrp[c]]);
+        const int *cr = &hcol[hrp[r]], *cc = &hcol[hrp[c]];
+        const int len = hrp[c + 1] - hrp[c];
+        for (int a = 0, i = 0; a < j; ++a) {  // both rows ascend
+          while (i < len && cc[i] < cr[a]) ++i;
+          if (i < len && cc[i] == cr[a]) b[j * (j - 1) / 2 + a] = (uint8_t)i;
         }
         b[NP + j] = (uint8_t)(htpos[p] - hrp[c]);
       }
@@ -1174,13 +1185,13 @@ struct Flow {
         hcol[hrp[r] + k] = slot[(size_t)r * W + k];
         if (slot[(size_t)r * W + k] == r) hdiag[r] = hrp[r] + k;
       }
+    // rows ascending meet a row's entries in their order
+    std::vector<int> met(hrp.begin(), hrp.end() - 1);
     for (int r = 0; r < n; ++r)
       for (int p = hrp[r]; p < hrp[r + 1]; ++p) {
-        int j = hcol[p];
-        const int *b = &hcol[hrp[j]], *e = &hcol[hrp[j + 1]];
-        const int *f = std::lower_bound(b, e, r);
-        CG_REQUIRE(f != e && *f == r, "pattern not symmetric");
-        htpos[p] = hrp[j] + (int)(f - b);
+        const int j = hcol[p], f = met[j]++;
+        CG_REQUIRE(f < hrp[j + 1] && hcol[f] == r, "pattern not symmetric");
+        htpos[p] = f;
       }
     // SELL-64: slice s holds rows 64s..64s+63, entry j of row r at
     // so[s] + 64 j + (r & 63); padding = own row id, zero value.
@@ -1330,9 +1341,7 @@ struct Flow {
         hinc[i] = e * 4 + k;
         uint32_t pk = 0;
         for (int l = 0; l < 4; ++l) {
-          const int *b = &h_col[h_rowptr[r]], *en = &h_col[h_rowptr[r + 1]];
-          const int *f = std::lower_bound(b, en, v[l]);
-          pk |= (uint32_t)(f - b) << (8 * l);
+          pk |= (uint32_t)row_slot(&h_col[h_rowptr[r]], h_rowptr[r + 1] - h_rowptr[r], v[l]) << (8 * l);
         }
         hoff[i] = pk;
       }
