@@ -422,8 +422,8 @@ __global__ void k_copy(size_t n, const double *src, double *dst);
 __global__ void k_fill(size_t n, double v, double *dst);
 
 // ------------------------------------- the PCG over surface tiles (tiles.h) --
-// A tile's columns in LDS order: colour 0, 1, 2; within a colour those whose final
-// x is needed first (x0: the tile's own), and the tile's own first of all.
+// A tile's columns in LDS order: colour 0, 1, 2; within a colour the tile's own
+// first (own), then, in colour 1, the others whose final x it needs (up to x1).
 struct TileDesc {
   int off, row;      // first entry of the tile's columns in the table, of its rows in TileSet::rows
   int n[3];          // columns of each colour whose forward sweep runs here

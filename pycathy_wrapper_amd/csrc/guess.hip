@@ -315,8 +315,9 @@ __global__ __launch_bounds__(kStepCols *kStepRows) void k_gstep(GradParts gp, Gr
 // biases, w + 4 the others and the head) over all tiles of the work-group and are
 // written once, as one split of the partials k_gstep sums.  Rounding points are those of the layer-by-layer
 // kernels (bf16 inputs, weights, activations, gradients; fp32 sums).
-// Bound by LDS latency and barriers (about 18 us per tile) and by writing the
-// partials (48 MB): a training step on 1024 columns of 31 levels took 550 us
+// Bound by LDS latency and barriers (about 18 us per tile, two tiles a group at 1024
+// columns of 31 levels) and by writing the partials (48 MB, 10 us); the products alone
+// would take 7 us at the card's rate.  A training step on 1024 columns of 31 levels took 550 us
 // in 31 launches, 65 us of them convolutions and 87 us weight gradients; it
 // takes 51 us here and 18 us in k_gstep.  With four waves instead of
 // eight (448 registers each) this kernel took 63 us.

@@ -302,7 +302,7 @@ __global__ __launch_bounds__(kRouteBlock) void k_route(RouteDev d, double deltat
     }
     return V;
   };
-  // the cell of the quad: its inflow, and the lane's branch
+  // the pair's cell: its inflow, and the lane's branch
   auto route = [&](int k, const RouteIds &I, const RouteVal &V) {
     auto feed = [&](int src, int loc) {
       if (src < 0) return 0.0;
